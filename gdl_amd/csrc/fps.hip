@@ -7,9 +7,9 @@
 // Four kernels, chosen by the largest cloud of the batch:
 //   bucketed (clouds of up to 8192 points, the common case): one 1024-thread workgroup per
 //     cloud, points ordered along a Hilbert cell grid so that each register slot of a wave holds
-//     a compact bucket of 64 points; a bucket is only updated when the new centroid can lower
-//     one of its distances (an exact test, see below), and the argmax is assembled from cached
-//     per-bucket maxima.
+//     a compact bucket of 64 points; a bucket is only updated when a new centroid can lower
+//     one of its distances (an exact test, see below), and several centroids are taken from the
+//     cached per-bucket maxima per round, where they provably follow each other.
 //   register (8193 to 16384 points): thread t owns local points t, t+256, ... (PTS of them)
 //     with x, y, z and the running min distance in VGPRs; every point is updated every
 //     iteration.
@@ -17,11 +17,11 @@
 //     curve in the workspace and bucket records in registers (see its section below).
 //   streaming (larger clouds): positions read from HBM/L2 each iteration, running min
 //     distance in the workspace.
-// Each reduces (distance bits, index) per iteration to one winner with one barrier: a wave max
-// of the bits (DPP), the lowest index among the lanes holding it, then either one LDS record per
-// wave double-buffered by iteration parity (register, streaming) or one LDS 64-bit atomic max per
-// wave on a (distance, index complement) key (bucketed, large).  Squared distances are
-// non-negative floats, whose bit patterns order like the values.
+// The register, large and streaming kernels reduce (distance bits, index) per iteration to one
+// winner with one barrier: a wave max of the bits (DPP), the lowest index among the lanes holding
+// it, then either one LDS record per wave double-buffered by iteration parity (register,
+// streaming) or one LDS 64-bit atomic max per wave on a (distance, index complement) key (large).
+// Squared distances are non-negative floats, whose bit patterns order like the values.
 #include "radix.hpp"
 
 namespace geo {
@@ -31,6 +31,7 @@ constexpr int kFpsThreads = 256;
 constexpr int kFpsWaves = kFpsThreads / kWave;
 constexpr int kFpsLdsPoints = 8192;  // register kernel centroid table: 8192 * 16 B of LDS
 constexpr int kFpsBucketThreads = 1024;
+constexpr int kFpsRound = 16;  // most centroids that one round of the bucketed kernel takes
 constexpr int kFpsStreamThreads = 1024;
 constexpr int kFpsStreamWaves = kFpsStreamThreads / kWave;
 
@@ -176,17 +177,33 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
 // ------------------------------------------------------------------ bucketed kernel ---
 //
 // Clouds of up to 8192 points.  The cloud is first ordered along a 16^3 Hilbert cell grid
-// (LDS counting sort), so the 64 points a wave holds in one register slot — a bucket — lie
-// close together.  Each bucket keeps its bounding box in lane s of six VGPRs and its (max
-// min-distance, lowest index attaining it, lane holding that point) as wave-uniform scalars, so
-// a wave's best is a few scalar max / compare instructions after an update instead of another
-// cross-lane reduction, and an updated bucket is re-reduced only when the point holding its
-// maximum fell.  Per iteration the wave tests all its buckets at once (one lane per bucket): with
+// (LDS counting sort), so the 64 points a wave holds in one register slot -- a bucket -- lie
+// close together.  Each bucket has its bounding box and a record of its farthest point: max min
+// distance, lowest index attaining it, position, and the rest bound: the most that any other point
+// of the bucket has left once that point is a centroid, max over p of min(md(p), d(p, farthest)).
+//
+// The loop takes several centroids per round.  Order all records by (distance, lower index), and
+// let i be ahead of j.  Record j is the greedy choice right after the records ahead of it if
+//   d(point i, point j) >= md(point j) for every i ahead (none of them lowers its point), and
+//   rest bound of i < md(point j) for every i ahead (no other point of their buckets reaches it):
+// every other point lies below its own bucket's record and values only fall, so nothing can come
+// between.  The round takes the records from the front up to the first that fails (the first one
+// never does).  Rounds therefore give exactly the one-at-a-time sequence; on 16 surface clouds of
+// 4096 points a round takes 7.6 centroids (at most 16), 135 rounds for 1024 samples, 1.6 us each,
+// where one centroid took 0.46 us: 470 -> 238 us.  A round costs two LDS barriers:
+//   check   every wave tests the listed records pairwise, lane = 16 * (j mod 4) + i
+//   update  the wave's buckets against the round's centroids (bound test below), records of the
+//           buckets whose farthest point fell; the wave with the most of them sets the pace
+//   rank    every wave places its own records among all (one ballot each) and lists the first 16
+// Half the threads with twice the buckets each measured 310 us, a quarter 504 us; the check made by
+// each record's own wave before the second barrier (no list of bounds) 240 us.
+//
+// Bound test, one lane per (bucket, centroid): with
 //   g_a = max(lo_a - c_a, c_a - hi_a, 0),  lb = (g_x*g_x + g_y*g_y) + g_z*g_z
 // evaluated with the same fp32 operations as the distance, every rounded operation is monotone,
 // so lb <= d(p, c) holds exactly for every point p of the bucket; when lb >= the bucket's max
-// min-distance no point of the bucket can change and the bucket is skipped.  Skipping is
-// therefore exact; only buckets near the new centroid pay for the update.
+// min-distance no point of the bucket can change and the pair is skipped.  Skipping is therefore
+// exact; a bucket's record is re-reduced only when its farthest point fell.
 constexpr int kCellBits = 4;                  // 16 cells per axis
 constexpr int kCells = 1 << (3 * kCellBits);  // 4096
 
@@ -311,27 +328,32 @@ __device__ void fps_hilbert_order(const float* __restrict__ P, int n, int* hist,
   __syncthreads();
 }
 
+// Order of the greedy choice as one double: distance bits (a non-negative float) above the index
+// complement, so the larger distance comes first and, among equal ones, the lower index.  A
+// positive double orders like its bit pattern, and 0x7f800000 (+inf as a float) in the high word
+// is still a finite double.
+__device__ __forceinline__ double fps_key(uint32_t bits, uint32_t idx) {
+  return __hiloint2double(static_cast<int>(bits), static_cast<int>(~idx));
+}
+
 template <int PTS, int THREADS>
 __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const float* __restrict__ pos, const int64_t* __restrict__ ptr,
     const int64_t* __restrict__ out_ptr, int64_t* __restrict__ out_idx,
     const int64_t* __restrict__ guard) {
   constexpr int WAVES = THREADS / kWave;
-  static_assert(PTS <= kWave, "one lane per bucket");
+  constexpr int NB = PTS * WAVES;              // buckets
+  constexpr int SETS = (NB + kWave - 1) / kWave;  // records per lane in the selection
+  constexpr int TESTS = (PTS + 3) / 4;         // bound tests per round: 4 slots x 16 centroids each
   // Launched before the host has seen the prepare kernel's summary: do nothing unless ptr was
   // valid and every cloud fits this variant (the host then launches the right one).
   if (guard != nullptr && (guard[2] != 0 || guard[1] > PTS * THREADS)) return;
-  // Cross-wave argmax: one 64-bit LDS atomic max per wave on the key
-  //   (it << 45) | (bits << 13) | (8191 - index)
-  // so the largest distance wins and, among equal distances, the lowest index (clouds here have
-  // at most 8192 points and iterations).  Iteration it uses slot it % 2; the iteration number in
-  // the key's top bits makes every key of it larger than any left from it - 2, so no slot is
-  // ever cleared; a slot is reused only after the barrier that every reader of its previous
-  // round passed first.
-  __shared__ unsigned long long slots[2];
+  __shared__ double rkey[NB];         // key of each bucket's farthest point, see fps_key
+  __shared__ float4 list[kFpsRound];  // the first records: position and (bits) rest bound
+  __shared__ uint2 lkey[kFpsRound];   // their min distance (bits) and index
   __shared__ int hist[kCells];
   __shared__ uint32_t red[6][WAVES];
-  extern __shared__ float4 table[];  // sort scratch (12 B/point), then positions by index
+  extern __shared__ int2 scratch[];  // sort scratch, 12 B per point
 
   const int b = blockIdx.x;
   const int64_t start = ptr[b];
@@ -349,15 +371,15 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
   const float* P = pos + start * 3;
 
   // 1-2. the cloud ordered along the Hilbert curve of its cell grid
-  int2* code_rank = reinterpret_cast<int2*>(table);
-  int* order = reinterpret_cast<int*>(reinterpret_cast<char*>(table) + 8 * static_cast<size_t>(n));
+  int2* code_rank = scratch;
+  int* order = reinterpret_cast<int*>(scratch + n);
   fps_hilbert_order<THREADS>(P, n, hist, red, code_rank, order);
 
   // 3. registers.  Bucket j = 64 consecutive sorted points; wave w owns buckets w, w+WAVES, ...
   //    (neighbouring buckets on different waves, so the buckets near a centroid spread over
   //    the SIMDs); slot s of wave w holds bucket s*WAVES + w.
-  float px[PTS], py[PTS], pz[PTS], md[PTS];
-  uint32_t oi[PTS];
+  float px[PTS], py[PTS], pz[PTS];
+  uint32_t md[PTS], oi[PTS];  // running min distance (bits), index
   // loads at clamped slots, values selected after (a load under `q < n` became a branch and a
   // wait before the next slot's)
 #pragma unroll
@@ -370,24 +392,21 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     px[s] = in ? x : 0.f;
     py[s] = in ? y : 0.f;
     pz[s] = in ? z : 0.f;
-    md[s] = in ? __builtin_inff() : 0.f;  // padding: never changes, never wins
+    md[s] = in ? 0x7f800000u : 0u;  // padding: never changes, never wins
   }
-  __syncthreads();  // order[] is dead: the scratch becomes the position table
-  // every point sits in exactly one slot (order is a permutation of 0..n-1, PTS * THREADS >= n):
-  // the table is written from the registers instead of read from memory again
-#pragma unroll
-  for (int s = 0; s < PTS; ++s)
-    if (oi[s] != 0xffffffffu) table[oi[s]] = make_float4(px[s], py[s], pz[s], 0.f);
-  if (t < 2) slots[t] = 0ull;
 
-  // 4. bucket records: box in lane s (bucket of slot s); max min-distance bits, lowest index
-  //    attaining the max and the lane holding that point as scalars bm[s], bi[s], al[s].
-  float blx = __builtin_inff(), bly = __builtin_inff(), blz = __builtin_inff();
-  float bhx = -__builtin_inff(), bhy = -__builtin_inff(), bhz = -__builtin_inff();
-  uint32_t bmax = 0u;
-  // Bucket records are wave-uniform, kept as scalars; bmax (lane s = bucket s) is the per-lane
-  // copy of bm the bound test reads.
-  uint32_t bm[PTS], bi[PTS], al[PTS];  // al: lane holding the max (lowest index), kWave = unknown
+  // 4. bucket records: box and max (bits) of slot 4 h + lane / 16 in the lane; the farthest point
+  //    (bits, index, lane, position) and the rest bound of slot s as scalars.
+  float blx[TESTS], bly[TESTS], blz[TESTS], bhx[TESTS], bhy[TESTS], bhz[TESTS];
+  uint32_t bmax[TESTS];
+  uint32_t bm[PTS], bi[PTS], al[PTS], rs[PTS];  // al: lane holding the max, kWave = unknown
+  float sx[PTS], sy[PTS], sz[PTS];
+#pragma unroll
+  for (int h = 0; h < TESTS; ++h) {
+    blx[h] = bly[h] = blz[h] = __builtin_inff();
+    bhx[h] = bhy[h] = bhz[h] = -__builtin_inff();
+    bmax[h] = 0u;
+  }
 #pragma unroll
   for (int s = 0; s < PTS; ++s) {
     const bool valid = oi[s] != 0xffffffffu;
@@ -397,86 +416,138 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const uint32_t h0 = wave_max_u32(valid ? float_order_key(px[s]) : 0u);
     const uint32_t h1 = wave_max_u32(valid ? float_order_key(py[s]) : 0u);
     const uint32_t h2 = wave_max_u32(valid ? float_order_key(pz[s]) : 0u);
-    const uint32_t mi = wave_min_u32(oi[s]);
-    bm[s] = mi != 0xffffffffu ? 0x7f800000u : 0u;
-    bi[s] = 0xffffffffu;
+    const bool any = (s * WAVES + w) * kWave < n;
+    // until the first update (all buckets take part in it): lane 0's point, nothing known
+    bm[s] = any ? 0x7f800000u : 0u;
+    bi[s] = __builtin_amdgcn_readfirstlane(oi[s]);
     al[s] = kWave;
-    if (lane == s && mi != 0xffffffffu) {
-      blx = float_from_order_key(l0); bly = float_from_order_key(l1); blz = float_from_order_key(l2);
-      bhx = float_from_order_key(h0); bhy = float_from_order_key(h1); bhz = float_from_order_key(h2);
-      bmax = 0x7f800000u;  // +inf: every bucket takes part in the first update
+    rs[s] = 0x7f800000u;
+    sx[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(px[s])));
+    sy[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(py[s])));
+    sz[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(pz[s])));
+    if (lane / 16 == s % 4 && any) {
+      blx[s / 4] = float_from_order_key(l0); bly[s / 4] = float_from_order_key(l1);
+      blz[s / 4] = float_from_order_key(l2); bhx[s / 4] = float_from_order_key(h0);
+      bhy[s / 4] = float_from_order_key(h1); bhz[s / 4] = float_from_order_key(h2);
+      bmax[s / 4] = 0x7f800000u;
     }
+    if (lane == 0) rkey[s * WAVES + w] = fps_key(bm[s], bi[s]);
   }
-  float cx = P[0], cy = P[1], cz = P[2];
-  if (t == 0) out_idx[o0] = start;
-  // The wave's best (bits, index), recomputed only after one of its buckets changed.
-  uint32_t wbits = 0u, widx = 0xffffffffu;
-  bool dirty = true;
-  __syncthreads();
+  if (t == 0) {
+    list[0] = make_float4(P[0], P[1], P[2], 0.f);
+    lkey[0] = make_uint2(0u, 0u);
+  }
+  lds_barrier();
 
-  for (int it = 1; it < k; ++it) {
-    float gx, gy, gz;
-    {
-#pragma clang fp contract(off)
-      gx = fmaxf(fmaxf(blx - cx, cx - bhx), 0.f);
-      gy = fmaxf(fmaxf(bly - cy, cy - bhy), 0.f);
-      gz = fmaxf(fmaxf(blz - cz, cz - bhz), 0.f);
-    }
-    const float lb = sqdist(gx, gy, gz, 0.f, 0.f, 0.f);
-    const uint64_t act = __ballot(__float_as_uint(lb) < bmax);  // bmax = 0 on lanes >= PTS
-    if (act) {
+  // records that exist: no more can be taken in one round
+  const int cap = min(kFpsRound, (n + kWave - 1) / kWave);
+  const int li = lane & (kFpsRound - 1);
+  int done = 0;
+  for (;;) {
+    // which of the listed records are the next centroids: record j is one if no record i ahead of
+    // it can lower its point, and no other point of a bucket ahead can reach it
+    const float4 c = list[li];
+    int A = 1;
+    if (done != 0) {
+      A = kFpsRound;
 #pragma unroll
-      for (int s = 0; s < PTS; ++s) {
-        if (act & (1ull << s)) {
-          // distances are non-negative floats, ordered like their bit patterns: the running
-          // minimum is an integer min (no NaN canonicalisation step)
-          const float d = sqdist(px[s], py[s], pz[s], cx, cy, cz);
-          const uint32_t old = __float_as_uint(md[s]);
-          const uint32_t mb = min(__float_as_uint(d), old);
-          md[s] = __uint_as_float(mb);
-          // Values only fall: while the point holding the bucket's max keeps its value, the
-          // record (max, lowest index attaining it) stands.  Most touched buckets end here.
-          if (al[s] < static_cast<uint32_t>(kWave) && !((__ballot(mb < old) >> al[s]) & 1ull))
-            continue;
-          const uint32_t m = wave_max_u32(mb);
-          bm[s] = m;
-          if (lane == s) bmax = m;
-          const uint64_t hit = __ballot(mb == m);
-          if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
-            al[s] = static_cast<uint32_t>(__builtin_ctzll(hit));
-            bi[s] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(oi[s]), al[s]));
-          } else {
-            bi[s] = wave_min_u32(mb == m ? oi[s] : 0xffffffffu);
-            al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(mb == m && oi[s] == bi[s]) | (1ull << 63)));
-          }
-          dirty = true;
+      for (int g = 0; g < kFpsRound; g += 8) {  // four records per step, lane = 16 * record + i
+        const int j0 = g + lane / 16, j1 = j0 + 4;
+        const float4 p0 = list[j0], p1 = list[j1];
+        const uint32_t k0 = lkey[j0].x, k1 = lkey[j1].x;
+        const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
+        const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
+        const uint32_t rb = __float_as_uint(c.w);
+        const uint64_t b0 = (__ballot(d0 < k0) | __ballot(rb >= k0)) & __ballot(li < j0);
+        const uint64_t b1 = (__ballot(d1 < k1) | __ballot(rb >= k1)) & __ballot(li < j1);
+        if (b0 | b1) {
+          A = g + (b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16;
+          break;
         }
       }
+      A = min(min(A, cap), k - done);
     }
-    if (dirty) {
-      // wave best: the largest bucket max, then the lowest index among the buckets holding it
-      // (all scalars)
-      uint32_t wb = 0u;
+    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + lkey[li].y;
+    done += A;
+    if (done >= k) break;
+
+    // update: the wave's buckets against the round's centroids
 #pragma unroll
-      for (int s = 0; s < PTS; ++s) wb = bm[s] > wb ? bm[s] : wb;
-      wbits = wb;
-      uint32_t best = 0xffffffffu;
+    for (int h = 0; h < TESTS; ++h) {
+      float gx, gy, gz;
+      {
+#pragma clang fp contract(off)
+        gx = fmaxf(fmaxf(blx[h] - c.x, c.x - bhx[h]), 0.f);
+        gy = fmaxf(fmaxf(bly[h] - c.y, c.y - bhy[h]), 0.f);
+        gz = fmaxf(fmaxf(blz[h] - c.z, c.z - bhz[h]), 0.f);
+      }
+      const float lb = sqdist(gx, gy, gz, 0.f, 0.f, 0.f);
+      const uint64_t act = __ballot(li < A && __float_as_uint(lb) < bmax[h]);
+      if (!act) continue;
 #pragma unroll
-      for (int s = 0; s < PTS; ++s) best = (bm[s] == wb && bi[s] < best) ? bi[s] : best;
-      widx = best;
-      dirty = false;
+      for (int s = 4 * h; s < PTS && s < 4 * h + 4; ++s) {
+        uint32_t m = static_cast<uint32_t>(act >> (16 * (s % 4))) & 0xffffu;
+        if (!m) continue;
+        const uint32_t old = md[s];
+        uint32_t mb = old;
+        do {
+          const int l = __builtin_ctz(m);
+          m &= m - 1;
+          const float cx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.x), l));
+          const float cy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.y), l));
+          const float cz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.z), l));
+          // distances are non-negative floats, ordered like their bit patterns: the running
+          // minimum is an integer min (no NaN canonicalisation step)
+          mb = min(mb, __float_as_uint(sqdist(px[s], py[s], pz[s], cx, cy, cz)));
+        } while (m);
+        md[s] = mb;
+        // Values only fall: while the point holding the bucket's max keeps its value, the record
+        // (max, lowest index attaining it) stands, and its rest bound still holds.
+        if (al[s] < static_cast<uint32_t>(kWave) && !((__ballot(mb < old) >> al[s]) & 1ull))
+          continue;
+        const uint32_t mx = wave_max_u32(mb);
+        const uint64_t hit = __ballot(mb == mx);
+        if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
+          al[s] = static_cast<uint32_t>(__builtin_ctzll(hit));
+          bi[s] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(oi[s]), al[s]));
+        } else {
+          bi[s] = wave_min_u32(mb == mx ? oi[s] : 0xffffffffu);
+          al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(mb == mx && oi[s] == bi[s]) | (1ull << 63)));
+        }
+        bm[s] = mx;
+        if (lane / 16 == s % 4) bmax[h] = mx;
+        if (lane == 0) rkey[s * WAVES + w] = fps_key(mx, bi[s]);
+        sx[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
+        sy[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
+        sz[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
+        // what the bucket's other points can reach once that point is a centroid (its own lane
+        // gives 0)
+        rs[s] = wave_max_u32(
+            min(mb, __float_as_uint(sqdist(px[s], py[s], pz[s], sx[s], sy[s], sz[s]))));
+      }
     }
-    // one lane of the wave issues the atomic (the build turns the atomic optimizer off for this
-    // file: its single-lane election would add three dependent VALU steps before the barrier)
-    if (lane == 0)
-      atomicMax(&slots[it & 1], (static_cast<unsigned long long>(it) << 45) |
-                                    (static_cast<unsigned long long>(wbits) << 13) |
-                                    static_cast<unsigned long long>(8191u - (widx & 8191u)));
     lds_barrier();  // waves share only LDS in this loop
-    const uint32_t gidx = 8191u - (static_cast<uint32_t>(slots[it & 1]) & 8191u);
-    const float4 c = table[gidx];
-    cx = c.x; cy = c.y; cz = c.z;
-    if (t == 0) out_idx[o0 + it] = start + gidx;
+
+    // rank: every wave places its own records among all of them and lists the first kFpsRound
+    double kk[SETS];
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) {
+      const int i = e * kWave + lane;
+      kk[e] = rkey[i < NB ? i : 0];
+      if (NB < kWave && i >= NB) kk[e] = 0.0;  // no key is below 0
+    }
+#pragma unroll
+    for (int s = 0; s < PTS; ++s) {
+      const double kj = fps_key(bm[s], bi[s]);
+      int rank = 0;
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) rank += __builtin_popcountll(__ballot(kk[e] > kj));
+      if (rank < kFpsRound && (s * WAVES + w) * kWave < n && lane == 0) {
+        list[rank] = make_float4(sx[s], sy[s], sz[s], __uint_as_float(rs[s]));
+        lkey[rank] = make_uint2(bm[s], bi[s]);
+      }
+    }
+    lds_barrier();
   }
 }
 
@@ -484,10 +555,10 @@ template <int PTS, int THREADS>
 int launch_bucket(const float* pos, const int64_t* ptr, const int64_t* out_ptr, int64_t B,
                   int64_t max_cloud, int64_t* out, hipStream_t st,
                   const int64_t* guard = nullptr) {
-  const size_t lds = static_cast<size_t>(max_cloud > 0 ? max_cloud : 1) * sizeof(float4);
+  const size_t lds = static_cast<size_t>(max_cloud > 0 ? max_cloud : 1) * 12;
   GEO_HIP_CHECK(hipFuncSetAttribute(
       reinterpret_cast<const void*>(&fps_bucket_kernel<PTS, THREADS>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFpsLdsPoints * sizeof(float4))));
+      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFpsLdsPoints * 12)));
   hipLaunchKernelGGL((fps_bucket_kernel<PTS, THREADS>), dim3(B), dim3(THREADS), lds, st, pos, ptr,
                      out_ptr, out, guard);
   GEO_LAUNCH_CHECK("fps_bucket_kernel");

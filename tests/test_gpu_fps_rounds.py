@@ -1,0 +1,35 @@
+"""Farthest point sampling takes several centroids per round where the greedy order allows it: the
+sequence must be the one-at-a-time one at the sizes and point sets where a round ends early."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(kind: str, n: int, seed: int) -> torch.Tensor:
+    g = torch.Generator().manual_seed(seed)
+    if kind == "cube":
+        return torch.rand(n, 3, generator=g)
+    if kind == "clumps":  # a few dense clumps far apart: the farthest points share buckets
+        c = torch.randn(7, 3, generator=g) * 10
+        return c[torch.randint(0, 7, (n,), generator=g)] + 0.01 * torch.randn(n, 3, generator=g)
+    if kind == "lattice":  # equal distances and repeated points everywhere
+        return torch.randint(0, 7, (n, 3), generator=g).float()
+    if kind == "line":  # boxes without volume, equal gaps
+        return torch.stack([torch.randperm(n, generator=g).float(), torch.zeros(n), torch.ones(n)], 1)
+    return torch.full((n, 3), 0.25)  # one point n times: every distance 0
+
+
+@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "line", "same"])
+@pytest.mark.parametrize("sizes", [[2, 63, 64, 65], [1023, 1024, 1025], [2048, 2049], [4096, 1, 130], [8192]])
+def test_fps_rounds_follow_the_greedy_order(kind, sizes):
+    from gdl_amd.csrc import fps_cuda
+    pos = _points(kind, sum(sizes), sum(sizes))
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    k = np.array([max(1, (3 * n) // 5) for n in sizes])
+    got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
+    np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
