@@ -826,13 +826,13 @@ def fps_uniform_hip(pos: Tensor, ptr: Tensor, num_samples: int) -> Tensor:
             return out
         ws_bytes = L.geo_fps_workspace_bytes(B, N, max_n)
         ws = _nat.workspace(ws_bytes, dev)
-        _nat.check(L.geo_fps(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n,
-                             _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
+        _nat.check(L.geo_fps_total(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, total,
+                                   _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
     return out
 
 
 def _fps_run(pos: Tensor, p: Tensor, B: int, prepare) -> Tensor:
-    """prepare (offsets, total, largest cloud, validity) -> one host sync -> geo_fps."""
+    """prepare (offsets, total, largest cloud, validity) -> one host sync -> geo_fps_total."""
     dev = pos.device
     N = pos.shape[0]
     L = _nat.lib()
@@ -850,8 +850,8 @@ def _fps_run(pos: Tensor, p: Tensor, B: int, prepare) -> Tensor:
             return out
         ws_bytes = L.geo_fps_workspace_bytes(B, N, max_n)
         ws = _nat.workspace(ws_bytes, dev)
-        _nat.check(L.geo_fps(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n,
-                             _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
+        _nat.check(L.geo_fps_total(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, total,
+                                   _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
     return out
 
 

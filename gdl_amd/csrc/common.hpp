@@ -187,6 +187,14 @@ __device__ __forceinline__ uint64_t wave_inclusive_sum_dpp(uint64_t v) {
   return v;
 }
 
+// Max over each 16-lane row (every lane must be active), the row's result in all its lanes.
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
+  v = max(v, dpp0_u32<kDppXor1>(v));
+  v = max(v, dpp0_u32<kDppXor2>(v));
+  v = max(v, dpp0_u32<kDppHalfMirror>(v));
+  return max(v, dpp0_u32<kDppMirror>(v));
+}
+
 // Max / min over lanes 0..15 only (row 0); other lanes' values are ignored.
 __device__ __forceinline__ uint32_t row0_max_u32(uint32_t v) {
   v = max(v, dpp0_u32<kDppXor1>(v));

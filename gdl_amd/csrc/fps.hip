@@ -10,18 +10,16 @@
 //     a compact bucket of 64 points; a bucket is only updated when a new centroid can lower
 //     one of its distances (an exact test, see below), and several centroids are taken from the
 //     cached per-bucket maxima per round, where they provably follow each other.
-//   register (8193 to 16384 points): thread t owns local points t, t+256, ... (PTS of them)
-//     with x, y, z and the running min distance in VGPRs; every point is updated every
-//     iteration.
-//   large (16385 to 196,608 points): the bucket scheme with points sorted along the Hilbert
-//     curve in the workspace and bucket records in registers (see its section below).
+//   register (8193 to 16384 points, few samples): thread t owns local points t, t+256, ... with x,
+//     y, z and the running min distance in VGPRs; every point is updated every iteration.
+//   large (8193 to 196,608 points): the bucket scheme with points sorted along the Hilbert curve
+//     in the workspace and bucket records in LDS (see its section below).
 //   streaming (larger clouds): positions read from HBM/L2 each iteration, running min
 //     distance in the workspace.
-// The register, large and streaming kernels reduce (distance bits, index) per iteration to one
-// winner with one barrier: a wave max of the bits (DPP), the lowest index among the lanes holding
-// it, then either one LDS record per wave double-buffered by iteration parity (register,
-// streaming) or one LDS 64-bit atomic max per wave on a (distance, index complement) key (large).
-// Squared distances are non-negative floats, whose bit patterns order like the values.
+// The register and streaming kernels reduce (distance bits, index) per iteration to one winner
+// with one barrier: a wave max of the bits (DPP), the lowest index among the lanes holding it, then
+// one LDS record per wave double-buffered by iteration parity.  Squared distances are non-negative
+// floats, whose bit patterns order like the values.
 #include "radix.hpp"
 
 namespace geo {
@@ -29,7 +27,9 @@ namespace {
 
 constexpr int kFpsThreads = 256;
 constexpr int kFpsWaves = kFpsThreads / kWave;
-constexpr int kFpsLdsPoints = 8192;  // register kernel centroid table: 8192 * 16 B of LDS
+constexpr int kFpsLdsPoints = 8192;         // largest cloud of the bucketed kernel
+constexpr int kFpsRegisterPoints = 16384;   // largest cloud of the register kernel
+constexpr int kFpsRegisterSamples = 80;     // most samples per cloud it is chosen for
 constexpr int kFpsBucketThreads = 1024;
 constexpr int kFpsRound = 16;  // most centroids that one round of the bucketed kernel takes
 constexpr int kFpsStreamThreads = 1024;
@@ -94,12 +94,11 @@ __device__ __forceinline__ void wave_argmax(uint32_t bits, uint32_t idx, uint32_
   widx = wave_min_u32(bits == wbits ? idx : 0xffffffffu);
 }
 
-template <int PTS, bool LDS_POS>
+template <int PTS>
 __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
     const float* __restrict__ pos, const int64_t* __restrict__ ptr,
     const int64_t* __restrict__ out_ptr, int64_t* __restrict__ out_idx) {
   __shared__ FpsSlot slots[2][kFpsWaves];
-  extern __shared__ float4 table[];  // LDS_POS: local positions, n entries
 
   const int b = blockIdx.x;
   const int64_t start = ptr[b];
@@ -124,7 +123,6 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
       py[s] = P[3 * l + 1];
       pz[s] = P[3 * l + 2];
       md[s] = __builtin_inff();
-      if constexpr (LDS_POS) table[l] = make_float4(px[s], py[s], pz[s], 0.f);
     } else {
       px[s] = py[s] = pz[s] = 0.f;
       md[s] = 0.f;  // never wins: its index is above every valid one
@@ -132,7 +130,6 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
   }
   float cx = P[0], cy = P[1], cz = P[2];
   if (t == 0) out_idx[o0] = start;
-  if constexpr (LDS_POS) __syncthreads();
 
   for (int it = 1; it < k; ++it) {
     uint32_t bbits = 0, bidx = 0xffffffffu;
@@ -164,12 +161,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
       }
     }
     gidx = __builtin_amdgcn_readfirstlane(gidx);
-    if constexpr (LDS_POS) {
-      const float4 c = table[gidx];
-      cx = c.x; cy = c.y; cz = c.z;
-    } else {
-      cx = P[3 * gidx]; cy = P[3 * gidx + 1]; cz = P[3 * gidx + 2];
-    }
+    cx = P[3 * gidx]; cy = P[3 * gidx + 1]; cz = P[3 * gidx + 2];
     if (t == 0) out_idx[o0 + it] = start + gidx;
   }
 }
@@ -620,26 +612,35 @@ __global__ __launch_bounds__(kFpsStreamThreads) void fps_stream_kernel(
 }
 
 // ---------------------------------------------------------------------------- large clouds ---
-// Clouds larger than the register kernel holds (up to kFpsLargeMaxPoints).  The batch is
+// Clouds larger than the bucketed kernel holds (up to kFpsLargeMaxPoints).  The batch is
 // reordered by a device radix sort on (cloud + 1, Hilbert position of the point in its cloud's
 // box), which keeps every cloud on its own index range, and each cloud is cut into buckets of 64
 // consecutive sorted points.  Positions (with the original index) and running min distances
 // stay in the workspace, 20 bytes per point, which for one cloud fits the L2 of the XCD that
-// runs it.  One 1024-thread workgroup per cloud; lane l of wave w holds the records of buckets
-// w + 16 (l + 64 r), r < kFpsLargeSlots: box, max min-distance, lowest index attaining it, the
-// lane of that point and its position.  Per iteration each wave tests its buckets with the exact
-// lower bound above, reloads and updates only the buckets the new centroid can change (two at a
-// time, so their loads overlap), re-reduces a bucket's record only when the point holding its
-// maximum fell (C5: 12% of touched buckets), rescans its best (distance, index) only when the
-// bucket that best came from changed (about one wave per iteration: the winner's), and the
-// workgroup agrees on the winner with one LDS 64-bit atomic max per wave on
-// (bits << 32) | (index complement << 4 | wave) and one LDS-only barrier.
+// runs it.  One 1024-thread workgroup per cloud takes several centroids per round, by the rule of
+// the bucketed kernel over the records in LDS:
+//   check   the listed records pairwise (every wave)
+//   test    boxes of 64 buckets against all centroids, then the buckets of the boxes that one may
+//           reach; touched buckets join a queue with the set of their centroids
+//   update  the queue shared by all waves, three buckets of a wave loaded together; records whose
+//           farthest point fell are re-reduced and their groups marked
+//   groups  buckets g, g + 128, ... form group g, so neighbouring buckets lie in different groups;
+//           best and second record of the marked groups, one 16-lane row each
+//   rank    no record other than a group's best exceeds the largest second record t0, so the bests
+//           above t0, in order, are the next records of the whole cloud: the list
+// A 131,072-point lidar frame to 16,384 samples: 1,634 rounds of 10.0 centroids and 5.5 us,
+// 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,200 cycles issues 455
+// vector instructions per wave (59% of what the CU's four SIMDs can issue in that time), 290 of
+// them in update.  Tried without gain: the queue's buckets handed to whichever wave is free (9.3 ms),
+// tests per 16 buckets with a centroid list per row (9.3), one bucket prefetched ahead (9.6), four
+// or eight loaded together (9.2, 9.6), min distances stored only where they fell (9.5: the
+// conditional store makes every later load wait for it).
 constexpr int kFpsLargeThreads = 1024;
 constexpr int kFpsLargeWaves = kFpsLargeThreads / kWave;
 constexpr int kFpsLargeSlots = 3;
+constexpr int kFpsLargeBatch = 3;  // a wave's queued buckets loaded together
 constexpr int64_t kFpsLargeMaxPoints =
     static_cast<int64_t>(kFpsLargeSlots) * kFpsLargeThreads * kWave;  // 196,608
-constexpr uint32_t kFpsLargeIdxMask = (1u << 18) - 1;                  // local index < 2^18
 constexpr int64_t kFpsLargeMaxClouds = (1 << 11) - 2;                  // cloud id + 1 in 11 bits
 
 // bbox[6 b .. 6 b + 5] = (lo x, lo y, lo z, hi x, hi y, hi z) of cloud b; one block per cloud.
@@ -704,25 +705,64 @@ __global__ void fps_large_keys_kernel(const float* __restrict__ pos, const int64
   keys[i] = (static_cast<uint32_t>(lo) << (3 * mbits)) | code;
 }
 
-// Sorted position j <- original point order[j]: (x, y, z, original index bits); md = +inf.
-__global__ void fps_large_gather_kernel(const float* __restrict__ pos,
-                                        const uint32_t* __restrict__ order, int64_t N,
-                                        float4* __restrict__ q, float* __restrict__ md) {
-  const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= N) return;
-  const uint32_t i = order[j];
-  q[j] = make_float4(pos[3 * static_cast<int64_t>(i)], pos[3 * static_cast<int64_t>(i) + 1],
-                     pos[3 * static_cast<int64_t>(i) + 2], __uint_as_float(i));
-  md[j] = __builtin_inff();
+// Bucket j of cloud b (64 sorted points, one wave): positions and original index bits in sorted
+// order, min distances +inf, and the bucket's box at boxes[a][fps_large_box0 + j] (lo x, y, z,
+// hi x, y, z by a).
+__device__ __forceinline__ int64_t fps_large_box0(int64_t start, int b) { return (start >> 6) + b; }
+
+__global__ __launch_bounds__(256) void fps_large_gather_kernel(
+    const float* __restrict__ pos, const uint32_t* __restrict__ order, const int64_t* __restrict__ ptr,
+    int64_t box_stride, float4* __restrict__ q, uint32_t* __restrict__ md, float* __restrict__ boxes) {
+  const int b = blockIdx.y;
+  const int64_t start = ptr[b], n = ptr[b + 1] - start;
+  const int64_t j = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
+  if (j * kWave >= n) return;
+  const int lane = lane_id();
+  const int64_t l = j * kWave + lane;
+  const int64_t at = start + (l < n ? l : n - 1);  // past the end: the last point again
+  const uint32_t i = order[at];
+  const float x = pos[3 * static_cast<int64_t>(i)], y = pos[3 * static_cast<int64_t>(i) + 1],
+              z = pos[3 * static_cast<int64_t>(i) + 2];
+  if (l < n) {
+    q[at] = make_float4(x, y, z, __uint_as_float(i));
+    md[at] = 0x7f800000u;
+  }
+  const uint32_t kx = float_order_key(x), ky = float_order_key(y), kz = float_order_key(z);
+  const float bx[6] = {float_from_order_key(wave_min_u32(kx)), float_from_order_key(wave_min_u32(ky)),
+                       float_from_order_key(wave_min_u32(kz)), float_from_order_key(wave_max_u32(kx)),
+                       float_from_order_key(wave_max_u32(ky)), float_from_order_key(wave_max_u32(kz))};
+  if (lane == 0) {
+#pragma unroll
+    for (int a = 0; a < 6; ++a) boxes[a * box_stride + fps_large_box0(start, b) + j] = bx[a];
+  }
 }
 
+// Bytes of dynamic LDS for clouds of up to nb buckets.
+constexpr int kFpsLargeGroups = 128;
+__host__ __device__ inline size_t fps_large_lds(int nb) {
+  return static_cast<size_t>(nb) * (sizeof(float4) + sizeof(double) + sizeof(uint32_t) + sizeof(uint16_t)) +
+         kFpsLargeGroups * sizeof(uint16_t) + 16;
+}
+
+template <int S>
 __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
-    const float* __restrict__ pos, const float4* __restrict__ Qall, float* __restrict__ Mall,
+    const float* __restrict__ pos, const float4* __restrict__ Qall, uint32_t* __restrict__ Mall,
+    const float* __restrict__ boxes, int64_t box_stride, int nb_max,
     const int64_t* __restrict__ ptr, const int64_t* __restrict__ out_ptr,
     int64_t* __restrict__ out_idx) {
-  constexpr int S = kFpsLargeSlots;
-  __shared__ unsigned long long slots[3];
-  __shared__ float4 cand[2][kFpsLargeWaves];
+  constexpr int G = kFpsLargeGroups;
+  constexpr int W = kFpsLargeWaves;
+  extern __shared__ float4 large_lds[];
+  float4* rec = large_lds;                                       // farthest point, (bits) rest bound
+  double* rkey = reinterpret_cast<double*>(rec + nb_max);        // its key, see fps_key
+  uint32_t* queue = reinterpret_cast<uint32_t*>(rkey + nb_max);  // bucket << 16 | centroids
+  uint16_t* dirty = reinterpret_cast<uint16_t*>(queue + nb_max); // groups whose records changed
+  __shared__ double gkey[G];         // best record of each group (buckets g, g + G, ...)
+  __shared__ uint32_t gbkt[G], gsec[G];  // its bucket; distance bits of the group's second record
+  __shared__ float4 list[kFpsRound];
+  __shared__ uint2 lkey[kFpsRound];
+  __shared__ int n_queue, n_dirty;
+
   const int b = blockIdx.x;
   const int64_t start = ptr[b];
   const int n = static_cast<int>(ptr[b + 1] - start);
@@ -737,207 +777,277 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
     return;
   }
   const float4* Q = Qall + start;
-  float* M = Mall + start;
+  uint32_t* M = Mall + start;
   const int nb = (n + kWave - 1) / kWave;
   const uint32_t ustart = static_cast<uint32_t>(start);
+  const int li = lane & (kFpsRound - 1);
+  const int row = lane / 16;
 
-  // Bucket records of this lane (empty buckets: +inf box, max 0, never tested or chosen).
-  float blx[S], bly[S], blz[S], bhx[S], bhy[S], bhz[S], bcx[S], bcy[S], bcz[S];
-  uint32_t bmax[S], bidx[S], blane[S];  // blane: lane (point) holding the max, 64 = unknown
+  // Slot r of wave w holds the boxes of buckets 64 (w + 16 r) + lane; lane 16 r + c (any c) the
+  // box of the whole slot and a bound of its records' distances.
+  float blx[S], bly[S], blz[S], bhx[S], bhy[S], bhz[S];
+  float slx = __builtin_inff(), sly = slx, slz = slx, shx = -slx, shy = -slx, shz = -slx;
+  uint32_t smax = 0u;
 #pragma unroll
   for (int r = 0; r < S; ++r) {
-    blane[r] = kWave;
-    blx[r] = bly[r] = blz[r] = __builtin_inff();
-    bhx[r] = bhy[r] = bhz[r] = -__builtin_inff();
-    bcx[r] = bcy[r] = bcz[r] = 0.f;
-    bmax[r] = 0u;
-    bidx[r] = 0xffffffffu;
-    const int bk = w + kFpsLargeWaves * (lane + kWave * r);
-    if (bk < nb) {
-      const int q0 = bk * kWave;
-      const int q1 = min(q0 + kWave, n);
-#pragma unroll 8
-      for (int q = q0; q < q1; ++q) {
-        const float4 p = Q[q];
-        blx[r] = fminf(blx[r], p.x); bly[r] = fminf(bly[r], p.y); blz[r] = fminf(blz[r], p.z);
-        bhx[r] = fmaxf(bhx[r], p.x); bhy[r] = fmaxf(bhy[r], p.y); bhz[r] = fmaxf(bhz[r], p.z);
-        const uint32_t li = __float_as_uint(p.w) - ustart;
-        if (li < bidx[r]) { bidx[r] = li; bcx[r] = p.x; bcy[r] = p.y; bcz[r] = p.z; }
-      }
-      bmax[r] = 0x7f800000u;  // +inf: every bucket takes part in the first update
+    const int bk = kWave * (w + W * r) + lane;
+    const bool in = bk < nb;
+    const float* bx = boxes + fps_large_box0(start, b) + (in ? bk : 0);
+    const float v[6] = {bx[0], bx[box_stride], bx[2 * box_stride], bx[3 * box_stride],
+                        bx[4 * box_stride], bx[5 * box_stride]};
+    blx[r] = in ? v[0] : __builtin_inff();
+    bly[r] = in ? v[1] : __builtin_inff();
+    blz[r] = in ? v[2] : __builtin_inff();
+    bhx[r] = in ? v[3] : -__builtin_inff();
+    bhy[r] = in ? v[4] : -__builtin_inff();
+    bhz[r] = in ? v[5] : -__builtin_inff();
+    const float l0 = float_from_order_key(wave_min_u32(float_order_key(blx[r])));
+    const float l1 = float_from_order_key(wave_min_u32(float_order_key(bly[r])));
+    const float l2 = float_from_order_key(wave_min_u32(float_order_key(blz[r])));
+    const float h0 = float_from_order_key(wave_max_u32(float_order_key(bhx[r])));
+    const float h1 = float_from_order_key(wave_max_u32(float_order_key(bhy[r])));
+    const float h2 = float_from_order_key(wave_max_u32(float_order_key(bhz[r])));
+    if (row == r && kWave * (w + W * r) < nb) {
+      slx = l0; sly = l1; slz = l2; shx = h0; shy = h1; shz = h2;
+      smax = 0x7f800000u;  // +inf: every bucket takes part in the first update
+    }
+    if (in) {  // until then: the bucket's first point, nothing known
+      const float4 p = Q[bk * kWave];
+      rec[bk] = make_float4(p.x, p.y, p.z, __builtin_inff());
+      rkey[bk] = fps_key(0x7f800000u, __float_as_uint(p.w) - ustart);
     }
   }
-  float cx = pos[3 * start], cy = pos[3 * start + 1], cz = pos[3 * start + 2];
+  if (t < G) dirty[t] = static_cast<uint16_t>(t);  // every group is formed in the first round
   if (t == 0) {
-    out_idx[o0] = start;
-    slots[0] = slots[1] = slots[2] = 0ull;
+    list[0] = make_float4(pos[3 * start], pos[3 * start + 1], pos[3 * start + 2], 0.f);
+    lkey[0] = make_uint2(0u, 0u);
+    n_queue = 0;
+    n_dirty = G;
   }
-  unsigned long long best_key = 0ull;
-  float4 best_c = make_float4(0.f, 0.f, 0.f, 0.f);
-  bool dirty = true;
-  int best_r = -1, best_l = 0;  // the bucket the wave's best record comes from (slot, lane)
   __syncthreads();
 
-  // slots that hold buckets at all: slot r holds buckets [1024 r, 1024 (r + 1)); the others are
-  // neither tested nor searched
-  const int s_used = (nb + kFpsLargeThreads - 1) / kFpsLargeThreads;
-
-  for (int it = 1; it < k; ++it) {
-    uint64_t act[S];
+  int done = 0, cap = 1;
+  for (;;) {
+    // check: as in the bucketed kernel, over the listed records
+    const float4 c = list[li];
+    int A = cap;
+    if (cap > 1) {
 #pragma unroll
-    for (int r = 0; r < S; ++r) {
-      act[r] = 0ull;
-      if (r < s_used) {  // wave-uniform
-        float gx, gy, gz;
-        {
-#pragma clang fp contract(off)
-          gx = fmaxf(fmaxf(blx[r] - cx, cx - bhx[r]), 0.f);
-          gy = fmaxf(fmaxf(bly[r] - cy, cy - bhy[r]), 0.f);
-          gz = fmaxf(fmaxf(blz[r] - cz, cz - bhz[r]), 0.f);
+      for (int g = 0; g < kFpsRound; g += 8) {  // four records per step, lane = 16 * record + i
+        const int j0 = g + row, j1 = j0 + 4;
+        const float4 p0 = list[j0], p1 = list[j1];
+        const uint32_t k0 = lkey[j0].x, k1 = lkey[j1].x;
+        const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
+        const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
+        const uint32_t rb = __float_as_uint(c.w);
+        const uint64_t b0 = (__ballot(d0 < k0) | __ballot(rb >= k0)) & __ballot(li < j0);
+        const uint64_t b1 = (__ballot(d1 < k1) | __ballot(rb >= k1)) & __ballot(li < j1);
+        if (b0 | b1) {
+          A = min(A, g + static_cast<int>(b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16);
+          break;
         }
-        const float lb = sqdist(gx, gy, gz, 0.f, 0.f, 0.f);
-        act[r] = __ballot(__float_as_uint(lb) < bmax[r]);
       }
     }
-    while (act[0] | act[1] | act[2]) {
-      // up to two affected buckets of this wave per round, their loads issued together (C5:
-      // two per round 27.3 ms, three 27.4, four 28.8: fewer rounds for the busiest wave, but
-      // every slot of a round costs its selection, address and bookkeeping)
-      constexpr int G = 2;
-      int rr[G], ll[G];
-#pragma unroll
-      for (int j = 0; j < G; ++j) {
-        rr[j] = act[0] ? 0 : (act[1] ? 1 : (act[2] ? 2 : -1));
-        ll[j] = 0;
-        if (rr[j] >= 0) {
-          const uint64_t m = rr[j] == 0 ? act[0] : (rr[j] == 1 ? act[1] : act[2]);
-          ll[j] = __builtin_ctzll(m);
-          const uint64_t cleared = m & (m - 1);
-          if (rr[j] == 0) act[0] = cleared; else if (rr[j] == 1) act[1] = cleared; else act[2] = cleared;
-        }
+    A = min(A, k - done);
+    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + lkey[li].y;
+    done += A;
+    if (done >= k) break;
+
+    // test: slots against centroids, lane = 16 * slot + centroid, then the buckets of the slots that
+    // a centroid may reach
+    {
+      float gx, gy, gz;
+      {
+#pragma clang fp contract(off)
+        gx = fmaxf(fmaxf(slx - c.x, c.x - shx), 0.f);
+        gy = fmaxf(fmaxf(sly - c.y, c.y - shy), 0.f);
+        gz = fmaxf(fmaxf(slz - c.z, c.z - shz), 0.f);
       }
-      float4 p[G];
-      float mo[G];
-      bool v[G];
+      const float slb = sqdist(gx, gy, gz, 0.f, 0.f, 0.f);
+      const uint64_t act = __ballot(__float_as_uint(slb) < smax) & __ballot(li < A);
+      if (act) {
+        uint32_t touched[S];
+        int total = 0;
 #pragma unroll
-      for (int j = 0; j < G; ++j) {
-        const int q = (w + kFpsLargeWaves * (ll[j] + kWave * (rr[j] < 0 ? 0 : rr[j]))) * kWave + lane;
-        v[j] = rr[j] >= 0 && q < n;
-        p[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-        mo[j] = 0.f;
-        if (rr[j] >= 0) {  // wave-uniform: no load left in flight for an unused slot
-          p[j] = Q[v[j] ? q : 0];
-          mo[j] = M[v[j] ? q : 0];
+        for (int r = 0; r < S; ++r) {
+          touched[r] = 0u;
+          uint32_t m = static_cast<uint32_t>(act >> (16 * r)) & 0xffffu;
+          if (!m) continue;
+          const int bk = kWave * (w + W * r) + lane;
+          const uint32_t mx = bk < nb ? static_cast<uint32_t>(__double2hiint(rkey[bk])) : 0u;
+          const uint32_t top = wave_max_u32(mx);
+          if (row == r) smax = top;
+          do {
+            const int l = __builtin_ctz(m);
+            m &= m - 1;
+            const float cx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.x), l));
+            const float cy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.y), l));
+            const float cz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.z), l));
+            float hx, hy, hz;
+            {
+#pragma clang fp contract(off)
+              hx = fmaxf(fmaxf(blx[r] - cx, cx - bhx[r]), 0.f);
+              hy = fmaxf(fmaxf(bly[r] - cy, cy - bhy[r]), 0.f);
+              hz = fmaxf(fmaxf(blz[r] - cz, cz - bhz[r]), 0.f);
+            }
+            const float lb = sqdist(hx, hy, hz, 0.f, 0.f, 0.f);
+            touched[r] |= __float_as_uint(lb) < mx ? 1u << l : 0u;
+          } while (m);
+          total += __builtin_popcountll(__ballot(touched[r] != 0u));
         }
-      }
+        if (total) {
+          int base = 0;
+          if (lane == 0) base = atomicAdd(&n_queue, total);
+          base = __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
-      for (int j = 0; j < G; ++j) {
-        if (rr[j] < 0) continue;  // wave-uniform
-        const int q = (w + kFpsLargeWaves * (ll[j] + kWave * rr[j])) * kWave + lane;
-        const float d = sqdist(p[j].x, p[j].y, p[j].z, cx, cy, cz);
-        const float m = __builtin_amdgcn_fmed3f(d, mo[j], -__builtin_inff());
-        const bool fell = v[j] && m < mo[j];
-        if (fell) M[q] = m;
-        // Values only fall, so while the point holding the bucket's maximum keeps its value the
-        // record (max, lowest index attaining it) stands: no other point can reach the max, and
-        // points tied with it have higher indices.  Most touched buckets end here.
-        const uint32_t al = static_cast<uint32_t>(__builtin_amdgcn_readlane(
-            static_cast<int>(rr[j] == 0 ? blane[0] : (rr[j] == 1 ? blane[1] : blane[2])), ll[j]));
-        if (al < static_cast<uint32_t>(kWave) && !((__ballot(fell) >> al) & 1ull)) continue;
-        const uint32_t bits = v[j] ? __float_as_uint(m) : 0u;
-        const uint32_t bm = wave_max_u32(bits);
-        const uint32_t li = __float_as_uint(p[j].w) - ustart;
-        const uint64_t at = __ballot(v[j] && bits == bm);
-        uint32_t ii;
-        int sl;
-        if (__builtin_popcountll(at) == 1) {  // wave-uniform; the usual case: one lane attains it
-          sl = __builtin_ctzll(at);
-          ii = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(li), sl));
-        } else {  // ties: the lowest index among them
-          ii = wave_min_u32(v[j] && bits == bm ? li : 0xffffffffu);
-          sl = __builtin_ctzll(__ballot(v[j] && bits == bm && li == ii) | (1ull << 63));
-        }
-        const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[j].x), sl));
-        const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[j].y), sl));
-        const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p[j].z), sl));
-        if (lane == ll[j]) {
-          if (rr[j] == 0) {
-            bmax[0] = bm; bidx[0] = ii; blane[0] = sl; bcx[0] = x; bcy[0] = y; bcz[0] = z;
-          } else if (rr[j] == 1) {
-            bmax[1] = bm; bidx[1] = ii; blane[1] = sl; bcx[1] = x; bcy[1] = y; bcz[1] = z;
-          } else {
-            bmax[2] = bm; bidx[2] = ii; blane[2] = sl; bcx[2] = x; bcy[2] = y; bcz[2] = z;
+          for (int r = 0; r < S; ++r) {
+            const uint64_t on = __ballot(touched[r] != 0u);
+            if (touched[r])
+              queue[base + __builtin_popcountll(on & lanemask_lt())] =
+                  static_cast<uint32_t>(kWave * (w + W * r) + lane) << 16 | touched[r];
+            base += __builtin_popcountll(on);
           }
         }
-        // a record's key (max, then lower index) never rises, so only a change of the bucket the
-        // wave's best came from can change the wave's best
-        if (rr[j] == best_r && ll[j] == best_l) dirty = true;
       }
     }
-    if (dirty) {  // the wave's best record: largest max, then lowest index
-      uint32_t m3 = 0u;
+    lds_barrier();
+
+    // update: the queued buckets in turn by all waves, kFpsLargeBatch of a wave's loaded at a time
+    const int total = __builtin_amdgcn_readfirstlane(n_queue);
+    for (int first = w; first < total; first += W * kFpsLargeBatch) {
+      uint32_t item[kFpsLargeBatch], mo[kFpsLargeBatch];
+      float4 p[kFpsLargeBatch];
+      // this wave's share of the queue, one item per lane (past the end: the last one again)
+      const uint32_t mine = queue[min(first + W * lane, total - 1)];
 #pragma unroll
-      for (int r = 0; r < S; ++r) m3 = max(m3, bmax[r]);
-      const uint32_t wh = wave_max_u32(m3);
-      uint64_t e[S];
-      int cnt = 0;
-#pragma unroll
-      for (int r = 0; r < S; ++r) {
-        e[r] = __ballot(bmax[r] == wh && bidx[r] != 0xffffffffu);
-        cnt += __builtin_popcountll(e[r]);
+      for (int u = 0; u < kFpsLargeBatch; ++u) {
+        item[u] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), u));
+        const int q = min(static_cast<int>(item[u] >> 16) * kWave + lane, n - 1);
+        p[u] = Q[q];
+        mo[u] = M[q];
       }
-      if (cnt != 1) {  // wave-uniform: ties (or no bucket at all): the lowest index among them
-        uint32_t li = 0xffffffffu;
 #pragma unroll
-        for (int r = 0; r < S; ++r) li = bmax[r] == wh ? min(li, bidx[r]) : li;
-        const uint32_t mi = wave_min_u32(li);
-#pragma unroll
-        for (int r = 0; r < S; ++r) e[r] = __ballot(bmax[r] == wh && bidx[r] == mi && mi != 0xffffffffu);
-      }
-      const int rs = e[0] ? 0 : (e[1] ? 1 : (e[2] ? 2 : -1));
-      best_r = rs;
-      if (rs < 0) {  // a wave without buckets never wins
-        best_key = 0ull;
-      } else {
-        const int ls = __builtin_ctzll(rs == 0 ? e[0] : (rs == 1 ? e[1] : e[2]));
-        best_l = ls;
-        uint32_t bi;
-        float ex, ey, ez;
-        if (rs == 0) {
-          bi = bidx[0]; ex = bcx[0]; ey = bcy[0]; ez = bcz[0];
-        } else if (rs == 1) {
-          bi = bidx[1]; ex = bcx[1]; ey = bcy[1]; ez = bcz[1];
+      for (int u = 0; u < kFpsLargeBatch; ++u) {
+        if (first + W * u >= total) break;
+        const float4 pt = p[u];
+        const int bk = static_cast<int>(item[u] >> 16);
+        const int q = bk * kWave + lane;
+        const uint32_t old = q < n ? mo[u] : 0u;  // past the end: never changes, never wins
+        const uint32_t holder = static_cast<uint32_t>(__double2loint(rkey[bk]));
+        uint32_t m = item[u] & 0xffffu;
+        uint32_t mb = old;
+        do {
+          const int l = __builtin_ctz(m);
+          m &= m - 1;
+          const float cx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.x), l));
+          const float cy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.y), l));
+          const float cz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.z), l));
+          mb = min(mb, __float_as_uint(sqdist(pt.x, pt.y, pt.z, cx, cy, cz)));
+        } while (m);
+        if (q < n) M[q] = mb;
+        // Values only fall: while the point holding the bucket's max keeps its value, the record
+        // (max, lowest index attaining it) stands, and its rest bound still holds.
+        const uint32_t nidx = ~(__float_as_uint(pt.w) - ustart);
+        if (done != 1 && (__ballot(mb < old) & __ballot(nidx == holder)) == 0ull) continue;
+        const uint32_t mx = wave_max_u32(mb);
+        const uint64_t hit = __ballot(mb == mx && q < n);
+        int sl;
+        uint32_t ni;
+        if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
+          sl = __builtin_ctzll(hit | (1ull << 63));
+          ni = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(nidx), sl));
         } else {
-          bi = bidx[2]; ex = bcx[2]; ey = bcy[2]; ez = bcz[2];
+          ni = wave_max_u32(mb == mx && q < n ? nidx : 0u);
+          sl = __builtin_ctzll(__ballot(mb == mx && q < n && nidx == ni) | (1ull << 63));
         }
-        bi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(bi), ls));
-        best_key = (static_cast<unsigned long long>(wh) << 32) |
-                   (((kFpsLargeIdxMask - bi) << 4) | static_cast<uint32_t>(w));
-        best_c = make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(ex), ls)),
-                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ey), ls)),
-                             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ez), ls)), 0.f);
+        const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.x), sl));
+        const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.y), sl));
+        const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.z), sl));
+        const uint32_t rest =
+            wave_max_u32(min(mb, __float_as_uint(sqdist(pt.x, pt.y, pt.z, x, y, z))));
+        if (lane == 0) {
+          rec[bk] = make_float4(x, y, z, __uint_as_float(rest));
+          rkey[bk] = fps_key(mx, ~ni);
+          dirty[atomicAdd(&n_dirty, 1)] = static_cast<uint16_t>(bk % G);
+        }
       }
-      dirty = false;
     }
-    const int ps = it % 3;
-    if (lane == 0) {
-      cand[it & 1][w] = best_c;
-      atomicMax(&slots[ps], best_key);
+    __syncthreads();  // min distances too: the next round's waves take other buckets
+
+    // groups: best and second record of every group with a changed record, one 16-lane row each
+    {
+      const int changed = __builtin_amdgcn_readfirstlane(n_dirty);
+      if (t == 0) n_queue = 0;
+      for (int at = 4 * w; at < changed; at += 4 * W) {
+        const int g = dirty[min(at + row, changed - 1)];
+        const int m0 = g + G * li, m1 = m0 + 16 * G;
+        double best = m0 < nb ? rkey[m0] : 0.0, other = 0.0;
+        int bk = m0;
+        if (S > 2) {  // more than 16 buckets per group
+          other = m1 < nb ? rkey[m1] : 0.0;
+          if (other > best) {
+            const double x = best;
+            best = other;
+            other = x;
+            bk = m1;
+          }
+        }
+        const uint32_t hi = static_cast<uint32_t>(__double2hiint(best));
+        const uint32_t top = row_max_u32(hi);
+        const uint32_t lo = hi == top ? static_cast<uint32_t>(__double2loint(best)) : 0u;
+        const uint32_t low = row_max_u32(lo);
+        const bool winner = hi == top && lo == low;  // one lane, or lanes without a record
+        const uint32_t sec = row_max_u32(winner ? static_cast<uint32_t>(__double2hiint(other)) : hi);
+        if (winner) {
+          gkey[g] = best;
+          gbkt[g] = bk;
+          gsec[g] = sec;
+        }
+      }
     }
-    if (t == 0) slots[ps == 2 ? 0 : ps + 1] = 0ull;
-    lds_barrier();  // each bucket's points are read and written by its own wave only
-    const unsigned long long key = slots[ps];
-    const uint32_t low = static_cast<uint32_t>(key);
-    const float4 c = cand[it & 1][low & 15u];
-    cx = c.x; cy = c.y; cz = c.z;
-    if (t == 0) out_idx[o0 + it] = start + (kFpsLargeIdxMask - ((low >> 4) & kFpsLargeIdxMask));
+    lds_barrier();
+
+    // rank: no record that is not a group's best exceeds t0; the bests above it, each placed among
+    // all of them, are the list
+    {
+      const double ka = gkey[lane], kb = gkey[kWave + lane];
+      const uint32_t t0 = wave_max_u32(max(gsec[lane], gsec[kWave + lane]));
+      if (t == 0) n_dirty = 0;
+      uint64_t ca = __ballot(static_cast<uint32_t>(__double2hiint(ka)) > t0);
+      uint64_t cb = __ballot(static_cast<uint32_t>(__double2hiint(kb)) > t0);
+      if (!(ca | cb)) {  // ties across groups: the very best record alone
+        const double m = fmax(ka, kb);
+        const uint32_t hi = wave_max_u32(static_cast<uint32_t>(__double2hiint(m)));
+        const uint32_t lo = wave_max_u32(
+            static_cast<uint32_t>(__double2hiint(m)) == hi ? static_cast<uint32_t>(__double2loint(m)) : 0u);
+        const double top = __hiloint2double(static_cast<int>(hi), static_cast<int>(lo));
+        ca = __ballot(ka == top);
+        cb = __ballot(kb == top);
+      }
+      const int na = __builtin_popcountll(ca), nc = na + __builtin_popcountll(cb);
+      const uint64_t lt = lanemask_lt();
+      const int pa = __builtin_popcountll(ca & lt), pb = na + __builtin_popcountll(cb & lt);
+      for (int at = w; at < nc; at += W) {
+        const uint64_t mine = at < na ? ca & __ballot(pa == at) : cb & __ballot(pb == at);
+        const int l = __builtin_ctzll(mine | (1ull << 63));
+        const uint64_t kj = readlane_u64(__double_as_longlong(at < na ? ka : kb), l);
+        const double dj = __longlong_as_double(static_cast<long long>(kj));
+        const int rank = __builtin_popcountll(__ballot(ka > dj)) + __builtin_popcountll(__ballot(kb > dj));
+        if (rank < kFpsRound && lane == 0) {
+          list[rank] = rec[gbkt[l + (at < na ? 0 : kWave)]];
+          lkey[rank] = make_uint2(static_cast<uint32_t>(kj >> 32), ~static_cast<uint32_t>(kj));
+        }
+      }
+      cap = min(max(nc, 1), kFpsRound);
+    }
+    lds_barrier();
   }
 }
 
 struct FpsLargeWs {
   float4* q;
-  float* md;
-  float* bbox;
+  uint32_t* md;
+  float *bbox, *boxes;
   uint32_t *keys, *skeys, *order;
   RadixBuffers rx;
 };
@@ -953,12 +1063,15 @@ int fps_large_key_bits(int64_t B, int* axis_bits) {
   return cbits + 3 * mbits;
 }
 
+int64_t fps_large_box_stride(int64_t B, int64_t N) { return N / kWave + B + 1; }
+
 FpsLargeWs carve_fps_large(void* base, int64_t B, int64_t N, size_t* bytes) {
   Carver c(base);
   FpsLargeWs w;
   w.q = c.take<float4>(N);
-  w.md = c.take<float>(N);
+  w.md = c.take<uint32_t>(N);
   w.bbox = c.take<float>(6 * (B > 0 ? B : 1));
+  w.boxes = c.take<float>(6 * fps_large_box_stride(B, N));
   w.keys = c.take<uint32_t>(N);
   w.skeys = c.take<uint32_t>(N);
   w.order = c.take<uint32_t>(N);
@@ -968,11 +1081,24 @@ FpsLargeWs carve_fps_large(void* base, int64_t B, int64_t N, size_t* bytes) {
 }
 
 bool fps_use_large(int64_t B, int64_t max_cloud) {
-  return max_cloud > 64 * kFpsThreads && max_cloud <= kFpsLargeMaxPoints && B <= kFpsLargeMaxClouds;
+  return max_cloud > kFpsLdsPoints && max_cloud <= kFpsLargeMaxPoints && B <= kFpsLargeMaxClouds;
+}
+
+template <int S>
+int launch_large_rounds(const float* pos, const FpsLargeWs& w, int64_t stride, int nb,
+                        const int64_t* ptr, const int64_t* out_ptr, int64_t B, int64_t* out,
+                        hipStream_t st) {
+  GEO_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&fps_large_kernel<S>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(fps_large_lds(S * kFpsLargeThreads))));
+  hipLaunchKernelGGL((fps_large_kernel<S>), dim3(B), dim3(kFpsLargeThreads), fps_large_lds(nb), st,
+                     pos, w.q, w.md, w.boxes, stride, nb, ptr, out_ptr, out);
+  GEO_LAUNCH_CHECK("fps_large_kernel");
+  return GEO_OK;
 }
 
 int launch_large(const float* pos, int64_t N, const int64_t* ptr, const int64_t* out_ptr,
-                 int64_t B, int64_t* out, void* workspace, hipStream_t st) {
+                 int64_t B, int64_t max_cloud, int64_t* out, void* workspace, hipStream_t st) {
   size_t bytes = 0;
   const FpsLargeWs w = carve_fps_large(workspace, B, N, &bytes);
   hipLaunchKernelGGL(fps_large_bbox_kernel, dim3(B), dim3(kFpsLargeThreads), 0, st, pos, ptr, w.bbox);
@@ -985,30 +1111,16 @@ int launch_large(const float* pos, int64_t N, const int64_t* ptr, const int64_t*
   GEO_LAUNCH_CHECK("fps_large_keys_kernel");
   int rc = radix_sort<kRxKeysIota>(w.keys, nullptr, N, 0, w.skeys, w.order, w.rx, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(fps_large_gather_kernel, dim3(grid), dim3(256), 0, st, pos, w.order, N, w.q, w.md);
+  const int64_t nb = ceil_div(max_cloud, kWave);
+  const int64_t stride = fps_large_box_stride(B, N);
+  hipLaunchKernelGGL(fps_large_gather_kernel, dim3(static_cast<unsigned>(ceil_div(nb, 4)), B), dim3(256),
+                     0, st, pos, w.order, ptr, stride, w.q, w.md, w.boxes);
   GEO_LAUNCH_CHECK("fps_large_gather_kernel");
-  hipLaunchKernelGGL(fps_large_kernel, dim3(B), dim3(kFpsLargeThreads), 0, st, pos, w.q, w.md, ptr,
-                     out_ptr, out);
-  GEO_LAUNCH_CHECK("fps_large_kernel");
-  return GEO_OK;
-}
-
-template <int PTS>
-int launch_register(const float* pos, const int64_t* ptr, const int64_t* out_ptr, int64_t B,
-                    int64_t max_cloud, int64_t* out, hipStream_t st) {
-  if (max_cloud <= kFpsLdsPoints) {
-    const size_t lds = static_cast<size_t>(max_cloud > 0 ? max_cloud : 1) * sizeof(float4);
-    GEO_HIP_CHECK(hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&fps_register_kernel<PTS, true>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFpsLdsPoints * sizeof(float4))));
-    hipLaunchKernelGGL((fps_register_kernel<PTS, true>), dim3(B), dim3(kFpsThreads), lds, st,
-                       pos, ptr, out_ptr, out);
-  } else {
-    hipLaunchKernelGGL((fps_register_kernel<PTS, false>), dim3(B), dim3(kFpsThreads), 0, st, pos,
-                       ptr, out_ptr, out);
-  }
-  GEO_LAUNCH_CHECK("fps_register_kernel");
-  return GEO_OK;
+  if (nb <= kFpsLargeThreads)
+    return launch_large_rounds<1>(pos, w, stride, static_cast<int>(nb), ptr, out_ptr, B, out, st);
+  if (nb <= 2 * kFpsLargeThreads)
+    return launch_large_rounds<2>(pos, w, stride, static_cast<int>(nb), ptr, out_ptr, B, out, st);
+  return launch_large_rounds<3>(pos, w, stride, static_cast<int>(nb), ptr, out_ptr, B, out, st);
 }
 
 }  // namespace
@@ -1075,13 +1187,21 @@ extern "C" size_t geo_fps_workspace_bytes(int64_t B, int64_t N_total, int64_t ma
     carve_fps_large(nullptr, B, N_total, &bytes);
     return bytes;
   }
-  if (max_cloud > 64 * kFpsThreads) return static_cast<size_t>(N_total > 0 ? N_total : 1) * 4;
+  if (max_cloud > kFpsRegisterPoints) return static_cast<size_t>(N_total > 0 ? N_total : 1) * 4;
   return 0;
 }
 
 extern "C" int geo_fps(const float* pos, int64_t N_total, const int64_t* ptr,
                        const int64_t* out_ptr, int64_t B, int64_t max_cloud, int64_t* out_idx,
                        void* workspace, size_t workspace_bytes, void* stream) {
+  return geo_fps_total(pos, N_total, ptr, out_ptr, B, max_cloud, N_total, out_idx, workspace,
+                       workspace_bytes, stream);
+}
+
+extern "C" int geo_fps_total(const float* pos, int64_t N_total, const int64_t* ptr,
+                             const int64_t* out_ptr, int64_t B, int64_t max_cloud, int64_t total,
+                             int64_t* out_idx, void* workspace, size_t workspace_bytes,
+                             void* stream) {
   GEO_REQUIRE(B >= 0 && N_total >= 0 && max_cloud >= 0, "fps: negative size");
   GEO_REQUIRE(max_cloud <= N_total, "fps: max_cloud %lld > N_total %lld", (long long)max_cloud,
               (long long)N_total);
@@ -1093,25 +1213,26 @@ extern "C" int geo_fps(const float* pos, int64_t N_total, const int64_t* ptr,
   if (need > 0 && (workspace == nullptr || workspace_bytes < static_cast<size_t>(need)))
     return set_error(GEO_ERR_WORKSPACE, "fps: workspace %zu bytes, need %lld", workspace_bytes,
                      (long long)need);
-  const int64_t per = ceil_div(max_cloud, kFpsThreads);
   if (max_cloud <= kFpsLdsPoints) {
     // 1024 threads: four waves per SIMD hide much of the per-iteration dependency chain.
     const int64_t p2 = ceil_div(max_cloud, kFpsBucketThreads);
     if (p2 <= 1) return launch_bucket<1, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
     if (p2 <= 2) return launch_bucket<2, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
     if (p2 <= 4) return launch_bucket<4, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-    if (p2 <= 8) return launch_bucket<8, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
     return launch_bucket<8, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
   }
-  if (per <= 1) return launch_register<1>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 2) return launch_register<2>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 4) return launch_register<4>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 8) return launch_register<8>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 16) return launch_register<16>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 32) return launch_register<32>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
-  if (per <= 64) return launch_register<64>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
+  // Up to 16,384 points and few samples per cloud: the register kernel, which has no set-up.  The
+  // large kernel's sort and first rounds cost about 90 us more, its later rounds a tenth as much
+  // per sample (12,000 points: 64 samples 197 against 225 us, 375 samples 1069 against 399 us,
+  // 6000 samples 16.9 against 2.2 ms); they cross at 73 to 87 samples between 8,200 and 16,384.
+  if (max_cloud <= kFpsRegisterPoints && (total <= kFpsRegisterSamples * B || !fps_use_large(B, max_cloud))) {
+    hipLaunchKernelGGL((fps_register_kernel<kFpsRegisterPoints / kFpsThreads>), dim3(B),
+                       dim3(kFpsThreads), 0, st, pos, ptr, out_ptr, out_idx);
+    GEO_LAUNCH_CHECK("fps_register_kernel");
+    return GEO_OK;
+  }
   if (fps_use_large(B, max_cloud))
-    return launch_large(pos, N_total, ptr, out_ptr, B, out_idx, workspace, st);
+    return launch_large(pos, N_total, ptr, out_ptr, B, max_cloud, out_idx, workspace, st);
   hipLaunchKernelGGL(fps_stream_kernel, dim3(B), dim3(kFpsStreamThreads), 0, st, pos, ptr,
                      out_ptr, out_idx, static_cast<float*>(workspace));
   GEO_LAUNCH_CHECK("fps_stream_kernel");

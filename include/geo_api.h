@@ -95,6 +95,11 @@ size_t geo_fps_workspace_bytes(int64_t B, int64_t N_total, int64_t max_cloud);
 int geo_fps(const float* pos, int64_t N_total, const int64_t* ptr, const int64_t* out_ptr,
             int64_t B, int64_t max_cloud, int64_t* out_idx, void* workspace,
             size_t workspace_bytes, void* stream);
+/* geo_fps told the batch's number of samples (info[0]): clouds of 8193 to 16,384 points with few
+ * samples each then take a kernel without set-up.  geo_fps alone assumes many. */
+int geo_fps_total(const float* pos, int64_t N_total, const int64_t* ptr, const int64_t* out_ptr,
+                  int64_t B, int64_t max_cloud, int64_t total, int64_t* out_idx, void* workspace,
+                  size_t workspace_bytes, void* stream);
 
 /* -------------------------------------------------------------------- KNN --- */
 /*

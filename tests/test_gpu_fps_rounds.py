@@ -33,3 +33,20 @@ def test_fps_rounds_follow_the_greedy_order(kind, sizes):
     k = np.array([max(1, (3 * n) // 5) for n in sizes])
     got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
+
+
+@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "line", "same"])
+@pytest.mark.parametrize("sizes, samples", [
+    ([8193, 3], 90),            # smallest cloud of the large kernel, above the few-samples rule
+    ([16384, 40], 60),          # few samples per cloud: register kernel
+    ([16385, 8000, 9000], 700),  # a batch off the 64-point grid
+    ([65536], 1200), ([65537], 900),      # one / two boxes per lane
+    ([131073], 900), ([196608], 700),     # three, and the largest cloud
+])
+def test_fps_rounds_of_large_clouds(kind, sizes, samples):
+    from gdl_amd.csrc import fps_cuda
+    pos = _points(kind, sum(sizes), len(sizes))
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    k = np.array([min(n, samples if kind != "same" else 40) for n in sizes])
+    got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
+    np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
