@@ -150,15 +150,16 @@ __device__ __forceinline__ EdgeScalars edge_from(const EdgeScalars& st, int j) {
 // Per-edge coefficients with the edge's scalars folded in, computed once by the lane that stages
 // the edge (instead of by every channel lane):
 //   c0 = r0 y0, c1 = r1 d, c2 = r2 y0, c3 = r3 d, c4 = r4 d, c5 = r5 y2, c6 = r6 y0, c8 = r8,
-//   d7[j][m] = r7 sum_i d_i cg[i][j][m]
+//   c7 = r7 d, d7[j][m] = r7 sum_i d_i cg[i][j][m]
 // (r_p = 0 for paths that are off).  The forward accumulates c0 s, c1 s, c2 v, c3 . v, c4 x v,
-// c5 s, c6 t, c8 |t|^2 and sum_j d7[j] v_j; the source-side backward the transposed products.
+// c5 s, c6 t, c8 |t|^2 and c7_i v_j, to whose sums it applies the CG table once per node; the
+// source-side backward accumulates the transposed products (path 7 through d7).
 template <bool T2>
 struct EdgeCoef {
   int32_t other;
   int32_t ok;
   float c0, c1[3], c2, c3[3], c4[3];
-  float c5[5], c6, c8, d7[3][5];
+  float c5[5], c6, c7[3], c8, d7[3][5];
 };
 
 __device__ __forceinline__ void cg_coef(const float* cg, const float d[3], float r, float D[3][5]);
@@ -189,6 +190,8 @@ __device__ __forceinline__ EdgeCoef<T2> coef_of(const SeEdges& g, const EdgeScal
     for (int m = 0; m < 5; ++m) c.c5[m] = q.r[5] * q.y2[m];
     c.c6 = q.r[6] * q.y0;
     c.c8 = q.r[8];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) c.c7[k] = q.r[7] * q.d[k];
     cg_coef(g.cg, q.d, q.r[7], c.d7);
   }
   return c;
@@ -214,6 +217,8 @@ __device__ __forceinline__ EdgeCoef<T2> coef_at(const EdgeCoef<T2>& st, int j) {
     c.c6 = rlane(st.c6, j);
     c.c8 = rlane(st.c8, j);
 #pragma unroll
+    for (int k = 0; k < 3; ++k) c.c7[k] = rlane(st.c7[k], j);
+#pragma unroll
     for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
       for (int m = 0; m < 5; ++m) c.d7[jj][m] = rlane(st.d7[jj][m], j);
@@ -221,8 +226,8 @@ __device__ __forceinline__ EdgeCoef<T2> coef_at(const EdgeCoef<T2>& st, int j) {
   return c;
 }
 
-// D[j][m] = r * sum_i d_i cg[i][j][m]: path 7's per-edge coefficients, so that a lane's share
-// is sum_j v_j D[j][m] (forward) or sum_m D[j][m] w_m (source-side backward).
+// D[j][m] = r * sum_i d_i cg[i][j][m]: path 7's per-edge coefficients of the source-side backward,
+// where a lane's share is sum_m D[j][m] w_m.
 // The table is read from device memory at a wave-uniform address (scalar loads, cached); a NULL
 // table (path 7 off) gives zeros.
 __device__ __forceinline__ void cg_coef(const float* cg, const float d[3], float r, float D[3][5]) {
@@ -238,6 +243,20 @@ __device__ __forceinline__ void cg_coef(const float* cg, const float d[3], float
 #pragma unroll
     for (int m = 0; m < 5; ++m)
       D[j][m] = r * ((d[0] * cg[j * 5 + m] + d[1] * cg[(3 + j) * 5 + m]) + d[2] * cg[(6 + j) * 5 + m]);
+}
+
+// Component m of path 7 from its sums b(i, j) = sum of r7 d_i v_j over a node's edges: the table
+// applied once per node (9 products per edge and channel instead of 15, and 3 coefficients per
+// edge instead of 15).
+template <class B>
+__device__ __forceinline__ float cg_apply(const float* cg, int m, const B& b) {
+  if (cg == nullptr) return 0.f;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s += cg[(3 * i + j) * 5 + m] * b(i, j);
+  return s;
 }
 
 __device__ __forceinline__ void zero_pad(float* row, int used, int K) {
@@ -263,13 +282,15 @@ constexpr int kSeUnroll = 2;  // edges whose source rows are in flight together 
 template <bool T2>
 struct NodeAcc {
   float A0, A1[3], A2[3], A3, A4[3];
-  float A5[5], A6[5], A7[5], A8;
+  float A5[5], A6[5], B[3][3], A8;  // B: path 7 before the CG table (cg_apply)
   __device__ __forceinline__ void zero() {
     A0 = A3 = A8 = 0.f;
 #pragma unroll
     for (int k = 0; k < 3; ++k) A1[k] = A2[k] = A4[k] = 0.f;
 #pragma unroll
-    for (int k = 0; k < 5; ++k) A5[k] = A6[k] = A7[k] = 0.f;
+    for (int k = 0; k < 5; ++k) A5[k] = A6[k] = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) B[k][0] = B[k][1] = B[k][2] = 0.f;
   }
 };
 
@@ -304,8 +325,9 @@ __device__ __forceinline__ void accumulate_edge(NodeAcc<T2>& A, const SeEdges& g
     }
     if (T2 && g.pc[7] >= 0 && t_out) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k)
-        A.A7[k] += (q.d7[0][k] * v[0] + q.d7[1][k] * v[1]) + q.d7[2][k] * v[2];
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) A.B[i][k] += q.c7[i] * v[k];
     }
   }
   if (ht) {
@@ -365,9 +387,9 @@ __device__ __forceinline__ void load_source(const SeFeat& f, int m, const LaneCh
 // xs [Ks] = A0 | A3 | A8, xv row k (k < 3, rows sv apart) = A1_k | A2_k | A4_k, xt row m
 // (m < 5, rows st apart) = A5_m | A6_m | A7_m.  A NULL row pointer skips that kind.
 template <bool T2>
-__device__ __forceinline__ void store_node(const NodeAcc<T2>& A, const SeFeat& f, int c, bool hs,
-                                           bool hv, bool ht, float* xs, float* xv, int sv,
-                                           float* xt, int st) {
+__device__ __forceinline__ void store_node(const NodeAcc<T2>& A, const SeFeat& f, const float* cg,
+                                           int c, bool hs, bool hv, bool ht, float* xs, float* xv,
+                                           int sv, float* xt, int st) {
   if (xs) {
     if (hs) xs[c] = A.A0;
     if (hv) xs[f.Cs + c] = A.A3;
@@ -388,7 +410,7 @@ __device__ __forceinline__ void store_node(const NodeAcc<T2>& A, const SeFeat& f
       float* row = xt + k * st;
       if (hs) row[c] = A.A5[k];
       if (ht) row[f.Cs + c] = A.A6[k];
-      if (hv) row[f.Cs + f.Ct + c] = A.A7[k];
+      if (hv) row[f.Cs + f.Ct + c] = cg_apply(cg, k, [&](int i, int j) { return A.B[i][j]; });
     }
   }
 }
@@ -434,7 +456,7 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_aggregate(SeEdges g, SeFea
         }
       }
     }
-    store_node<T2>(A, f, c, hs, hv, ht, Xs ? Xs + n * Ks : nullptr, Xv ? Xv + n * 3 * Kv : nullptr,
+    store_node<T2>(A, f, g.cg, c, hs, hv, ht, Xs ? Xs + n * Ks : nullptr, Xv ? Xv + n * 3 * Kv : nullptr,
                    Kv, (T2 && Xt) ? Xt + n * 5 * Kt : nullptr, Kt);
   }
   if (Xs) zero_pad(Xs + n * Ks, f.Cs + f.Cv + f.Ct, Ks);
@@ -741,7 +763,7 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused(SeEdges g, SeFeat f,
     int cur = 0, cur_end = e1;  // node being summed and its flat end
     auto flush = [&](int i) {
       const int nt = wave * kFuNodes + i;
-      store_node<T2>(A, f, c, hs, hv, ht, ts ? ts + nt * p.ld[0] : nullptr,
+      store_node<T2>(A, f, g.cg, c, hs, hv, ht, ts ? ts + nt * p.ld[0] : nullptr,
                      tv ? tv + nt * 3 * p.ld[1] : nullptr, p.ld[1],
                      tt ? tt + nt * 5 * p.ld[2] : nullptr, p.ld[2]);
       A.zero();
@@ -781,15 +803,24 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused(SeEdges g, SeFeat f,
   fused_tile_out<T2>(p, lds, node0, g.N, wave, lane);
 }
 
-// ------------------------------ fused forward, one node per 16-lane row (no type-2 paths) ---
-// Layers without type-2 features or outputs whose Cs <= 64 and Cv <= 16 (Cs a multiple of 4;
-// e.g. 64 scalar + 16 vector channels): a wave sums four nodes at once, one per 16-lane row.
-// Lane j of a row holds scalar channels 4j..4j+3 and vector channel j, so one 16-byte load (s)
-// and one 12-byte load (v) per lane fetch a source row for each of the four nodes -- two
-// vector-memory instructions per four edges where the channel-per-lane walk above issues four
-// per edge.  That walk keeps the texture address unit busy ~70% of its time (counters at C2);
-// this one needs an eighth of its instructions.  A row's edges are staged one per lane, 16 per
-// round, and edge u's source and coefficients reach the row's lanes by DPP row_newbcast:u.
+// ------------------------------------------------ fused forward, one node per 16-lane row ---
+// Layers of up to 128 scalar, 32 vector and 16 type-2 channels: a wave sums four nodes at once, one
+// per 16-lane row.  Lane j of a row holds SC scalar channels (SC j .., and with SC = 8 the four from
+// 4 j and the four from 64 + 4 j), VC vector channels (j, 16 + j) and type-2 channel j, so one
+// 16-byte load (s) and one 12-byte load (v) per lane fetch a 64 + 16 channel source row for each of
+// the four nodes -- two vector-memory instructions per four edges where the channel-per-lane walk
+// above issues four per edge.  That walk keeps the texture address unit busy ~70% of its time
+// (counters at C2), and reads every coefficient of every edge from a lane of its own
+// (v_readlane); this one needs an eighth of its load and a third of its vector instructions.  A
+// row's edges are staged one per lane, 16 per round, and edge u's source and coefficients reach the
+// row's lanes by DPP row_newbcast:u.  Path 7 sums r7 d_i v_j (9 products per channel) over the edges
+// and applies the CG table once per node, instead of 15 coefficients per edge.
+// Kernel times against the channel-per-lane walk at 16 clouds of 4096 points (C2 graph; with type-2
+// channels 8 clouds, 128 + 32 channels 4): scalar + vector (+ type-2) channels 16 + 8 47 -> 38 us
+// (four scalar channels per lane before), 15 + 7 107 -> 39, 64 + 32 142 -> 87, 128 + 32 97 -> 50,
+// 32 + 16 + 8 156 -> 53, 64 + 16 + 8 199 -> 85; 64 + 16 62 -> 60 (no second zeroing of absent edges).
+// Without type-2 channels four source rows are in flight per lane, with them two (32 + 16 + 8:
+// four 63 us, the wave's registers then leave room for fewer waves; one 53 us).
 constexpr int kRowNodes = kFuTile / kSeWaves;  // nodes per wave = 16-lane rows
 constexpr int kRowStage = 16;                  // edges staged per row per round
 constexpr uint32_t kPastRows = 0x80000000u;    // a byte offset past every array (each < 2 GiB)
@@ -814,20 +845,32 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// Per-lane sums of the row's node: scalar channels 4j..4j+3 (A0, A1_k) and vector channel j
-// (A2_k, A3, A4_k).
+// Per-lane sums of the row's node over its edges (names as in the aggregate layout above).
+template <int SC, int VC, bool T2>
 struct RowAcc {
-  float A0[4], A1[3][4];
-  float A2[3], A3, A4[3];
+  float A0[SC], A1[3][SC];
+  float A2[3][VC], A3[VC], A4[3][VC];
+  float A5[T2 ? 5 : 0][SC], A6[T2 ? 5 : 0], A8[T2 ? 1 : 0];
+  float B[T2 ? 3 : 0][3][VC];  // path 7 before the CG table (cg_apply)
 };
 
-// Staging of the row kernel: the lane's edge at CSR position pos (when valid) -- its source, the
-// radial weights of paths 0-4, the direction (one 12-byte load) and Y_0^0 -- as coefficients
-// (coef_of's c0..c4).  The loads go through buffer resources and a lane without an edge reads
-// past the arrays (zeros), so none of them waits on a branch or on the source load; only the
-// permutation, when there is one, comes first.  Every array here is below 2 GiB (the host checks).
-__device__ __forceinline__ EdgeCoef<false> stage_rows(const SeEdges& g, int pos, bool valid) {
+// Per-edge coefficients of the row kernels (EdgeCoef's; path 7 as c7 = r7 d).
+template <bool T2>
+struct RowCoef {
+  int32_t other, ok;
+  float c0, c1[3], c2, c3[3], c4[3];
+  float c5[T2 ? 5 : 0], c6[T2 ? 1 : 0], c7[T2 ? 3 : 0], c8[T2 ? 1 : 0];
+};
+
+// Staging of the row kernels: the lane's edge at CSR position pos (when valid) -- its source, the
+// radial weights, the direction (one 12-byte load), Y_0^0 and Y_2 -- as coefficients.  The loads go
+// through buffer resources and a lane without an edge reads past the arrays (zeros), so none of them
+// waits on a branch or on the source load; only the permutation, when there is one, comes first.
+// Every array here is below 2 GiB (the host checks).
+template <bool T2>
+__device__ __forceinline__ RowCoef<T2> stage_rows(const SeEdges& g, int pos, bool valid) {
   constexpr uint32_t kPast = kPastRows;
+  constexpr int NP = T2 ? kSePaths : 5;
   int e = valid ? pos : -1;
   if (g.perm) {
     const auto rp = row_rsrc(g.perm, g.E * 4);
@@ -840,21 +883,28 @@ __device__ __forceinline__ EdgeCoef<false> stage_rows(const SeEdges& g, int pos,
   const uint32_t lo = w[0], hi = w[1];
   const int64_t o = static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
   const auto rr = row_rsrc(g.R, g.E * g.P * 4);
-  float r[5];
+  float r[NP];
 #pragma unroll
-  for (int i = 0; i < 5; ++i)
+  for (int i = 0; i < NP; ++i)
     r[i] = g.pc[i] >= 0 ? ld_row(rr, ein ? 4u * (ue * g.P + g.pc[i]) : kPast) : 0.f;
   const auto rd = row_rsrc(g.dir, g.E * 12);
   const auto dv = __builtin_amdgcn_raw_buffer_load_b96(rd, ein ? 12u * ue : kPast, 0, 0);
   const float d[3] = {__uint_as_float(dv[0]), __uint_as_float(dv[1]), __uint_as_float(dv[2])};
   const auto ry = row_rsrc(g.Y, g.E * g.ysh * 4);
   const float y0 = ld_row(ry, ein ? 4u * ue * g.ysh : kPast);
+  float y2[T2 ? 5 : 1];
+  if constexpr (T2) {
+    const bool l2 = g.ysh >= 9;  // path 5 is off without
+    const uint32_t at = ein && l2 ? 4u * ue * g.ysh + 16u : kPast;
+#pragma unroll
+    for (int m = 0; m < 5; ++m) y2[m] = ld_row(ry, at + 4u * m);
+  }
   const bool ok = ein && o >= 0 && o < g.N;
-  EdgeCoef<false> c;
+  RowCoef<T2> c;
   c.other = ok ? static_cast<int32_t>(o) : 0;
   c.ok = ok ? 1 : 0;
 #pragma unroll
-  for (int i = 0; i < 5; ++i) r[i] = ok ? r[i] : 0.f;
+  for (int i = 0; i < NP; ++i) r[i] = ok ? r[i] : 0.f;
   c.c0 = r[0] * y0;
   c.c2 = r[2] * y0;
 #pragma unroll
@@ -863,11 +913,22 @@ __device__ __forceinline__ EdgeCoef<false> stage_rows(const SeEdges& g, int pos,
     c.c3[k] = r[3] * d[k];
     c.c4[k] = r[4] * d[k];
   }
+  if constexpr (T2) {
+#pragma unroll
+    for (int m = 0; m < 5; ++m) c.c5[m] = r[5] * y2[m];
+    c.c6[0] = r[6] * y0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) c.c7[k] = r[7] * d[k];
+    c.c8[0] = r[8];
+  }
   return c;
 }
 
-template <int U>
+// U: source rows in flight per lane.
+template <int U, int SC, int VC, bool T2>
 __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused_rows(SeEdges g, SeFeat f, SeFused p) {
+  static_assert(SC == 1 || SC == 2 || SC == 4 || SC == 8, "scalar channels per lane");
+  constexpr int SL = SC < 4 ? SC : 4;  // channels of one load
   extern __shared__ floatx4 fu_lds[];
   float* lds = reinterpret_cast<float*>(fu_lds);
   const int64_t node0 = xcd_block() * kFuTile;  // grid = ceil(N / kFuTile): node0 < N
@@ -882,87 +943,132 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused_rows(SeEdges g, SeFe
   const int deg = b - a;
   const int maxdeg = max(max(__builtin_amdgcn_readlane(deg, 0), __builtin_amdgcn_readlane(deg, 16)),
                          max(__builtin_amdgcn_readlane(deg, 32), __builtin_amdgcn_readlane(deg, 48)));
-  // whole-array resources (the host keeps both arrays below 4 GiB): a lane past the row's
+  // whole-array resources (the host keeps the arrays below 2 GiB): a lane past the row's
   // channels reads the next row (unused) or, past the array, zeros
   const auto rs = row_rsrc(f.s, static_cast<int>(g.N * f.Cs * 4));
   const auto rv = row_rsrc(f.v, static_cast<int>(g.N * f.Cv * 12));
-  const uint32_t rowb_s = 4u * f.Cs, rowb_v = 12u * f.Cv;
-  const uint32_t js = 16u * j, jv = 12u * j;
+  const auto rt = row_rsrc(f.t, static_cast<int>(g.N * f.Ct * 20));
+  const uint32_t rowb_s = 4u * f.Cs, rowb_v = 12u * f.Cv, rowb_t = 20u * f.Ct;
+  const uint32_t js = 4u * SL * j, jv = 12u * j, jt = 20u * j;
 
-  RowAcc A;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    A.A0[i] = 0.f;
-    A.A1[0][i] = A.A1[1][i] = A.A1[2][i] = 0.f;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) A.A2[k] = A.A4[k] = 0.f;
-  A.A3 = 0.f;
+  RowAcc<SC, VC, T2> A = {};
 
   for (int base = 0; base < maxdeg; base += kRowStage) {
-    const EdgeCoef<false> st = stage_rows(g, a + base + j, base + j < deg);
+    const RowCoef<T2> st = stage_rows<T2>(g, a + base + j, base + j < deg);
     const int cnt = min(kRowStage, maxdeg - base);
     static_for<0, kRowStage / U>([&](auto ci) {
       constexpr int c0 = decltype(ci)::value * U;
       if (c0 >= cnt) return;
-      floatx4 sx[U];
-      float vx[U][3];
+      float sx[U][SC], vx[U][VC][3], tx[U][T2 ? 5 : 1];
       static_for<0, U>([&](auto ui) {  // the U source rows of every row in flight together
-        constexpr int u = c0 + decltype(ui)::value;
-        // a row without edge u (its node has fewer edges) reads past the arrays: zeros, no traffic
+        constexpr int uu = decltype(ui)::value;
+        constexpr int u = c0 + uu;
+        // an edge that is not there (past the row's degree, or a source out of range) reads past
+        // the arrays: zeros, no traffic, so nothing of row 0 can leak into its (zero) products
         const bool have = row_bcast<u>(st.ok) != 0;
         const uint32_t m = static_cast<uint32_t>(row_bcast<u>(st.other));
-        const auto ls = __builtin_amdgcn_raw_buffer_load_b128(rs, have ? m * rowb_s + js : kPastRows,
-                                                              0, 0);
-        const auto lv = __builtin_amdgcn_raw_buffer_load_b96(rv, have ? m * rowb_v + jv : kPastRows,
-                                                             0, 0);
-        // element by value: __builtin_bit_cast of a vector element reads the vector's first
+        const uint32_t os = have ? m * rowb_s + js : kPastRows;
+        // elements by value: __builtin_bit_cast of a vector element reads the vector's first
         // element whatever the index
+        if constexpr (SL == 4) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sx[decltype(ui)::value][i] = __uint_as_float(ls[i]);
+          for (int h = 0; h < SC / 4; ++h) {
+            const auto ls = __builtin_amdgcn_raw_buffer_load_b128(rs, os + 256u * h, 0, 0);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) vx[decltype(ui)::value][k] = __uint_as_float(lv[k]);
+            for (int i = 0; i < 4; ++i) sx[uu][4 * h + i] = __uint_as_float(ls[i]);
+          }
+        } else if constexpr (SL == 2) {
+          const auto ls = __builtin_amdgcn_raw_buffer_load_b64(rs, os, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) sx[uu][i] = __uint_as_float(ls[i]);
+        } else {
+          sx[uu][0] = ld_row(rs, os);
+        }
+        const uint32_t ov = have ? m * rowb_v + jv : kPastRows;
+#pragma unroll
+        for (int h = 0; h < VC; ++h) {
+          const auto lv = __builtin_amdgcn_raw_buffer_load_b96(rv, ov + 192u * h, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) vx[uu][h][k] = __uint_as_float(lv[k]);
+        }
+        if constexpr (T2) {
+          const uint32_t ot = have ? m * rowb_t + jt : kPastRows;
+          const auto lt = __builtin_amdgcn_raw_buffer_load_b128(rt, ot, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) tx[uu][k] = __uint_as_float(lt[k]);
+          tx[uu][4] = ld_row(rt, ot + 16u);
+        }
       });
       static_for<0, U>([&](auto ui) {
         constexpr int uu = decltype(ui)::value;
         constexpr int u = c0 + uu;
-        // an edge that is not there (past the row's degree, or a source out of range) adds
-        // nothing: its values are replaced by zeros, so a non-finite row 0 cannot leak in
-        const bool ok = row_bcast<u>(st.ok) != 0;
-        float x[4], v[3];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = ok ? sx[uu][i] : 0.f;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) v[k] = ok ? vx[uu][k] : 0.f;
+        const float* x = sx[uu];
         if (g.pc[0] >= 0) {
           const float c = row_bcast<u>(st.c0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) A.A0[i] += c * x[i];
+          for (int i = 0; i < SC; ++i) A.A0[i] += c * x[i];
         }
         if (g.pc[1] >= 0) {
 #pragma unroll
           for (int k = 0; k < 3; ++k) {
             const float c = row_bcast<u>(st.c1[k]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) A.A1[k][i] += c * x[i];
+            for (int i = 0; i < SC; ++i) A.A1[k][i] += c * x[i];
           }
         }
         if (g.pc[2] >= 0) {
           const float c = row_bcast<u>(st.c2);
 #pragma unroll
-          for (int k = 0; k < 3; ++k) A.A2[k] += c * v[k];
+          for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int h = 0; h < VC; ++h) A.A2[k][h] += c * vx[uu][h][k];
         }
         if (g.pc[3] >= 0) {
           const float d0 = row_bcast<u>(st.c3[0]), d1 = row_bcast<u>(st.c3[1]);
           const float d2 = row_bcast<u>(st.c3[2]);
-          A.A3 += (d0 * v[0] + d1 * v[1]) + d2 * v[2];
+#pragma unroll
+          for (int h = 0; h < VC; ++h)
+            A.A3[h] += (d0 * vx[uu][h][0] + d1 * vx[uu][h][1]) + d2 * vx[uu][h][2];
         }
         if (g.pc[4] >= 0) {
           const float e0 = row_bcast<u>(st.c4[0]), e1 = row_bcast<u>(st.c4[1]);
           const float e2 = row_bcast<u>(st.c4[2]);
-          A.A4[0] += e1 * v[2] - e2 * v[1];
-          A.A4[1] += e2 * v[0] - e0 * v[2];
-          A.A4[2] += e0 * v[1] - e1 * v[0];
+#pragma unroll
+          for (int h = 0; h < VC; ++h) {
+            const float* v = vx[uu][h];
+            A.A4[0][h] += e1 * v[2] - e2 * v[1];
+            A.A4[1][h] += e2 * v[0] - e0 * v[2];
+            A.A4[2][h] += e0 * v[1] - e1 * v[0];
+          }
+        }
+        if constexpr (T2) {
+          if (g.pc[5] >= 0) {
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+              const float c = row_bcast<u>(st.c5[m]);
+#pragma unroll
+              for (int i = 0; i < SC; ++i) A.A5[m][i] += c * x[i];
+            }
+          }
+          const float* t = tx[uu];
+          if (g.pc[6] >= 0) {
+            const float c = row_bcast<u>(st.c6[0]);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) A.A6[m] += c * t[m];
+          }
+          if (g.pc[7] >= 0) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              const float c = row_bcast<u>(st.c7[i]);
+#pragma unroll
+              for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int h = 0; h < VC; ++h) A.B[i][k][h] += c * vx[uu][h][k];
+            }
+          }
+          if (g.pc[8] >= 0)
+            A.A8[0] += row_bcast<u>(st.c8[0]) *
+                       ((((t[0] * t[0] + t[1] * t[1]) + t[2] * t[2]) + t[3] * t[3]) + t[4] * t[4]);
         }
       });
     });
@@ -971,33 +1077,88 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused_rows(SeEdges g, SeFe
   // the node's aggregate rows into the tile (layout as se3_fwd_aggregate's rows)
   float* ts = p.O[0] > 0 ? lds + p.off[0] + nt * p.ld[0] : nullptr;
   float* tv = p.O[1] > 0 ? lds + p.off[1] + nt * 3 * p.ld[1] : nullptr;
-  if (4 * j < f.Cs) {
-    if (ts) *reinterpret_cast<floatx4*>(ts + 4 * j) = floatx4{A.A0[0], A.A0[1], A.A0[2], A.A0[3]};
-    if (tv)
+  float* tt = T2 && p.O[2] > 0 ? lds + p.off[2] + nt * 5 * p.ld[2] : nullptr;
+  const auto put = [&](float* row, const float* v) {  // the lane's scalar channels of one row
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        *reinterpret_cast<floatx4*>(tv + k * p.ld[1] + 4 * j) =
-            floatx4{A.A1[k][0], A.A1[k][1], A.A1[k][2], A.A1[k][3]};
-  }
-  if (j < f.Cv) {
-    if (ts) ts[f.Cs + j] = A.A3;
+    for (int h = 0; h < SC / SL; ++h) {
+      const int c = 64 * h + SL * j;
+      if (c >= f.Cs) continue;
+      if constexpr (SL == 4) {
+        *reinterpret_cast<floatx4*>(row + c) = floatx4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < SL; ++i) row[c + i] = v[i];
+      }
+    }
+  };
+  if (ts) put(ts, A.A0);
+  if (tv)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) put(tv + k * p.ld[1], A.A1[k]);
+#pragma unroll
+  for (int h = 0; h < VC; ++h) {
+    const int c = 16 * h + j;
+    if (c >= f.Cv) continue;
+    if (ts) ts[f.Cs + c] = A.A3[h];
     if (tv)
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        tv[k * p.ld[1] + f.Cs + j] = A.A2[k];
-        tv[k * p.ld[1] + f.Cs + f.Cv + j] = A.A4[k];
+        tv[k * p.ld[1] + f.Cs + c] = A.A2[k][h];
+        tv[k * p.ld[1] + f.Cs + f.Cv + c] = A.A4[k][h];
       }
   }
+  if constexpr (T2) {
+    if (ts && j < f.Ct) ts[f.Cs + f.Cv + j] = A.A8[0];
+    if (tt) {
+#pragma unroll
+      for (int m = 0; m < 5; ++m) {
+        put(tt + m * p.ld[2], A.A5[m]);
+        if (j < f.Ct) tt[m * p.ld[2] + f.Cs + j] = A.A6[m];
+      }
+#pragma unroll
+      for (int h = 0; h < VC; ++h)
+#pragma unroll
+        for (int m = 0; m < 5; ++m) {
+          const float s7 = cg_apply(g.cg, m, [&](int i, int k) { return A.B[i][k][h]; });
+          if (16 * h + j < f.Cv) tt[m * p.ld[2] + f.Cs + f.Ct + 16 * h + j] = s7;
+        }
+    }
+  }
   __syncthreads();
-  fused_tile_out<false>(p, lds, node0, g.N, wave, lane);
+  fused_tile_out<T2>(p, lds, node0, g.N, wave, lane);
 }
 
-// Whether se3_fwd_fused_rows covers the layer (see its comment), with every array it reads
-// through a buffer resource below 2 GiB.
-bool fused_rows_ok(int64_t N, int Cs, int Cv, bool t2, int64_t E, int P, int ysh) {
+// Whether the row kernel covers the layer: its channels fit the lanes, and every array it reads
+// through a buffer resource is below 2 GiB.
+bool fused_rows_ok(int64_t N, int Cs, int Cv, int Ct, int64_t E, int P, int ysh) {
   const int64_t lim = int64_t{1} << 31;
-  return !t2 && Cs <= 64 && Cv <= 16 && Cs % 4 == 0 && N * Cs * 4 < lim && N * Cv * 12 < lim &&
-         E * 12 < lim && E * P * 4 < lim && E * ysh * 4 < lim;
+  return Cs <= 128 && Cv <= 32 && Ct <= 16 && (Cs <= 16 || (Cs <= 32 ? Cs % 2 == 0 : Cs % 4 == 0)) &&
+         N * Cs * 4 < lim && N * Cv * 12 < lim && N * Ct * 20 < lim && E * 12 < lim &&
+         E * P * 4 < lim && E * ysh * 4 < lim;
+}
+
+// The row kernel with the fewest channels per lane that hold the layer's.
+template <bool T2>
+void launch_fused_rows(const dim3& grid, size_t lds, hipStream_t st, const SeEdges& g, const SeFeat& f,
+                       const SeFused& p) {
+#define GEO_ROWS(U_, SC_, VC_)                                                                      \
+  hipLaunchKernelGGL((se3_fwd_fused_rows<U_, SC_, VC_, T2>), grid, dim3(kSeThreads), lds, st, g, f, p)
+  constexpr int U = T2 ? 2 : 4;
+  if (f.Cv <= 16) {
+    if (f.Cs <= 16) GEO_ROWS(U, 1, 1);
+    else if (f.Cs <= 32) GEO_ROWS(U, 2, 1);
+    else if (f.Cs <= 64) GEO_ROWS(U, 4, 1);
+    else GEO_ROWS(2, 8, 1);
+  } else if (f.Cs <= 32 && f.Cs % 2 == 0) {
+    GEO_ROWS(U, 2, 2);
+  } else if (f.Cs <= 64 && f.Cs % 4 == 0) {
+    GEO_ROWS(2, 4, 2);
+  } else if (f.Cs % 4 == 0) {
+    GEO_ROWS(2, 8, 2);
+  } else {
+    GEO_ROWS(U, 1, 2);
+  }
+#undef GEO_ROWS
 }
 
 // LDS layout of the fused kernel's tile: per present kind, kFuTile * G rows of K + 4 floats.
@@ -1958,7 +2119,7 @@ __global__ __launch_bounds__(kSeThreads) void se3_bwd_src_rows(SeEdges g, const 
   float z0[4] = {0.f, 0.f, 0.f, 0.f}, z3[3][4] = {};
   float z1 = 0.f, z2[3] = {0.f, 0.f, 0.f}, z4[3] = {0.f, 0.f, 0.f};
   for (int base = 0; base < maxdeg; base += kRowStage) {
-    const EdgeCoef<false> st = stage_rows(g, a + base + j, base + j < deg);
+    const RowCoef<false> st = stage_rows<false>(g, a + base + j, base + j < deg);
     const int cnt = min(kRowStage, maxdeg - base);
     static_for<0, kRowStage / U>([&](auto ci) {
       constexpr int c0 = decltype(ci)::value * U;
@@ -2256,9 +2417,10 @@ extern "C" int geo_se3_fwd_fused(const float* s, const float* v, const float* t,
                   path_cols[7] >= 0 || path_cols[8] >= 0;
   const dim3 grid(static_cast<unsigned>(ceil_div(N, kFuTile)));
   hipStream_t st = as_stream(stream);
-  if (fused_rows_ok(N, Cs, Cv, t2, E, P, ysh))
-    hipLaunchKernelGGL((se3_fwd_fused_rows<4>), grid, dim3(kSeThreads), lds, st, g, f, p);
-  else if (t2)
+  if (fused_rows_ok(N, Cs, Cv, Ct, E, P, ysh)) {
+    if (t2) launch_fused_rows<true>(grid, lds, st, g, f, p);
+    else launch_fused_rows<false>(grid, lds, st, g, f, p);
+  } else if (t2)
     hipLaunchKernelGGL((se3_fwd_fused<true, 4>), grid, dim3(kSeThreads), lds, st, g, f, p);
   else
     hipLaunchKernelGGL((se3_fwd_fused<false, 8>), grid, dim3(kSeThreads), lds, st, g, f, p);
