@@ -88,6 +88,29 @@ struct Vec {
   }
 };
 
+// Whether any element of the vector is NaN.
+template <typename T, int VB>
+__device__ __forceinline__ bool any_nan(const Vec<T, VB>& v) {
+  if constexpr (sizeof(T) == 2 && VB >= 4) {  // two bfloat16 per dword: packed 16-bit maximum
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 m = {0, 0};
+#pragma unroll
+    for (int i = 0; i < VB / 4; ++i) {
+      uint32_t w;
+      if constexpr (VB == 16) w = i == 0 ? v.raw.x : (i == 1 ? v.raw.y : (i == 2 ? v.raw.z : v.raw.w));
+      else if constexpr (VB == 8) w = i == 0 ? v.raw.x : v.raw.y;
+      else w = v.raw;
+      m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w & 0x7fff7fffu));
+    }
+    return m.x > 0x7f80 || m.y > 0x7f80;
+  } else {
+    bool n = false;
+#pragma unroll
+    for (int i = 0; i < VB / static_cast<int>(sizeof(T)); ++i) n |= to_acc(v.e[i]) != to_acc(v.e[i]);
+    return n;
+  }
+}
+
 // EPV int32 argmax entries belonging to one vector slice (4..32 bytes).
 template <int N>
 struct IVec {
@@ -131,6 +154,20 @@ template <typename A>
 __device__ __forceinline__ bool max_gt(A a, A b) { return a != a ? (b == b) : (a > b); }
 template <typename A>
 __device__ __forceinline__ bool max_eq(A a, A b) { return a != a ? (b != b) : (a == b); }
+
+// Output and record of one element from its running maximum, first position and count of rows that
+// attain it.  Selects on values formed beforehand: as short-circuit conditions these were three
+// branches per element, about a third of the merge kernel's instructions for bfloat16.
+template <typename T, typename A>
+__device__ __forceinline__ void max_result(A acc, int first, int cnt, int tie_mode, T& out, int& arg) {
+  const T v = from_acc<T>(acc);
+  const T zero = from_acc<T>(A(0));
+  const bool one = (cnt == 1) | (tie_mode == 1);
+  const int rec = one ? first : -cnt;
+  const bool none = cnt == 0;
+  out = none ? zero : v;
+  arg = none ? -1 : rec;
+}
 
 template <typename A>
 __device__ __forceinline__ A shfl_xor_acc(A v, int m) { return __shfl_xor(v, m, kWave); }
@@ -251,8 +288,9 @@ __global__ __launch_bounds__(kSegThreads) void seg_fwd_kernel(
           IVec<EPV> a;
 #pragma unroll
           for (int i = 0; i < EPV; ++i) {
-            res.e[i] = cnt[i] == 0 ? from_acc<T>(A(0)) : from_acc<T>(acc[i]);
-            a.e[i] = cnt[i] == 0 ? -1 : ((cnt[i] == 1 || tie_mode == 1) ? first[i] : -cnt[i]);
+            T o;
+            max_result<T>(acc[i], first[i], cnt[i], tie_mode, o, a.e[i]);
+            res.e[i] = o;
           }
           a.store(arg + s * C + col_off);
         } else if constexpr (OP == GEO_REDUCE_MEAN) {
@@ -412,8 +450,9 @@ __global__ __launch_bounds__(kMergeThreads) void seg_fwd_merge_kernel(
         IVec<EPV> a;
 #pragma unroll
         for (int i = 0; i < EPV; ++i) {
-          res.e[i] = cnt[i] == 0 ? from_acc<T>(A(0)) : from_acc<T>(acc[i]);
-          a.e[i] = cnt[i] == 0 ? -1 : ((cnt[i] == 1 || tie_mode == 1) ? first[i] : -cnt[i]);
+          T o;
+          max_result<T>(acc[i], first[i], cnt[i], tie_mode, o, a.e[i]);
+          res.e[i] = o;
         }
         a.store(arg + s * C + col_off);
       } else if constexpr (OP == GEO_REDUCE_MEAN) {
@@ -444,11 +483,12 @@ __global__ __launch_bounds__(kMergeThreads) void seg_fwd_merge_kernel(
       else park_partial();
     };
 
-    auto locate = [&](int f0, int* e, int* rows) {
+    auto locate = [&](int f0, int* j, int* e, int* rows) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int f = f0 + u;
-        const int b = __shfl(base, lane_of(seg_of(f)), kWave);
+        j[u] = seg_of(f);
+        const int b = __shfl(base, lane_of(j[u]), kWave);
         e[u] = f < hi ? b + f : 0;
       }
 #pragma unroll
@@ -456,8 +496,8 @@ __global__ __launch_bounds__(kMergeThreads) void seg_fwd_merge_kernel(
     };
 
     reset(0x7fffffff);
-    int e[U], rows[U];
-    locate(lo, e, rows);
+    int seg[U], e[U], rows[U];
+    locate(lo, seg, e, rows);
     for (int k = 0; k < steps; ++k) {
       const int f0 = lo + k * U;
       V buf[U];
@@ -466,26 +506,53 @@ __global__ __launch_bounds__(kMergeThreads) void seg_fwd_merge_kernel(
         const bool ok = f0 + u < hi && static_cast<unsigned>(rows[u]) < static_cast<unsigned>(E);
         buf[u].load_stream(msg + row_off(ok ? rows[u] : 0, C) + col_off);
       }
-      int ecur[MAX ? U : 1];
+      int jrow[U], ecur[MAX ? U : 1];
       uint32_t rok = 0;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        jrow[u] = seg[u];
         if constexpr (MAX) ecur[u] = e[u];
         rok |= static_cast<uint32_t>(static_cast<unsigned>(rows[u]) < static_cast<unsigned>(E)) << u;
       }
-      locate(f0 + U, e, rows);
+      locate(f0 + U, seg, e, rows);
+      // Max without a NaN among the step's rows (one wave-uniform test): plain compares, false for
+      // a running maximum that is NaN, which then stands as it should; an absent row is replaced
+      // by NaNs, which no compare takes.  Six vector instructions per element where the NaN-aware
+      // form below takes eleven and eight scalar mask operations (bf16, 588k rows of 64 channels:
+      // 40.5 -> 33.5 us with the branch-free max_result; 4.3 M rows of 128: 371 -> 303 us).
+      bool plain = MAX;
+      if constexpr (MAX) {
+        bool nan = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) nan |= any_nan(buf[u]);
+        plain = __ballot(nan) == 0;
+      }
       // Row values are consumed through selects only, so all U loads stay ahead of first use.
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int f = f0 + u;
         const bool live = f < hi;
-        const int j = seg_of(f);
+        const int j = jrow[u];
         if (live && j != jcur) {
           if (jcur >= 0) finish();
           reset(MAX ? ecur[MAX ? u : 0] : 0);
           jcur = j;
         }
         const bool take = live && ((rok >> u) & 1u);
+        if constexpr (MAX) {
+          if (plain) {  // wave-uniform
+            const int pos = ecur[u];
+#pragma unroll
+            for (int i = 0; i < EPV; ++i) {
+              const A v = take ? to_acc(buf[u].e[i]) : static_cast<A>(__builtin_nanf(""));
+              const bool gt = v > acc[i], eq = v == acc[i];
+              first[i] = gt ? pos : first[i];
+              cnt[i] = gt ? 1 : cnt[i] + (eq ? 1 : 0);
+              acc[i] = gt ? v : acc[i];
+            }
+            continue;
+          }
+        }
 #pragma unroll
         for (int i = 0; i < EPV; ++i) {
           const A v = to_acc(buf[u].e[i]);
@@ -552,10 +619,10 @@ __global__ __launch_bounds__(kMergeThreads) void seg_fwd_merge_kernel(
   }
 }
 
+// Backward of sum and mean.
 template <typename T, int VB, int OP>
 __global__ __launch_bounds__(kSegThreads) void seg_bwd_kernel(
-    const T* __restrict__ grad_out, const T* __restrict__ msg, const T* __restrict__ fwd_out,
-    const int32_t* __restrict__ arg, const int32_t* __restrict__ col_sorted,
+    const T* __restrict__ grad_out, const int32_t* __restrict__ col_sorted,
     const int32_t* __restrict__ perm, const int32_t* __restrict__ seg_start,
     const int32_t* __restrict__ seg_end, int32_t E, int64_t S, int64_t C, int vpr, int log_l,
     int rows_per_wave, T* __restrict__ grad_msg) {
@@ -615,39 +682,119 @@ __global__ __launch_bounds__(kSegThreads) void seg_bwd_kernel(
       }
       if constexpr (OP == GEO_REDUCE_SUM) {
         res = gv;
-      } else if constexpr (OP == GEO_REDUCE_MEAN) {
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) res.e[i] = from_acc<T>(to_acc(gv.e[i]) / scale);
       } else {
-        IVec<EPV> a;
-        if (s_ok) {
-          a.load(arg + row_off(s, C) + col_off);
+        // bfloat16: the float product with the rounded reciprocal is within 1.5 ulp of the quotient,
+        // and a quotient of an 8-bit significand by n <= 4096 that is not exact lies at least 2^-9 / n
+        // (relative) from any point halfway between two bfloat16 values, so both round to the same
+        // one; one division per row instead of EPV
+        if (sizeof(T) == 2 && __ballot(scale > A(4096)) == 0) {
+          const A inv = A(1) / scale;
+#pragma unroll
+          for (int i = 0; i < EPV; ++i) res.e[i] = from_acc<T>(to_acc(gv.e[i]) * inv);
         } else {
 #pragma unroll
-          for (int i = 0; i < EPV; ++i) a.e[i] = -1;
-        }
-        bool any_tie = false;
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) any_tie |= a.e[i] <= -2;
-        V mv, ov;
-        if (any_tie) {
-          mv.load(msg + row_off(p, C) + col_off);
-          ov.load(fwd_out + row_off(s, C) + col_off);
-        }
-#pragma unroll
-        for (int i = 0; i < EPV; ++i) {
-          A r = A(0);
-          if (a.e[i] == static_cast<int>(e)) {
-            r = to_acc(gv.e[i]);
-          } else if (a.e[i] <= -2) {
-            if (max_eq(to_acc(mv.e[i]), to_acc(ov.e[i])))
-              r = to_acc(gv.e[i]) / static_cast<A>(-a.e[i]);
-          }
-          res.e[i] = from_acc<T>(r);
+          for (int i = 0; i < EPV; ++i) res.e[i] = from_acc<T>(to_acc(gv.e[i]) / scale);
         }
       }
       res.store(grad_msg + row_off(p, C) + col_off);
     }
+    }
+  }
+}
+
+// Backward of max: the same row walk.  A row's gradient is the output's where its position is the
+// recorded one, its share where the record counts tied maxima and its message equals the output,
+// and 0 elsewhere.  The rows' gradient and record loads are issued together, at clamped rows, and
+// the message and output rows of a step are read only if one of its elements is tied (bf16 values
+// tie often); the shares are formed only for element columns where some lane needs one.  With a
+// branch around each row's loads, four rows at a time, 588k rows of 64 channels took 36.5 us (bf16)
+// and 33.4 us (fp32) against 30.9 and 28.8 us; one row at a time takes 37.7 and 33.3 us, four 38.6
+// and 29.3.  Every message row is read again where values tie, which sets the bf16 time: 2.2 TB/s of
+// algorithmic bytes, about 4 of actual ones, at 4.3 M rows of 128 channels (587 -> 533 us).
+template <typename T, int VB>
+__global__ __launch_bounds__(kSegThreads) void seg_bwd_max_kernel(
+    const T* __restrict__ grad_out, const T* __restrict__ msg, const T* __restrict__ fwd_out,
+    const int32_t* __restrict__ arg, const int32_t* __restrict__ col_sorted,
+    const int32_t* __restrict__ perm, int32_t E, int64_t S, int64_t C, int vpr, int log_l,
+    int rows_per_wave, T* __restrict__ grad_msg) {
+  using A = typename AccT<T>::type;
+  using V = Vec<T, VB>;
+  constexpr int EPV = V::EPV;
+  constexpr int U = 2;
+  const int lane = lane_id();
+  const int L = 1 << log_l;
+  const int R = kWave >> log_l;
+  const int g = lane >> log_l;
+  const int vl = lane & (L - 1);
+  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kSegWaves + (threadIdx.x / kWave);
+  const int64_t e_begin = wave * rows_per_wave;
+  const int64_t e_stop = min(static_cast<int64_t>(E), e_begin + rows_per_wave);
+  const int ncol_iter = (vpr + L - 1) >> log_l;
+
+  for (int64_t e1 = e_begin; e1 < e_stop; e1 += static_cast<int64_t>(R) * U) {
+    const int64_t e0 = e1 + g;
+    int ss[U], pp[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t e = min(e0 + static_cast<int64_t>(u) * R, e_stop - 1);
+      ss[u] = col_sorted[e];
+      pp[u] = perm ? perm[e] : static_cast<int>(e);
+    }
+    bool s_ok[U], p_ok[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      s_ok[u] = static_cast<unsigned>(ss[u]) < static_cast<unsigned>(S);
+      // not a permutation: the row is not written
+      p_ok[u] = e0 + static_cast<int64_t>(u) * R < e_stop &&
+                static_cast<unsigned>(pp[u]) < static_cast<unsigned>(E);
+      ss[u] = s_ok[u] ? ss[u] : 0;  // S > 0
+      pp[u] = p_ok[u] ? pp[u] : 0;
+    }
+    for (int ci = 0; ci < ncol_iter; ++ci) {
+      const int vb = vl + ci * L;
+      const bool col_ok = vb < vpr;
+      const int64_t col_off = col_ok ? static_cast<int64_t>(vb) * EPV : 0;
+      V gv[U];
+      IVec<EPV> a[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        gv[u].load(grad_out + row_off(ss[u], C) + col_off);
+        a[u].load(arg + row_off(ss[u], C) + col_off);
+      }
+      int low = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) low = min(low, s_ok[u] ? a[u].e[i] : 0);
+      V res[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = static_cast<int>(e0 + static_cast<int64_t>(u) * R);
+#pragma unroll
+        for (int i = 0; i < EPV; ++i) res[u].e[i] = s_ok[u] && a[u].e[i] == e ? gv[u].e[i] : T(0);
+      }
+      if (__ballot(low <= -2)) {  // some element is tied
+        V mv[U], ov[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          mv[u].load(msg + row_off(pp[u], C) + col_off);
+          ov[u].load(fwd_out + row_off(ss[u], C) + col_off);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < EPV; ++i) {
+            const bool share = s_ok[u] && a[u].e[i] <= -2 &&
+                               max_eq(to_acc(mv[u].e[i]), to_acc(ov[u].e[i]));
+            if (__ballot(share)) {
+              const A q = to_acc(gv[u].e[i]) / static_cast<A>(-a[u].e[i]);
+              if (share) res[u].e[i] = from_acc<T>(q);
+            }
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (p_ok[u] && col_ok) res[u].store(grad_msg + row_off(pp[u], C) + col_off);
     }
   }
 }
@@ -734,9 +881,14 @@ int launch_bwd(const Layout& lay, const T* grad_out, const T* msg, const T* fwd_
 #define GEO_BWD_CASE(VBV)                                                                    \
   case VBV:                                                                                  \
     if constexpr (VBV >= static_cast<int>(sizeof(T))) {                                      \
-      hipLaunchKernelGGL((seg_bwd_kernel<T, VBV, OP>), dim3(blocks), dim3(kSegThreads), 0, st, \
-                         grad_out, msg, fwd_out, arg, cs, perm, ns, ne, E, S, C, lay.vpr,     \
-                         lay.log_l, rpw, grad_msg);                                          \
+      if (OP == GEO_REDUCE_MAX && S > 0)                                                     \
+        hipLaunchKernelGGL((seg_bwd_max_kernel<T, VBV>), dim3(blocks), dim3(kSegThreads), 0, st, \
+                           grad_out, msg, fwd_out, arg, cs, perm, E, S, C, lay.vpr, lay.log_l, rpw, \
+                           grad_msg);                                                        \
+      else  /* without segments every row is zero: the sum kernel writes them */             \
+        hipLaunchKernelGGL((seg_bwd_kernel<T, VBV, OP == GEO_REDUCE_MEAN ? OP : GEO_REDUCE_SUM>), \
+                           dim3(blocks), dim3(kSegThreads), 0, st,                           \
+                           grad_out, cs, perm, ns, ne, E, S, C, lay.vpr, lay.log_l, rpw, grad_msg); \
     }                                                                                        \
     break;
   switch (lay.vb) {
