@@ -195,7 +195,28 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The device's current stream as the raw handle (the Stream object costs microseconds)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def plain_eager(x: torch.Tensor) -> bool:
+    """True for a plain tensor in ordinary eager execution: an op may call its implementation
+    directly.  Tensor subclasses, torch.compile, jit tracing, function transforms (torch.func),
+    forward-mode differentiation, batched gradients and dispatch or function modes take the
+    registered custom op, which all of them can see."""
+    return (type(x) is torch.Tensor and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._functorch.is_legacy_batchedtensor(x)
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None)
+
+
+def f32c(t: torch.Tensor) -> torch.Tensor:
+    """t as contiguous float32: itself where it already is."""
+    return t if t.dtype is torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
 
 
 _SAME_DEVICE = contextlib.nullcontext()

@@ -48,6 +48,8 @@ def _hip_ready() -> bool:
 
 
 def _i64(t: Tensor, device: torch.device) -> Tensor:
+    if t.dtype is torch.int64 and t.device == device and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.int64).contiguous()
 
 

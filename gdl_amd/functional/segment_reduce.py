@@ -23,6 +23,7 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
+from gdl_amd._native import plain_eager
 from gdl_amd.csrc import (
     segment_reduce_available,
     segment_reduce_backward_hip,
@@ -142,6 +143,36 @@ _segment_reduce_mean_op.register_autograd(_backward_mean, setup_context=_setup_s
 _segment_reduce_max_op.register_autograd(_backward_max, setup_context=_setup_max)
 
 
+class _SegmentReduceEager(torch.autograd.Function):
+    """Eager mode: the custom ops' forward and backward kernels called directly.  The custom-op
+    layers (schema defaults, dispatch, the registered autograd) cost more host time per call than
+    pooling a batch of graphs takes on the GPU; where anything but plain eager execution is under
+    way the custom ops are used (plain_eager)."""
+
+    @staticmethod
+    def forward(ctx, msg, col_sorted, perm, node_start, node_end, N, reduce, tie_mode):
+        out, arg = segment_reduce_forward_hip(msg, perm, node_start, node_end, N, reduce, tie_mode)
+        saved = (msg, out, arg) if reduce == "max" else ()
+        ctx.save_for_backward(col_sorted, perm, node_start, node_end, *saved)
+        ctx.E, ctx.reduce = msg.shape[0], reduce
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        col_sorted, perm, node_start, node_end, *saved = ctx.saved_tensors
+        msg, out, arg = saved if saved else (None, None, None)
+        # gradients that are recorded themselves (create_graph) go through the op, whose backward
+        # is an error: the kernel's output alone would look like a constant
+        if torch.is_grad_enabled() or not plain_eager(grad_out):
+            g = torch.ops.geoembodied.segment_reduce_backward(
+                grad_out, col_sorted, perm, node_start, node_end, msg, out, arg, ctx.E,
+                _REDUCE_NAMES.index(ctx.reduce))
+        else:
+            g = segment_reduce_backward_hip(grad_out, col_sorted, perm, node_start, node_end, ctx.E,
+                                            ctx.reduce, msg=msg, out=out, arg=arg)
+        return g, None, None, None, None, None, None, None
+
+
 class SegmentReduceFunction(torch.autograd.Function):
     """Segment sum as an autograd.Function (reference name; functional/segment_reduce.py:112-158).
 
@@ -184,6 +215,15 @@ def segment_reduce(
     Returns:
         [N, C] aggregated features in msg's dtype.
     """
+    if reduce == "max" and max_ties not in ("split", "first"):
+        raise ValueError(f"max_ties must be 'split' or 'first', got {max_ties!r}")
+    csr = (col_sorted, perm, node_start, node_end)
+    if (reduce in _REDUCE_NAMES and type(N) is int and all(type(t) is Tensor for t in csr)
+            and plain_eager(msg)):
+        ties = 1 if max_ties == "first" and reduce == "max" else 0
+        if torch.is_grad_enabled() and msg.requires_grad:
+            return _SegmentReduceEager.apply(msg, *csr, N, reduce, ties)
+        return segment_reduce_forward_hip(msg, perm, node_start, node_end, N, reduce, ties)[0]
     if reduce == "sum":
         return torch.ops.geoembodied.segment_reduce_sum(msg, col_sorted, perm, node_start,
                                                         node_end, N)
@@ -191,8 +231,6 @@ def segment_reduce(
         return torch.ops.geoembodied.segment_reduce_mean(msg, col_sorted, perm, node_start,
                                                          node_end, N)
     if reduce == "max":
-        if max_ties not in ("split", "first"):
-            raise ValueError(f"max_ties must be 'split' or 'first', got {max_ties!r}")
         out, _ = torch.ops.geoembodied.segment_reduce_max(
             msg, col_sorted, perm, node_start, node_end, N, 0 if max_ties == "split" else 1)
         return out

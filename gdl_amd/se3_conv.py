@@ -28,7 +28,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from gdl_amd import _native as _nat
-from gdl_amd.csrc import _require_gpu, source_csr
+from gdl_amd.csrc import _i32, _i64, _require_gpu, source_csr
 
 PATH_NAMES = ("w_ss", "w_sv", "w_vv_scalar", "w_vs", "w_vv_cross", "w_st2", "w_t2t2", "w_vt2", "w_t2s")
 
@@ -517,19 +517,19 @@ def se3_message_aggregate(
     dev = scalars.device
     N = int(graph.N)
     f32 = torch.float32
-    s = scalars.to(f32).contiguous()
-    v = vectors.to(f32).contiguous()
+    s = _nat.f32c(scalars)
+    v = _nat.f32c(vectors)
     Cv = v.shape[1]
     if s.shape[0] != N or v.shape[0] != N or v.shape[2] != 3:
         raise ValueError(f"se3_message_aggregate: features {tuple(s.shape)}, {tuple(v.shape)} for N={N}")
-    t = type2.to(f32).contiguous() if type2 is not None else None
+    t = _nat.f32c(type2) if type2 is not None else None
     Ct = t.shape[1] if t is not None else 0
-    Y = graph.Y.to(f32).contiguous()
+    Y = _nat.f32c(graph.Y)
     ysh = Y.shape[1]
     pc = path_columns(weights, t is not None and Ct > 0, ysh >= 9, Ct2_out)
     if t is not None and Ct == 0:
         t = None
-    R = R.to(f32).contiguous()
+    R = _nat.f32c(R)
     P = R.shape[1]
     if max(pc) >= P:
         raise ValueError(f"se3_message_aggregate: {max(pc) + 1} paths run but R has {P} columns")
@@ -542,22 +542,19 @@ def se3_message_aggregate(
     if pc[7] >= 0:
         cg = (cg_11_2.to(device=dev, dtype=f32).contiguous() if cg_11_2 is not None
               else _cg_on(dev))
-    row = graph.row.to(device=dev, dtype=torch.int64).contiguous()
-    col = graph.col.to(device=dev, dtype=torch.int64).contiguous()
-    perm = None if getattr(graph, "_perm_identity", False) else \
-        graph.perm.to(device=dev, dtype=torch.int32).contiguous()
-    ns = graph.node_start.to(device=dev, dtype=torch.int32).contiguous()
-    ne = graph.node_end.to(device=dev, dtype=torch.int32).contiguous()
+    row, col = _i64(graph.row, dev), _i64(graph.col, dev)
+    perm = None if getattr(graph, "_perm_identity", False) else _i32(graph.perm, dev)
+    ns, ne = _i32(graph.node_start, dev), _i32(graph.node_end, dev)
     avg = graph.avg_degree
     avg = (avg.to(device=dev, dtype=f32).contiguous() if avg is not None
            else torch.ones(N, dtype=f32, device=dev))
     m = None
     if mask is not None:
         m = mask.to(device=dev, dtype=torch.bool).reshape(-1).contiguous()
-    b = bias.to(f32).contiguous() if bias is not None and Cs_out > 0 else None
-    Wl = [(weights.get(k).to(f32).contiguous() if weights.get(k) is not None else None)
-          for k in PATH_NAMES]
-    direction = graph.direction.to(f32).contiguous()
+    b = _nat.f32c(bias) if bias is not None and Cs_out > 0 else None
+    Wl = [weights.get(k) for k in PATH_NAMES]
+    Wl = [_nat.f32c(w) if w is not None else None for w in Wl]
+    direction = _nat.f32c(graph.direction)
     args = (s, v, t, row, col, perm, ns, ne, direction, Y, R, avg, m, b, cg, dims, *Wl)
     if _plain_eager(s):
         s_out, v_out, t_out, _, _, _ = _SE3ConvEager.apply(*args)
@@ -668,8 +665,7 @@ def radial_mlp(dist: Tensor, freqs: Tensor, cutoff: float, W1: Tensor, b1: Tenso
     matrix-core kernels up to 16 basis functions, 64 hidden units and 16 outputs, LDS-tiled
     kernels beyond), differentiable with respect to dist and the four weights."""
     _require_gpu("radial_mlp", dist)
-    f = torch.float32
-    c = [x.to(f).contiguous() for x in (dist, freqs, W1, b1, W2, b2)]
+    c = [_nat.f32c(x) for x in (dist, freqs, W1, b1, W2, b2)]
     args = (c[0], c[1], float(cutoff), c[2], c[3], c[4], c[5])
     if _plain_eager(c[0]):
         return _RadialEager.apply(*args)
@@ -760,8 +756,8 @@ class SE3Conv(nn.Module):
             return s_out, v_out
         with torch.autocast(scalars.device.type, enabled=False):
             R = self.radial_basis(graph.dist.to(torch.float32))
-            weights = {k: (getattr(self, k).weight if getattr(self, k) is not None else None)
-                       for k in PATH_NAMES}
+            paths = ((k, getattr(self, k)) for k in PATH_NAMES)
+            weights = {k: (p.weight if p is not None else None) for k, p in paths}
             t_in = type2 if (type2 is not None and self.in_type2_channels > 0) else None
             out = se3_message_aggregate(
                 scalars, vectors, graph, R, weights, self.out_scalar_channels,
