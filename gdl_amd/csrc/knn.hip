@@ -166,8 +166,7 @@ int launch_knn(const float* query, int64_t Nq, const float* source, int64_t Ns,
 // cell edge and shrunk by 1e-5 relative (the fp32 distance of a farther point can round down
 // by less than that).  The stop test is strict, so a source at exactly the k-th distance with a
 // smaller index cannot be missed.  Candidates arrive in cell order, so the register list keeps
-// the total order (d, j) explicitly, as one 64-bit key per entry (distance bits, index): one
-// unsigned compare per step instead of a distance compare plus an index tie-break.
+// the total order (d, j) explicitly, as one 64-bit key per entry (distance bits, index).
 constexpr int kKnnGridThreads = 256;
 constexpr int kKnnSetupThreads = 1024;
 constexpr int kKnnGridMaxAxis = 1024;
@@ -177,6 +176,10 @@ constexpr int kKnnCellCap = 2;            // cells per point
 constexpr int64_t kKnnWideSources = 65536; // one cloud this large: a wave per query for k <= 8
 constexpr int kKnnBoxParts = 64;           // most workgroups per cloud for the bounding box
 constexpr int64_t kKnnBoxChunk = 16384;    // points per bounding-box workgroup
+constexpr int64_t kKnnCloudCells = 65;     // cells of a cloud beyond kKnnCellCap per point, with the end entry
+constexpr int kKnnBuildCells = 16384;      // most cells of a cloud whose grid one workgroup builds (LDS)
+constexpr int64_t kKnnBuildSources = 81920; // most sources of a call that takes that way
+constexpr int kKnnBuildPts = 8;            // points per thread held in registers there
 
 struct KnnGrid {
   float ox, oy, oz, inv_h, h;
@@ -199,7 +202,7 @@ KnnGridWs carve_knn_grid(void* base, int64_t Ns, int64_t B, size_t* bytes) {
   Carver c(base);
   KnnGridWs w;
   const int64_t nn = Ns > 0 ? Ns : 1, bb = B > 0 ? B : 1;
-  w.cells_max = kKnnCellCap * Ns + 64 * bb;
+  w.cells_max = kKnnCellCap * Ns + kKnnCloudCells * bb;
   w.grid = c.take<KnnGrid>(bb);
   w.cell_cnt = c.take<int32_t>(w.cells_max + 1);
   w.cell_scan = c.take<uint64_t>(scan_lookback_elems(w.cells_max + 1));
@@ -253,6 +256,50 @@ __global__ __launch_bounds__(kKnnSetupThreads) void knn_grid_box_part(
   }
 }
 
+// The grid of a cloud of n points with the bounding box lo..hi and at most `cap` cells.
+__device__ KnnGrid knn_make_grid(const float (&lo)[3], const float (&hi)[3], int64_t n, int k, double cap) {
+  KnnGrid g{0.f, 0.f, 0.f, 0.f, 0.f, 1, 1, 1, 0, 1};
+  double ext[3];
+  bool finite = n > 0;
+  for (int a = 0; a < 3; ++a) {
+    ext[a] = static_cast<double>(hi[a]) - static_cast<double>(lo[a]);
+    finite = finite && ext[a] >= 0.0 && ext[a] < 1e30;
+  }
+  if (finite) {
+    const double emax = fmax(fmax(ext[0], ext[1]), ext[2]);
+    const double target = fmax(kKnnCellTarget * k, 1.0);
+    double h = emax;  // fixed point of h = cbrt(prod max(ext, h) * target / n)
+    for (int it = 0; it < 12 && h > 0.0; ++it) {
+      const double next = cbrt(fmax(ext[0], h) * fmax(ext[1], h) * fmax(ext[2], h) * target / static_cast<double>(n));
+      if (next == h) break;  // settled: the further steps would repeat it
+      h = next;
+    }
+    if (h > 0.0) {
+      int64_t d[3] = {1, 1, 1};
+      bool ok = false;
+      for (int it = 0; it < 64 && !ok; ++it) {
+        double prod = 1.0, worst = 0.0;
+        for (int a = 0; a < 3; ++a) {
+          const double q = floor(ext[a] / h) + 1.0;
+          d[a] = q < 4.0 * kKnnGridMaxAxis ? static_cast<int64_t>(q) : 4 * kKnnGridMaxAxis;
+          prod *= static_cast<double>(d[a]);
+          worst = fmax(worst, static_cast<double>(d[a]) / kKnnGridMaxAxis);
+        }
+        ok = prod <= cap && worst <= 1.0;
+        if (!ok) h *= fmax(fmax(cbrt(prod / cap), worst), 1.0) * 1.01;
+      }
+      if (ok) {
+        g.ox = lo[0]; g.oy = lo[1]; g.oz = lo[2];
+        g.inv_h = static_cast<float>(1.0 / h);
+        g.h = static_cast<float>(h * (1.0 - 1e-6));
+        g.dx = static_cast<int>(d[0]); g.dy = static_cast<int>(d[1]); g.dz = static_cast<int>(d[2]);
+      }
+    }
+  }
+  g.ncells = n > 0 ? g.dx * g.dy * g.dz : 0;
+  return g;
+}
+
 // One block per source cloud: bounding box (from `parts` partial boxes when parts > 0), then
 // (thread 0) the grid of that cloud.
 __global__ __launch_bounds__(kKnnSetupThreads) void knn_grid_setup(
@@ -301,44 +348,7 @@ __global__ __launch_bounds__(kKnnSetupThreads) void knn_grid_setup(
     hi[a] = float_from_order_key(m1);
   }
   const int64_t n = sc - sa;
-  KnnGrid g{0.f, 0.f, 0.f, 0.f, 0.f, 1, 1, 1, 0, 1};
-  double ext[3];
-  bool finite = n > 0;
-  for (int a = 0; a < 3; ++a) {
-    ext[a] = static_cast<double>(hi[a]) - static_cast<double>(lo[a]);
-    finite = finite && ext[a] >= 0.0 && ext[a] < 1e30;
-  }
-  if (finite) {
-    const double emax = fmax(fmax(ext[0], ext[1]), ext[2]);
-    const double target = fmax(kKnnCellTarget * k, 1.0);
-    double h = emax;  // fixed point of h = cbrt(prod max(ext, h) * target / n)
-    for (int it = 0; it < 12 && h > 0.0; ++it)
-      h = cbrt(fmax(ext[0], h) * fmax(ext[1], h) * fmax(ext[2], h) * target / static_cast<double>(n));
-    if (h > 0.0) {
-      const double cap = kKnnCellCap * static_cast<double>(n) + 64.0;
-      int64_t d[3] = {1, 1, 1};
-      bool ok = false;
-      for (int it = 0; it < 64 && !ok; ++it) {
-        double prod = 1.0, worst = 0.0;
-        for (int a = 0; a < 3; ++a) {
-          const double q = floor(ext[a] / h) + 1.0;
-          d[a] = q < 4.0 * kKnnGridMaxAxis ? static_cast<int64_t>(q) : 4 * kKnnGridMaxAxis;
-          prod *= static_cast<double>(d[a]);
-          worst = fmax(worst, static_cast<double>(d[a]) / kKnnGridMaxAxis);
-        }
-        ok = prod <= cap && worst <= 1.0;
-        if (!ok) h *= fmax(fmax(cbrt(prod / cap), worst), 1.0) * 1.01;
-      }
-      if (ok) {
-        g.ox = lo[0]; g.oy = lo[1]; g.oz = lo[2];
-        g.inv_h = static_cast<float>(1.0 / h);
-        g.h = static_cast<float>(h * (1.0 - 1e-6));
-        g.dx = static_cast<int>(d[0]); g.dy = static_cast<int>(d[1]); g.dz = static_cast<int>(d[2]);
-      }
-    }
-  }
-  g.ncells = n > 0 ? g.dx * g.dy * g.dz : 0;
-  grid[b] = g;
+  grid[b] = knn_make_grid(lo, hi, n, k, kKnnCellCap * static_cast<double>(n) + 64.0);
 }
 
 // Single block: cell bases (exclusive scan of the cells per cloud).
@@ -403,72 +413,250 @@ __global__ __launch_bounds__(kKnnGridThreads) void knn_grid_scatter(const float*
       make_float4(source[3 * i], source[3 * i + 1], source[3 * i + 2], __int_as_float(static_cast<int>(i)));
 }
 
-// Candidate key: the distance's bits above the source index.  Squared distances are
-// non-negative floats, whose bits order like the values, so one unsigned compare of keys gives
-// the total order used throughout: distance, then source index.  An empty slot holds ~0.
-__device__ __forceinline__ uint64_t knn_key(float d, int j) {
-  return (static_cast<uint64_t>(__float_as_uint(d)) << 32) | static_cast<uint32_t>(j);
-}
-
-// Sorted top-KMAX list of one lane; inserts (d, j) if it is among the KMAX smallest (infinite and
-// NaN distances never enter).
-template <int KMAX>
-__device__ __forceinline__ void knn_insert(uint64_t (&L)[KMAX], float d, int j) {
-  const uint64_t key = knn_key(d, j);
-  if (__float_as_uint(d) < 0x7f800000u && key < L[KMAX - 1]) {
+// The whole grid of one cloud by one workgroup: bounding box, cells counted in LDS, exclusive
+// scan, scatter.  Cloud b's cells start at kKnnCellCap * ptr[b] + kKnnCloudCells * b, so no scan
+// over clouds is needed, and its end entry is its own.  The first kKnnBuildPts * 1024 points stay
+// in registers through all passes, points beyond are read again (their ranks go through global
+// memory).
+// What bounds it: the latency of one load, three barriers' worth of reductions and the serial
+// grid parameters; 16 clouds of 4096 points 7 us, against 27 us and six launches for box, cell
+// bases, zero fill, count, scan and scatter over all clouds (each 2.5 to 6 us, latency as well).
+__global__ __launch_bounds__(kKnnSetupThreads) void knn_grid_build(
+    const float* __restrict__ source, int64_t Ns, const int64_t* __restrict__ ptr_s, int k, KnnGridWs w) {
+  constexpr int T = kKnnSetupThreads, W = T / kWave;
+  __shared__ int cnt[kKnnBuildCells];
+  __shared__ uint32_t red[6][W];
+  __shared__ KnnGrid sg;
+  const int b = blockIdx.x;
+  const int64_t sa = clamp_range(ptr_s[b], Ns);
+  const int64_t sc = max(sa, clamp_range(ptr_s[b + 1], Ns));
+  const int n = static_cast<int>(sc - sa);
+  const float* pts = source + 3 * sa;
+  const int t = threadIdx.x, wv = t / kWave;
+  float px[kKnnBuildPts], py[kKnnBuildPts], pz[kKnnBuildPts];
+  uint32_t mn[3] = {~0u, ~0u, ~0u}, mx[3] = {0u, 0u, 0u};
+  auto grow = [&](float x, float y, float z) {
+    const uint32_t kk[3] = {float_order_key(x), float_order_key(y), float_order_key(z)};
 #pragma unroll
-    for (int m = KMAX - 1; m > 0; --m) {
-      const uint64_t kept = key < L[m] ? key : L[m];
-      L[m] = key < L[m - 1] ? L[m - 1] : kept;
+    for (int a = 0; a < 3; ++a) { mn[a] = min(mn[a], kk[a]); mx[a] = max(mx[a], kk[a]); }
+  };
+  // the points beyond the registers, a batch of independent loads at a time
+  auto rest = [&](auto f) {
+    for (int i0 = kKnnBuildPts * T + t; i0 < n; i0 += kKnnBuildPts * T) {
+      float x[kKnnBuildPts], y[kKnnBuildPts], z[kKnnBuildPts];
+#pragma unroll
+      for (int s = 0; s < kKnnBuildPts; ++s) {
+        const int i = min(i0 + s * T, n - 1);
+        x[s] = pts[3 * i]; y[s] = pts[3 * i + 1]; z[s] = pts[3 * i + 2];
+      }
+#pragma unroll
+      for (int s = 0; s < kKnnBuildPts; ++s)
+        if (i0 + s * T < n) f(i0 + s * T, x[s], y[s], z[s]);
     }
-    L[0] = key < L[0] ? key : L[0];
+  };
+#pragma unroll
+  for (int s = 0; s < kKnnBuildPts; ++s) {
+    const int i = s * T + t;
+    px[s] = py[s] = pz[s] = 0.f;
+    if (i < n) { px[s] = pts[3 * i]; py[s] = pts[3 * i + 1]; pz[s] = pts[3 * i + 2]; }
+  }
+  for (int c = t; c < kKnnBuildCells / 4; c += T) reinterpret_cast<int4*>(cnt)[c] = make_int4(0, 0, 0, 0);
+#pragma unroll
+  for (int s = 0; s < kKnnBuildPts; ++s)
+    if (s * T + t < n) grow(px[s], py[s], pz[s]);
+  rest([&](int, float x, float y, float z) { grow(x, y, z); });
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    mn[a] = wave_min_u32(mn[a]);
+    mx[a] = wave_max_u32(mx[a]);
+  }
+  if (lane_id() == 0) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) { red[a][wv] = mn[a]; red[3 + a][wv] = mx[a]; }
+  }
+  __syncthreads();
+  if (t == 0) {
+    float lo[3], hi[3];
+    for (int a = 0; a < 3; ++a) {
+      uint32_t m0 = red[a][0], m1 = red[3 + a][0];
+#pragma unroll
+      for (int ww = 1; ww < W; ++ww) { m0 = min(m0, red[a][ww]); m1 = max(m1, red[3 + a][ww]); }
+      lo[a] = float_from_order_key(m0);
+      hi[a] = float_from_order_key(m1);
+    }
+    const double cells = kKnnCellCap * static_cast<double>(n) + 64.0;
+    KnnGrid g = knn_make_grid(lo, hi, n, k, fmin(cells, static_cast<double>(kKnnBuildCells)));
+    g.base = static_cast<int>(kKnnCellCap * sa + kKnnCloudCells * b);
+    sg = g;
+    w.grid[b] = g;
+  }
+  __syncthreads();
+  const KnnGrid g = sg;
+  auto cell_of = [&](float x, float y, float z) {
+    float u;
+    const int cx = knn_cell_coord(x, g.ox, g.inv_h, g.dx, &u);
+    const int cy = knn_cell_coord(y, g.oy, g.inv_h, g.dy, &u);
+    const int cz = knn_cell_coord(z, g.oz, g.inv_h, g.dz, &u);
+    return (cx * g.dy + cy) * g.dz + cz;
+  };
+  int cell[kKnnBuildPts], rank[kKnnBuildPts];
+#pragma unroll
+  for (int s = 0; s < kKnnBuildPts; ++s) {
+    cell[s] = rank[s] = 0;
+    if (s * T + t < n) {
+      cell[s] = cell_of(px[s], py[s], pz[s]);
+      rank[s] = atomicAdd(&cnt[cell[s]], 1);
+    }
+  }
+  rest([&](int i, float x, float y, float z) { w.pt_rank[sa + i] = atomicAdd(&cnt[cell_of(x, y, z)], 1); });
+  __syncthreads();
+  // exclusive scan: `per` consecutive cells a thread, the sums over the waves in LDS
+  const int per = (g.ncells + T - 1) / T;
+  const int c0 = min(t * per, g.ncells), c1 = min(c0 + per, g.ncells);
+  int sum = 0;
+  for (int c = c0; c < c1; ++c) sum += cnt[c];
+  const int inc = static_cast<int>(wave_inclusive_sum_dpp(static_cast<uint32_t>(sum)));
+  if (lane_id() == kWave - 1) red[0][wv] = static_cast<uint32_t>(inc);
+  __syncthreads();
+  int off = static_cast<int>(sa) + inc - sum;
+  for (int ww = 0; ww < wv; ++ww) off += static_cast<int>(red[0][ww]);
+  for (int c = c0; c < c1; ++c) {
+    const int v = cnt[c];
+    cnt[c] = off;
+    off += v;
+  }
+  __syncthreads();
+  for (int c = t; c < g.ncells; c += T) w.cell_start[g.base + c] = cnt[c];
+  if (t == 0) w.cell_start[g.base + g.ncells] = static_cast<int>(sc);
+#pragma unroll
+  for (int s = 0; s < kKnnBuildPts; ++s) {
+    const int i = s * T + t;
+    if (i < n)
+      w.spos[cnt[cell[s]] + rank[s]] = make_float4(px[s], py[s], pz[s], __int_as_float(static_cast<int>(sa) + i));
+  }
+  rest([&](int i, float x, float y, float z) {
+    w.spos[cnt[cell_of(x, y, z)] + w.pt_rank[sa + i]] =
+        make_float4(x, y, z, __int_as_float(static_cast<int>(sa) + i));
+  });
+}
+
+// Candidate key: the distance's bits above the source index, read as a double.  Squared distances
+// are non-negative floats, whose bits order like the values, and positive doubles order like their
+// bits, so one compare gives the total order used throughout (distance, then source index), and
+// min and max are one instruction each.  No key has the exponent of an infinity or a NaN: the high
+// word is at most 0x7f800000.  An empty slot holds kKnnNone, above every finite distance.
+__device__ __forceinline__ double knn_key(float d, int j) {
+  return __hiloint2double(__float_as_int(d), j);
+}
+__device__ __forceinline__ double knn_none() { return __hiloint2double(0x7f800000, 0); }
+__device__ __forceinline__ double knn_min(double a, double b) {
+  double r;  // the instruction itself: fmin() would first quieten operands that are never NaN
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double knn_max(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// Sorted list of one lane, of which at most the first `used` slots are taken; inserts (d, j) if it
+// is below the last slot and below lim (infinite and NaN distances never enter).
+template <int KMAX>
+__device__ __forceinline__ void knn_insert(double (&L)[KMAX], int used, double lim, float d, int j) {
+  const double key = knn_key(d, j);
+  if (__float_as_uint(d) < 0x7f800000u && key < lim && key < L[KMAX - 1]) {
+#pragma unroll
+    for (int m = KMAX - 1; m > 0; --m)
+      if (m <= used) L[m] = knn_max(L[m - 1], knn_min(key, L[m]));
+    L[0] = knn_min(key, L[0]);
   }
 }
 
-// Merge with the list of the lane `mask` away: keep the KMAX smallest of both, sorted.  The
-// element-wise minimum of one list and the other reversed is bitonic and holds exactly the KMAX
-// smallest; half-cleaners sort it.  Both lanes end with the same list.
-template <int KMAX>
-__device__ __forceinline__ void knn_merge_xor(uint64_t (&L)[KMAX], int mask) {
-  uint64_t P[KMAX];
+// Merge with the list of another lane (at lane ^ MASK, or mirrored where every lane of the halves
+// holds the same list): keep the KMAX smallest of both, sorted.  The element-wise minimum of one
+// list and the other reversed is bitonic and holds exactly the KMAX smallest; half-cleaners sort
+// it.  Both lanes end with the same list.
+template <int KMAX, int MASK>
+__device__ __forceinline__ void knn_merge(double (&L)[KMAX]) {
+  auto other = [](int v) -> int {
+    if constexpr (MASK == 1) return static_cast<int>(dpp_u32<kDppXor1>(static_cast<uint32_t>(v)));
+    else if constexpr (MASK == 2) return static_cast<int>(dpp_u32<kDppXor2>(static_cast<uint32_t>(v)));
+    else if constexpr (MASK == 4) return static_cast<int>(dpp_u32<kDppHalfMirror>(static_cast<uint32_t>(v)));
+    else if constexpr (MASK == 8) return static_cast<int>(dpp_u32<kDppMirror>(static_cast<uint32_t>(v)));
+    else return __shfl_xor(v, MASK, kWave);
+  };
+  double P[KMAX];
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i) {
-    const uint32_t lo = static_cast<uint32_t>(__shfl_xor(static_cast<int>(static_cast<uint32_t>(L[i])), mask, kWave));
-    const uint32_t hi = static_cast<uint32_t>(__shfl_xor(static_cast<int>(static_cast<uint32_t>(L[i] >> 32)), mask, kWave));
-    P[i] = (static_cast<uint64_t>(hi) << 32) | lo;
-  }
+  for (int i = 0; i < KMAX; ++i) P[i] = __hiloint2double(other(__double2hiint(L[i])), other(__double2loint(L[i])));
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i) {
-    const uint64_t o = P[KMAX - 1 - i];
-    L[i] = o < L[i] ? o : L[i];
-  }
+  for (int i = 0; i < KMAX; ++i) L[i] = knn_min(L[i], P[KMAX - 1 - i]);
 #pragma unroll
   for (int sd = KMAX / 2; sd > 0; sd >>= 1) {
 #pragma unroll
     for (int i = 0; i < KMAX; ++i) {
       if ((i & sd) == 0) {
-        const uint64_t a = L[i], c = L[i + sd];
-        const bool sw = c < a;
-        L[i] = sw ? c : a;
-        L[i + sd] = sw ? a : c;
+        const double a = L[i], c = L[i + sd];
+        L[i] = knn_min(a, c);
+        L[i + sd] = knn_max(a, c);
       }
     }
   }
 }
+template <int KMAX, int G>
+__device__ __forceinline__ void knn_merge_group(double (&L)[KMAX]) {
+  knn_merge<KMAX, 1>(L);
+  knn_merge<KMAX, 2>(L);
+  knn_merge<KMAX, 4>(L);
+  if constexpr (G >= 16) knn_merge<KMAX, 8>(L);
+  if constexpr (G >= 32) knn_merge<KMAX, 16>(L);
+  if constexpr (G >= 64) knn_merge<KMAX, 32>(L);
+}
 
 // G lanes per query: the lanes of a group split every visited cell range (consecutive sources,
-// so the group's loads are contiguous), each keeps its own sorted top-KMAX, the stop test counts
-// the group's candidates below the bound (exact: a lane that dropped a candidate below the bound
-// already holds KMAX >= k of them), and the lists are merged pairwise at the end.
+// so the group's loads are contiguous), and each keeps its own sorted list of its KMAX nearest.
+// After every step the lists are merged, the stop test reads the k-th key, and where the search
+// goes on lane 0 keeps the merged list and the others start empty.
+//
+// What bounded the earlier form of this search was the chain of dependent loads: it read the
+// bounds of one row of cells and then that row's points, nine times for the 27 cells around the
+// query and 34 times for the next shell, and the 64-bit integer list steps beside it.  Here
+//  - the first step takes the 27 cells at once: the nine rows' bounds come with one load per lane
+//    and the first G points of every row with nine independent loads (G = 64, a query in a dense
+//    part of one large cloud, starts with the query's own cell instead);
+//  - in a later shell every lane forms one row (or one of the two cells) of the shell, drops it or
+//    cuts its z range if the k-th distance rules it out, and reads its bounds; the group then
+//    goes through the ranges that are left, two at a time;
+//  - the list steps are one minimum and one maximum of doubles per slot (knn_key), and the i-th
+//    point of the first step can only have i slots in front of it.
+// A dropped row or cell is at least its distance in cell units minus 1e-3 of a cell per axis away,
+// scaled and shrunk as the stop test's bound is.
+// Whole calls with the one-workgroup grid, before -> now: 16 clouds of 4096 points on a sphere, a
+// quarter of them as queries, k = 16 60 -> 27 us, k = 3 43 -> 21 us; cubes of 4096 points, k = 16 87
+// -> 29 us.  With the grid by six launches as before: 32 cubes x 4096 queries, k = 32 821 -> 253 us;
+// a lidar frame of 131,072 points against itself, k = 8 500 -> 325 us, a quarter of it k = 16 407 ->
+// 318 us; 512 cubes of 1024 points, k = 3 133 -> 96 us.
 template <int KMAX, int G>
 __global__ __launch_bounds__(kKnnGridThreads) void knn_grid_query(
     const float* __restrict__ query, int64_t Nq, const int64_t* __restrict__ ptr_q, int64_t B,
     KnnGridWs w, int k, int64_t* __restrict__ out_idx, float* __restrict__ out_dist) {
+  constexpr bool kBlock = G < kWave;  // first step: 27 cells
   const int64_t gt = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t q = gt / G;
-  const int gl = static_cast<int>(gt % G);
+  const int lane = lane_id(), gl = lane % G, gb = lane - gl;
+  int64_t b = 0;
+  if (B <= kWave) {
+    // the wave's 64 / G queries against all cloud ends at once
+    const int64_t end = lane < B ? ptr_q[lane + 1] : INT64_MAX;
+    const int64_t q0 = (gt - lane) / G;
+#pragma unroll
+    for (int i = 0; i < kWave / G; ++i) {
+      const int c = __popcll(__ballot(end <= q0 + i));
+      if (gb == i * G) b = c;
+    }
+  }
   if (q >= Nq) return;  // whole groups leave together (G divides the block)
-  const int64_t b = cloud_of_index(ptr_q, B, q);
+  if (B > kWave) b = cloud_of_index(ptr_q, B, q);
   const bool covered = b < B && q >= ptr_q[b] && q < ptr_q[b + 1];
   if (!covered || w.grid[b].ncells == 0) {  // no cloud, or an empty source cloud: padding
     for (int i = gl; i < k; i += G) {
@@ -478,38 +666,60 @@ __global__ __launch_bounds__(kKnnGridThreads) void knn_grid_query(
     return;
   }
   const KnnGrid g = w.grid[b];
+  const int32_t* __restrict__ cell_start = w.cell_start + g.base;
   const float qx = query[3 * q], qy = query[3 * q + 1], qz = query[3 * q + 2];
   float ux, uy, uz;
   const int cx = knn_cell_coord(qx, g.ox, g.inv_h, g.dx, &ux);
   const int cy = knn_cell_coord(qy, g.oy, g.inv_h, g.dy, &uy);
   const int cz = knn_cell_coord(qz, g.oz, g.inv_h, g.dz, &uz);
-  uint64_t L[KMAX];
+  const double none = knn_none();
+  double L[KMAX];
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i) L[i] = ~0ull;
+  for (int i = 0; i < KMAX; ++i) L[i] = none;
+  double lim = none;  // the k-th key so far
 
-  auto visit = [&](int a, int e) {
-    for (int p = a + gl; p < e; p += G) {
-      const float4 s = w.spos[p];
-      knn_insert<KMAX>(L, sqdist(qx, qy, qz, s.x, s.y, s.z), __float_as_int(s.w));
-    }
+  auto insert = [&](const float4& s, int used) {
+    knn_insert<KMAX>(L, used, lim, sqdist(qx, qy, qz, s.x, s.y, s.z), __float_as_int(s.w));
   };
-  const int maxr = max(max(g.dx, g.dy), g.dz);
-  for (int r = 0; r <= maxr; ++r) {
-    const int x0 = max(cx - r, 0), x1 = min(cx + r, g.dx - 1);
-    const int y0 = max(cy - r, 0), y1 = min(cy + r, g.dy - 1);
-    const int z0 = max(cz - r, 0), z1 = min(cz + r, g.dz - 1);
-    for (int ix = x0; ix <= x1; ++ix) {
-      const bool xface = ix == cx - r || ix == cx + r;
-      for (int iy = y0; iy <= y1; ++iy) {
-        const int c0 = g.base + (ix * g.dy + iy) * g.dz;
-        if (xface || iy == cy - r || iy == cy + r) {
-          visit(w.cell_start[c0 + z0], w.cell_start[c0 + z1 + 1]);
-        } else {
-          if (cz - r >= 0) visit(w.cell_start[c0 + cz - r], w.cell_start[c0 + cz - r + 1]);
-          if (cz + r < g.dz) visit(w.cell_start[c0 + cz + r], w.cell_start[c0 + cz + r + 1]);
-        }
+  int r = kBlock ? 1 : 0;
+  if constexpr (kBlock) {
+    auto bounds = [&](int i) {  // of the i-th of the nine rows
+      const int ix = cx - 1 + i / 3, iy = cy - 1 + i % 3;
+      int2 v = make_int2(0, 0);
+      if (i < 9 && ix >= 0 && ix < g.dx && iy >= 0 && iy < g.dy) {
+        const int c = (ix * g.dy + iy) * g.dz;
+        v = make_int2(cell_start[c + max(cz - 1, 0)], cell_start[c + min(cz + 1, g.dz - 1) + 1]);
       }
+      return v;
+    };
+    const int2 own = bounds(gl);
+    int2 row[9];
+    float4 s[9];
+    if constexpr (G < 9) row[8] = bounds(8);
+    bool more = false;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+      if (i < G) row[i] = make_int2(__shfl(own.x, gb + i, kWave), __shfl(own.y, gb + i, kWave));
+      const int p = row[i].x + gl;
+      s[i] = w.spos[p < row[i].y ? p : 0];
+      more = more || row[i].x + G < row[i].y;
     }
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+      if (row[i].x + gl < row[i].y) insert(s[i], i);
+    if (more) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+        for (int p = row[i].x + G + gl; p < row[i].y; p += G) insert(w.spos[p], KMAX);
+    }
+  } else {
+    const int c = (cx * g.dy + cy) * g.dz + cz;
+    for (int p = cell_start[c] + gl, e = cell_start[c + 1]; p < e; p += G) insert(w.spos[p], KMAX);
+  }
+  const int maxr = max(max(g.dx, g.dy), g.dz);
+  const float ih2 = 1.00003f / (g.h * g.h);
+  for (;;) {
+    knn_merge_group<KMAX, G>(L);
     // distance (cell units) from the query to the faces of the visited block that still have
     // cells beyond them
     float gap = __builtin_inff();
@@ -522,24 +732,77 @@ __global__ __launch_bounds__(kKnnGridThreads) void knn_grid_query(
     if (gap == __builtin_inff()) break;  // every cell of the cloud visited
     const float gr = (gap - 1e-3f) * g.h;
     const float bound = gap > 1e-3f ? gr * gr * (1.0f - 1e-5f) : 0.0f;
-    const uint64_t bound_key = static_cast<uint64_t>(__float_as_uint(bound)) << 32;
-    int below = 0;
 #pragma unroll
-    for (int i = 0; i < KMAX; ++i) below += L[i] < bound_key ? 1 : 0;
+    for (int i = 0; i < KMAX; ++i)
+      if (i == k - 1) lim = L[i];
+    if (lim < knn_key(bound, 0) || ++r > maxr) break;
+    if (gl != 0) {
 #pragma unroll
-    for (int m = 1; m < G; m <<= 1) below += __shfl_xor(below, m, kWave);
-    if (below >= k) break;
+      for (int i = 0; i < KMAX; ++i) L[i] = none;
+    }
+    // shell r: rows on its x and y faces whole, the others by their two end cells
+    const float kd = __int_as_float(__double2hiint(lim));  // inf while fewer than k are known
+    const float cut = kd * ih2;                            // in squared cell units
+    const int x0 = max(cx - r, 0), y0 = max(cy - r, 0);
+    const int ny = min(cy + r, g.dy - 1) - y0 + 1;
+    const int items = 2 * (min(cx + r, g.dx - 1) - x0 + 1) * ny;
+    for (int t0 = 0; t0 < items; t0 += G) {
+      const int t = t0 + gl;
+      int2 own = make_int2(0, 0);
+      if (t < items) {
+        const unsigned rw = static_cast<unsigned>(t) >> 1;
+        const int ix = x0 + static_cast<int>(rw / static_cast<unsigned>(ny));
+        const int iy = y0 + static_cast<int>(rw % static_cast<unsigned>(ny));
+        const float fx = static_cast<float>(ix), fy = static_cast<float>(iy);
+        const float dx = fmaxf(fmaxf(fx - ux, ux - fx - 1.0f) - 1e-3f, 0.0f);
+        const float dy = fmaxf(fmaxf(fy - uy, uy - fy - 1.0f) - 1e-3f, 0.0f);
+        const float rem = cut - (dx * dx + dy * dy);
+        int za = 0, zb = -1;
+        if (!(rem < 0.0f)) {
+          const float rz = sqrtf(rem) + 2e-3f;
+          const bool face = ix == cx - r || ix == cx + r || iy == cy - r || iy == cy + r;
+          if (!face) {
+            za = zb = (t & 1) ? cz + r : cz - r;
+            const float fz = static_cast<float>(za);
+            if (za < 0 || za >= g.dz || fz - uz > rz || uz - fz - 1.0f > rz) zb = za - 1;
+          } else if ((t & 1) == 0) {
+            // a cell that ends below uz - rz or begins above uz + rz is too far
+            const float z0 = static_cast<float>(max(cz - r, 0)), z1 = static_cast<float>(min(cz + r, g.dz - 1));
+            za = static_cast<int>(fminf(fmaxf(floorf(uz - rz), z0), z1 + 1.0f));
+            zb = static_cast<int>(fmaxf(fminf(floorf(uz + rz), z1), z0 - 1.0f));
+          }
+        }
+        if (za <= zb) {
+          const int c = (ix * g.dy + iy) * g.dz;
+          own = make_int2(cell_start[c + za], cell_start[c + zb + 1]);
+        }
+      }
+      uint64_t left = __ballot(own.x < own.y) >> gb;
+      if constexpr (G < kWave) left &= (1ull << G) - 1;
+      while (left != 0) {
+        const int i0 = __builtin_ctzll(left);
+        left &= left - 1;
+        const int i1 = left != 0 ? __builtin_ctzll(left) : i0;
+        const bool two = left != 0;
+        left &= left - 1;
+        const int a0 = __shfl(own.x, gb + i0, kWave), e0 = __shfl(own.y, gb + i0, kWave);
+        const int a1 = __shfl(own.x, gb + i1, kWave), e1 = two ? __shfl(own.y, gb + i1, kWave) : a1;
+        const float4 s0 = w.spos[a0 + gl < e0 ? a0 + gl : 0], s1 = w.spos[a1 + gl < e1 ? a1 + gl : 0];
+        if (a0 + gl < e0) insert(s0, KMAX);
+        if (a1 + gl < e1) insert(s1, KMAX);
+        for (int p = a0 + G + gl; p < e0; p += G) insert(w.spos[p], KMAX);
+        for (int p = a1 + G + gl; p < e1; p += G) insert(w.spos[p], KMAX);
+      }
+    }
   }
-#pragma unroll
-  for (int m = 1; m < G; m <<= 1) knn_merge_xor<KMAX>(L, m);
   int64_t* oi = out_idx + q * k;
   float* od = out_dist + q * k;
 #pragma unroll
   for (int i = 0; i < KMAX; ++i) {
     if (i < k && i % G == gl) {
-      const bool any = L[i] != ~0ull;
-      oi[i] = any ? static_cast<int64_t>(static_cast<int32_t>(static_cast<uint32_t>(L[i]))) : -1;
-      od[i] = any ? __uint_as_float(static_cast<uint32_t>(L[i] >> 32)) : 1e30f;
+      const bool any = L[i] < none;
+      oi[i] = any ? static_cast<int64_t>(__double2loint(L[i])) : -1;
+      od[i] = any ? __int_as_float(__double2hiint(L[i])) : 1e30f;
     }
   }
 }
@@ -553,36 +816,47 @@ int launch_knn_grid(const float* query, int64_t Nq, const float* source, int64_t
                     float* out_dist, void* workspace, hipStream_t st) {
   size_t bytes = 0;
   const KnnGridWs w = carve_knn_grid(workspace, Ns, B, &bytes);
-  // Clouds of more than 2 * kKnnBoxChunk points on average: the bounding box is reduced by up to
-  // kKnnBoxParts workgroups per cloud first (one workgroup reading a 131,072-point cloud took
-  // 23 us), the setup then combines their partial boxes.
-  const int64_t avg = ceil_div(Ns, B);
-  const int64_t want = ceil_div(avg, kKnnBoxChunk);
-  const int parts = avg > 2 * kKnnBoxChunk ? static_cast<int>(want < kKnnBoxParts ? want : kKnnBoxParts) : 0;
-  if (parts > 0) {
-    hipLaunchKernelGGL(knn_grid_box_part, dim3(parts, static_cast<unsigned>(B)),
-                       dim3(kKnnSetupThreads), 0, st, source, Ns, ptr_s, parts, w.box_part);
-    GEO_LAUNCH_CHECK("knn_grid_box_part");
+  // Clouds of up to kKnnBuildCells / kKnnCellCap points on average: each cloud's grid by one
+  // workgroup, 7 us and one launch against 27 us and six (16 clouds of 4096 points).  The sizes are not known here, and
+  // one cloud may hold nearly all points: one workgroup needs as long as the six launches for about
+  // 25,000 points and 70 us more for 65,000 (four clouds of 16,384 and four of 1 point, k = 16, 70
+  // -> 46 us in all; 15 clouds of 64 points and one of 64,576 92 -> 133 us), so the sum is bounded.
+  if (Ns <= B * (kKnnBuildCells / kKnnCellCap) && Ns <= kKnnBuildSources) {
+    hipLaunchKernelGGL(knn_grid_build, dim3(static_cast<unsigned>(B)), dim3(kKnnSetupThreads), 0, st, source, Ns,
+                       ptr_s, k, w);
+    GEO_LAUNCH_CHECK("knn_grid_build");
+  } else {
+    // Clouds of more than 2 * kKnnBoxChunk points on average: the bounding box is reduced by up to
+    // kKnnBoxParts workgroups per cloud first (one workgroup reading a 131,072-point cloud took
+    // 23 us), the setup then combines their partial boxes.
+    const int64_t avg = ceil_div(Ns, B);
+    const int64_t want = ceil_div(avg, kKnnBoxChunk);
+    const int parts = avg > 2 * kKnnBoxChunk ? static_cast<int>(want < kKnnBoxParts ? want : kKnnBoxParts) : 0;
+    if (parts > 0) {
+      hipLaunchKernelGGL(knn_grid_box_part, dim3(parts, static_cast<unsigned>(B)),
+                         dim3(kKnnSetupThreads), 0, st, source, Ns, ptr_s, parts, w.box_part);
+      GEO_LAUNCH_CHECK("knn_grid_box_part");
+    }
+    hipLaunchKernelGGL(knn_grid_setup, dim3(B), dim3(kKnnSetupThreads), 0, st, source, Ns, ptr_s, k,
+                       w.grid, w.box_part, parts);
+    GEO_LAUNCH_CHECK("knn_grid_setup");
+    hipLaunchKernelGGL(knn_grid_base, dim3(1), dim3(kScanThreads), 0, st, w.grid, B);
+    GEO_LAUNCH_CHECK("knn_grid_base");
+    // cell counts and the scan's look-back status are carved next to each other: one zero fill
+    const int64_t zero_words =
+        (reinterpret_cast<char*>(w.cell_scan + scan_lookback_elems(w.cells_max + 1)) -
+         reinterpret_cast<char*>(w.cell_cnt)) / static_cast<int64_t>(sizeof(int32_t));
+    int rc = device_fill<int32_t>(w.cell_cnt, zero_words, 0, st);
+    if (rc) return rc;
+    const unsigned gs = static_cast<unsigned>(ceil_div(Ns, kKnnGridThreads));
+    hipLaunchKernelGGL(knn_grid_cell, dim3(gs), dim3(kKnnGridThreads), 0, st, source, Ns, ptr_s, B, w);
+    GEO_LAUNCH_CHECK("knn_grid_cell");
+    rc = device_exclusive_scan_lookback<int32_t, int32_t>(w.cell_cnt, w.cells_max + 1, w.cell_start,
+                                                          nullptr, false, w.cell_scan, st);
+    if (rc) return rc;
+    hipLaunchKernelGGL(knn_grid_scatter, dim3(gs), dim3(kKnnGridThreads), 0, st, source, Ns, w);
+    GEO_LAUNCH_CHECK("knn_grid_scatter");
   }
-  hipLaunchKernelGGL(knn_grid_setup, dim3(B), dim3(kKnnSetupThreads), 0, st, source, Ns, ptr_s, k,
-                     w.grid, w.box_part, parts);
-  GEO_LAUNCH_CHECK("knn_grid_setup");
-  hipLaunchKernelGGL(knn_grid_base, dim3(1), dim3(kScanThreads), 0, st, w.grid, B);
-  GEO_LAUNCH_CHECK("knn_grid_base");
-  // cell counts and the scan's look-back status are carved next to each other: one zero fill
-  const int64_t zero_words =
-      (reinterpret_cast<char*>(w.cell_scan + scan_lookback_elems(w.cells_max + 1)) -
-       reinterpret_cast<char*>(w.cell_cnt)) / static_cast<int64_t>(sizeof(int32_t));
-  int rc = device_fill<int32_t>(w.cell_cnt, zero_words, 0, st);
-  if (rc) return rc;
-  const unsigned gs = static_cast<unsigned>(ceil_div(Ns, kKnnGridThreads));
-  hipLaunchKernelGGL(knn_grid_cell, dim3(gs), dim3(kKnnGridThreads), 0, st, source, Ns, ptr_s, B, w);
-  GEO_LAUNCH_CHECK("knn_grid_cell");
-  rc = device_exclusive_scan_lookback<int32_t, int32_t>(w.cell_cnt, w.cells_max + 1, w.cell_start,
-                                                        nullptr, false, w.cell_scan, st);
-  if (rc) return rc;
-  hipLaunchKernelGGL(knn_grid_scatter, dim3(gs), dim3(kKnnGridThreads), 0, st, source, Ns, w);
-  GEO_LAUNCH_CHECK("knn_grid_scatter");
   // Lanes per query: a wave runs as long as its slowest query.  In one scene-scale cloud (a
   // lidar frame) density varies by orders of magnitude, so the few queries in dense regions
   // scan hundreds of candidates: a whole wave per query for k <= 8 there (C5 with 8 lanes
