@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kKnnGridThreads) void knn_grid_scatter(const float*
 // in registers through all passes, points beyond are read again (their ranks go through global
 // memory).
 // What bounds it: the latency of one load, three barriers' worth of reductions and the serial
-// grid parameters; 16 clouds of 4096 points 7 us, against 27 us and six launches for box, cell
+// grid parameters; 16 clouds of about 4096 points 10 us, against 27 us and six launches for box, cell
 // bases, zero fill, count, scan and scatter over all clouds (each 2.5 to 6 us, latency as well).
 __global__ __launch_bounds__(kKnnSetupThreads) void knn_grid_build(
     const float* __restrict__ source, int64_t Ns, const int64_t* __restrict__ ptr_s, int k, KnnGridWs w) {
@@ -817,7 +817,7 @@ int launch_knn_grid(const float* query, int64_t Nq, const float* source, int64_t
   size_t bytes = 0;
   const KnnGridWs w = carve_knn_grid(workspace, Ns, B, &bytes);
   // Clouds of up to kKnnBuildCells / kKnnCellCap points on average: each cloud's grid by one
-  // workgroup, 7 us and one launch against 27 us and six (16 clouds of 4096 points).  The sizes are not known here, and
+  // workgroup, 10 us and one launch against 27 us and six (16 clouds of about 4096 points).  The sizes are not known here, and
   // one cloud may hold nearly all points: one workgroup needs as long as the six launches for about
   // 25,000 points and 70 us more for 65,000 (four clouds of 16,384 and four of 1 point, k = 16, 70
   // -> 46 us in all; 15 clouds of 64 points and one of 64,576 92 -> 133 us), so the sum is bounded.

@@ -25,8 +25,8 @@
 // geo_radius_emit:
 //   rg_compact  kRgGroup lanes per target: the list sorted by source index into the CSR row;
 //               targets with more than K sources (or long lists) are done by the whole wave:
-//               the K smallest (d, j) by a radix select on the distance bits of the in-radius
-//               candidates staged in LDS (a binary search over the stencil beyond kRgSelCap)
+//               the K smallest (d, j) by a histogram of the distances of the in-radius
+//               candidates, staged in LDS (all of them, or those up to the K-th's bin)
 //   rg_emit     (lists too large for the workspace) re-scans the stencil per target instead
 // Traversal order inside a cell is not deterministic (atomic ranks) and does not matter: the
 // accepted set is defined by a total order and the output is sorted.
@@ -733,8 +733,14 @@ __global__ __launch_bounds__(kRgThreads) void rg_count(RgWs w, const int64_t* __
   };
 #pragma unroll
   for (int r = 0; r < 9; ++r) take(sv[r], sub < rn[r]);
-  for (int r = 0; r < 9; ++r) {
-    for (int m0 = kRgGroup; m0 < rn[r]; m0 += kRgGroup) {  // group-uniform trip count
+  // A target with more than K sources is searched again by rg_compact, which needs to know only
+  // that there are more: the group stops there.  The runs through the target's own column and the
+  // four beside it come first, where more of the sources are in radius.
+  constexpr int kOrder[9] = {4, 1, 3, 5, 7, 0, 2, 6, 8};
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const int r = kOrder[i];
+    for (int m0 = kRgGroup; m0 < rn[r] && c <= K; m0 += kRgGroup) {  // group-uniform trip count
       const bool ok = m0 + sub < rn[r];
       take(ok ? w.spos[ra[r] + m0 + sub] : make_float4(0.f, 0.f, 0.f, 0.f), ok);
     }
@@ -752,8 +758,14 @@ __global__ __launch_bounds__(kRgThreads) void rg_count(RgWs w, const int64_t* __
 // than K sources, or lists longer than the registers hold, are done afterwards by the whole
 // wave, one at a time (rg_wave_target).
 constexpr int kRgSlots = 8;
-// In-radius candidates of one target whose distance bits a wave keeps in LDS for the selection.
-constexpr int kRgSelCap = 1024;
+// Candidates of one target whose distance bits a wave keeps in LDS for the selection.
+// The waves wait for LDS and L2 more than they compute, so how many fit a CU counts, against the
+// targets with more candidates, which read the stencil twice: a lidar frame of 131,072 points at
+// radius 0.5 and K = 64 takes 278 us in all with 512 (20 KB per workgroup), 293 with 768, 315 with
+// 1024, 303 with 384 and 326 with 256.  Large K keep 1024, so that they are still staged.
+constexpr int kRgSelCap = 512;
+constexpr int kRgSelCapMax = 1024;
+constexpr int kRgSelSmallK = 256;  // up to this K the smaller number
 // Chunks of 64 stencil sources loaded together when staging (eight measured 1.5% slower at C5).
 constexpr int kRgStageLoads = 4;
 
@@ -787,15 +799,23 @@ __device__ __forceinline__ void wave_scan_runs(const RgWs& w, const int (&ra)[9]
   }
 }
 
-// One target done by the whole wave: c = its count of in-radius sources (c > 0).
+// One target done by the whole wave: c = its count of in-radius sources (c > 0; more than K is
+// known only as such).
 //  c <= K: the list L[0..c) (complete) sorted by index, 64 entries per step.
 //  c > K:  the K smallest (d, j): the in-radius sources as (distance bits, index) pairs collected
-//          in LDS in one stencil pass (c <= kRgSelCap; beyond that every step re-scans the
-//          stencil), the K-th distance d* by radix select on the bits (binary search over the
-//          stencil beyond kRgSelCap), the index threshold j*
-//          among the sources at d* when they are more than needed, the accepted sources compacted
-//          in place and sorted by index.
+//          in LDS in one stencil pass and counted by distance, the K-th (d*, j*) by that histogram
+//          and its rank within the bin, the accepted sources compacted in place and sorted by index.
+//          Where more than CAP are in radius, a second pass stages those up to the K-th's bin (split
+//          first if it is too full); where K or the ties are still more, every step re-scans the
+//          stencil.
+// What bounds it is the staging pass (about 1200 stencil sources per dense target of a lidar frame)
+// and the chain of LDS steps behind it.  The selection used to be a radix select of four passes over
+// the staged keys, and targets with more than 1024 in-radius sources a binary search of about 32
+// passes over the stencil: that frame 374 -> 278 us in all, radius 0.8 and K = 16 1717 -> 524 us; a
+// sphere of 65,536 points at about 160 sources and K = 64 249 -> 186 us, a cube of 20,000 at about
+// 2000 15.4 -> 0.85 ms.
 // The target's row offset o, and for c > K its position and stencil runs, come from the caller.
+template <int CAP>
 __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t i, int c, int64_t o,
                                float qx, float qy, float qz, const int (&ra)[9], const int (&rn)[9],
                                int64_t* __restrict__ row_out, int64_t* __restrict__ col_out,
@@ -805,45 +825,116 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
   int32_t* L = w.list + i * K;
   if (c > K) {
     const int qi = static_cast<int>(i);
-    const bool inl = c <= kRgSelCap;
-    int n = 0;
-    if (inl) {
-      // stage A: in-radius (distance bits, index) into LDS (wave compaction).  The nine runs are
-      // one index space (source t of the stencil is ra[r] + t - pre[r] in the run r holding it),
-      // so kRgStageLoads chunks of 64 sources are loaded together.
-      int pre[9];
-      pre[0] = 0;
+    // stage A: in-radius (distance bits, index) into LDS (wave compaction), counted by distance in
+    // 256 equal bins of [0, r2).  The nine runs are one index space (source t of the stencil is
+    // ra[r] + t - pre[r] in the run r holding it), so kRgStageLoads chunks of 64 sources are loaded
+    // together; few runs begin inside one such batch, and only those are compared per lane.
+    int pre[9];
+    pre[0] = 0;
 #pragma unroll
-      for (int r = 1; r < 9; ++r) pre[r] = pre[r - 1] + rn[r - 1];
-      const int tot = pre[8] + rn[8];
+    for (int r = 1; r < 9; ++r) pre[r] = pre[r - 1] + rn[r - 1];
+    const int tot = pre[8] + rn[8];
+    // bin of a distance: monotone in it; r2 beyond what the scale can express: one bin
+    const float scale = r2 > 1e-30f && r2 < 1e30f ? 256.0f / r2 : 0.0f;
+    auto bin_of = [&](float d) { return static_cast<int>(fminf(d * scale, 255.0f)); };
+    for (int q = lane; q < 256; q += kWave) hist[q] = 0;
+    wave_lds_fence();
+    // The K-th is known to lie in bin `bin`, among the candidates whose distance bits match prefix
+    // in the bits decided (all of them to begin with).
+    int bin = 255;
+    uint32_t prefix = 0u, decided = 0u;
+    auto member = [&](uint32_t v) {
+      return bin_of(__uint_as_float(v)) == bin && (v & decided) == prefix;
+    };
+    // (stages the sources up to that part and returns their number, which may exceed the LDS)
+    auto stage = [&](bool first) -> int {
+      int n = 0;
       for (int base = 0; base < tot; base += kWave * kRgStageLoads) {  // wave-uniform
+        int from = ra[0];
+        int off[kRgStageLoads];
+#pragma unroll
+        for (int r = 1; r < 9; ++r) from = base >= pre[r] ? ra[r] - pre[r] : from;
+#pragma unroll
+        for (int u = 0; u < kRgStageLoads; ++u) off[u] = from;
+#pragma unroll
+        for (int r = 1; r < 9; ++r) {
+          if (pre[r] > base && pre[r] < base + kWave * kRgStageLoads) {  // wave-uniform
+#pragma unroll
+            for (int u = 0; u < kRgStageLoads; ++u)
+              off[u] = base + u * kWave + lane >= pre[r] ? ra[r] - pre[r] : off[u];
+          }
+        }
         float4 sv[kRgStageLoads];
 #pragma unroll
         for (int u = 0; u < kRgStageLoads; ++u) {
           const int t = base + u * kWave + lane;
-          int off = ra[0];
-#pragma unroll
-          for (int r = 1; r < 9; ++r) off = t >= pre[r] ? ra[r] - pre[r] : off;
-          sv[u] = t < tot ? w.spos[off + t] : make_float4(0.f, 0.f, 0.f, 0.f);
+          sv[u] = t < tot ? w.spos[off[u] + t] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
         for (int u = 0; u < kRgStageLoads; ++u) {
           const int t = base + u * kWave + lane;
           const float d = sqdist(qx, qy, qz, sv[u].x, sv[u].y, sv[u].z);
           const int j = __float_as_int(sv[u].w);
-          const bool a = t < tot && (lp || j != qi) && d < r2;
+          const int db = bin_of(d);
+          const bool a = t < tot && (lp || j != qi) && d < r2 &&
+                         (db < bin || (db == bin && (__float_as_uint(d) & decided) <= prefix));
           const uint64_t m = __ballot(a);
           const int slot = n + static_cast<int>(__popcll(m & lanemask_lt()));
-          if (a && slot < kRgSelCap) {
-            key[slot] = __float_as_uint(d);
-            idx[slot] = j;
+          if (a) {
+            if (slot < CAP) {
+              key[slot] = __float_as_uint(d);
+              idx[slot] = j;
+            }
+            if (first) atomicAdd(&hist[db], 1);
           }
           n += static_cast<int>(__popcll(m));
         }
       }
-      n = n < kRgSelCap ? n : kRgSelCap;
       wave_lds_fence();
+      return n;
+    };
+    int n = stage(true);
+    // stage B: the K-th smallest (distance, index).  First the bin that holds it, by one wave scan
+    // of the histogram (lane l holds bins 4l .. 4l + 3).
+    int k = K;   // rank of the K-th among the candidates not yet ruled out (1 <= k <= their count)
+    int at = 0;  // the candidates in the bin; in the end the sources at d*
+    auto pick = [&]() -> int {  // the histogram bin with the k-th; k and at become its own
+      const int h0 = hist[4 * lane], h1 = hist[4 * lane + 1], h2 = hist[4 * lane + 2];
+      const int h3 = hist[4 * lane + 3];
+      const int sum = h0 + h1 + h2 + h3;
+      const int excl = static_cast<int>(wave_inclusive_sum_dpp(static_cast<uint32_t>(sum))) - sum;
+      const int L = __builtin_ctzll(__ballot(excl < k && k <= excl + sum) | (1ull << 63));
+      int d = 4 * lane, below = excl, hs = h0;
+      if (k > below + h0) {
+        d += 1; below += h0; hs = h1;
+        if (k > below + h1) {
+          d += 1; below += h1; hs = h2;
+          if (k > below + h2) { d += 1; below += h2; hs = h3; }
+        }
+      }
+      k -= __builtin_amdgcn_readlane(below, L);
+      at = __builtin_amdgcn_readlane(hs, L);
+      wave_lds_fence();  // every lane has read the histogram before it is written again
+      return __builtin_amdgcn_readlane(d, L);
+    };
+    bin = pick();
+    // More in radius than the LDS holds: the sources up to that bin are staged by a second pass; a
+    // bin too full for that is split by the distance bits, 8 per pass over the stencil, first.
+    int shift = 24;
+    while (n > CAP && K <= CAP && K - k + at > CAP && shift >= 0) {
+      for (int q = lane; q < 256; q += kWave) hist[q] = 0;
+      wave_lds_fence();
+      wave_scan_runs(w, ra, rn, qx, qy, qz, [&](float d, int j, bool ok) {
+        const uint32_t v = __float_as_uint(d);
+        if (ok && (lp || j != qi) && d < r2 && member(v)) atomicAdd(&hist[(v >> shift) & 255u], 1);
+      });
+      wave_lds_fence();
+      prefix |= static_cast<uint32_t>(pick()) << shift;
+      decided |= 0xffu << shift;
+      shift -= 8;
     }
+    const bool inl = n <= CAP || K - k + at <= CAP;
+    if (n > CAP && inl) n = stage(false);
     // in-radius sources with bits <= dmax (< when strict), or with bits == dmax and j <= jmax
     // (jmax >= 0)
     auto count_le = [&](uint32_t dmax, bool strict, int jmax) -> int {
@@ -860,44 +951,72 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
       }
       return static_cast<int>(wave_sum_dpp(static_cast<uint32_t>(t)));
     };
-    // stage B: the K-th smallest distance bits (every in-radius d has bits < bits(r2)).  Staged
-    // candidates: a radix select, 8 bits per pass -- a 256-bin LDS histogram of the keys that
-    // match the digits chosen so far, then the bin holding the K-th by one wave scan (lane l
-    // holds bins 4l .. 4l + 3).  Otherwise a binary search on the bits over the stencil.
-    uint32_t dstar;
-    int less = 0, at = 0;  // sources below d*, sources at d*
+    // Staged: where the bin holds at most 64 candidates, the K-th by its rank among them, one per
+    // lane.  A fuller bin is split by a radix select on the distance bits, 8 per pass, until few
+    // enough are left or all bits are decided.  Not staged (K or the ties at d* exceed the LDS): a
+    // binary search on the bits over the stencil.
+    uint32_t dstar = 0;
+    int less = 0;  // sources below d*
+    int jstar = 0x7fffffff;
+    bool found = false;
     if (inl) {
-      uint32_t prefix = 0u, decided = 0u;
-      int k = K;  // rank of the K-th among the keys that match prefix (1 <= k <= their count)
-      for (int shift = 24; shift >= 0; shift -= 8) {
+      for (; shift >= 0 && at > kWave; shift -= 8) {
         for (int q = lane; q < 256; q += kWave) hist[q] = 0;
         wave_lds_fence();
         for (int m = lane; m < n; m += kWave) {
           const uint32_t v = key[m];
-          if ((v & decided) == prefix) atomicAdd(&hist[(v >> shift) & 255u], 1);
+          if (member(v)) atomicAdd(&hist[(v >> shift) & 255u], 1);
         }
         wave_lds_fence();
-        const int h0 = hist[4 * lane], h1 = hist[4 * lane + 1], h2 = hist[4 * lane + 2];
-        const int h3 = hist[4 * lane + 3];
-        const int sum = h0 + h1 + h2 + h3;
-        const int excl = static_cast<int>(wave_inclusive_sum_dpp(static_cast<uint32_t>(sum))) - sum;
-        const int L = __builtin_ctzll(__ballot(excl < k && k <= excl + sum) | (1ull << 63));
-        int d = 4 * lane, below = excl, hs = h0;
-        if (k > below + h0) {
-          d += 1; below += h0; hs = h1;
-          if (k > below + h1) {
-            d += 1; below += h1; hs = h2;
-            if (k > below + h2) { d += 1; below += h2; hs = h3; }
+        prefix |= static_cast<uint32_t>(pick()) << shift;
+        decided |= 0xffu << shift;
+      }
+      found = at <= kWave;
+      if (found) {
+        // The sources below the bin (or its part) are accepted, compacted in place over the LDS
+        // indices (a slot never passes the position being read), its members go to one lane each,
+        // and the first k of these by rank complete the accepted ones.
+        int2* mem = reinterpret_cast<int2*>(hist);  // the members' distance bits and indices
+        int m0 = 0, a0 = 0;
+        for (int base = 0; base < n; base += kWave * kRgStageLoads) {  // wave-uniform trip count
+          uint32_t kv[kRgStageLoads];
+          int jv[kRgStageLoads];
+#pragma unroll
+          for (int u = 0; u < kRgStageLoads; ++u) {
+            const int m = min(base + u * kWave + lane, n - 1);
+            kv[u] = key[m];
+            jv[u] = idx[m];
+          }
+          wave_lds_fence();  // every lane has read its entries before any slot is written
+#pragma unroll
+          for (int u = 0; u < kRgStageLoads; ++u) {
+            const bool real = base + u * kWave + lane < n;
+            const int vb = bin_of(__uint_as_float(kv[u]));
+            const bool part = real && vb == bin;
+            const bool a = real && (vb < bin || (part && (kv[u] & decided) < prefix));
+            const bool in = part && (kv[u] & decided) == prefix;
+            const uint64_t ba = __ballot(a), bm = __ballot(in);
+            if (a) idx[a0 + static_cast<int>(__popcll(ba & lanemask_lt()))] = jv[u];
+            if (in) mem[m0 + static_cast<int>(__popcll(bm & lanemask_lt()))] = make_int2(static_cast<int>(kv[u]), jv[u]);
+            a0 += static_cast<int>(__popcll(ba));
+            m0 += static_cast<int>(__popcll(bm));
           }
         }
-        k -= __builtin_amdgcn_readlane(below, L);
-        at = __builtin_amdgcn_readlane(hs, L);  // after the last pass: the sources at d*
-        prefix |= static_cast<uint32_t>(__builtin_amdgcn_readlane(d, L)) << shift;
-        decided |= 0xffu << shift;
-        wave_lds_fence();  // every lane has read the histogram before the next pass clears it
+        wave_lds_fence();
+        const uint32_t v = static_cast<uint32_t>(mem[lane].x);
+        const int j = mem[lane].y;
+        int rank = 0;
+        for (int q = 0; q < m0; ++q) {  // broadcast reads
+          const int2 u = mem[q];
+          const uint32_t ub = static_cast<uint32_t>(u.x);
+          rank += (ub < v) | ((ub == v) & (u.y < j));
+        }
+        if (lane < m0 && rank < k) idx[a0 + rank] = j;  // a0 + k = K
+        wave_lds_fence();
+      } else {
+        dstar = prefix;
+        less = K - k;
       }
-      dstar = prefix;
-      less = K - k;
     } else {
       uint32_t lo = 0, hi = __float_as_uint(r2) - 1u;
       while (lo < hi) {
@@ -910,8 +1029,7 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
     }
     // stage C: index threshold among the sources at d* when they are more than needed
     const int need = K - less;
-    int jstar = 0x7fffffff;
-    if (at > need) {
+    if (!found && at > need) {
       int jlo = 0, jhi = 0x7ffffffe;
       while (jlo < jhi) {
         const int mid = jlo + ((jhi - jlo) >> 1);
@@ -920,12 +1038,12 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
       jstar = jlo;
     }
     auto accept = [&](uint32_t db, int j) { return db < dstar || (db == dstar && j <= jstar); };
-    // stage D: the K accepted sources, compacted in place over the LDS indices (a slot never
-    // passes the position being read) or into the list when K exceeds the LDS; stage E: ranked
-    // by index.  The two forms are separate so that the LDS one reads with LDS instructions.
-    if (inl && K <= kRgSelCap) {
+    // stage D: the K accepted sources, compacted in place over the LDS indices (done already where
+    // the K-th came from its bin) or into the list; stage E: ranked by index.  The two forms are
+    // separate so that the LDS one reads with LDS instructions.
+    if (inl) {
       int m0 = 0;
-      for (int base = 0; base < n; base += kWave) {  // wave-uniform trip count
+      for (int base = 0; base < n && !found; base += kWave) {  // wave-uniform trip count
         const int m = base + lane;
         const bool a = m < n && accept(key[m], idx[m]);
         const int j = m < n ? idx[m] : 0;
@@ -950,24 +1068,13 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
       }
     } else {
       int m0 = 0;
-      if (inl) {
-        for (int base = 0; base < n; base += kWave) {  // wave-uniform trip count
-          const int m = base + lane;
-          const bool a = m < n && accept(key[m], idx[m]);
-          const uint64_t bm = __ballot(a);
-          const int slot = m0 + static_cast<int>(__popcll(bm & lanemask_lt()));
-          if (a && slot < K) L[slot] = idx[m];
-          m0 += static_cast<int>(__popcll(bm));
-        }
-      } else {
-        wave_scan_runs(w, ra, rn, qx, qy, qz, [&](float d, int j, bool ok) {
-          const bool a = ok && (lp || j != qi) && d < r2 && accept(__float_as_uint(d), j);
-          const uint64_t bm = __ballot(a);
-          const int slot = m0 + static_cast<int>(__popcll(bm & lanemask_lt()));
-          if (a && slot < K) L[slot] = j;
-          m0 += static_cast<int>(__popcll(bm));
-        });
-      }
+      wave_scan_runs(w, ra, rn, qx, qy, qz, [&](float d, int j, bool ok) {
+        const bool a = ok && (lp || j != qi) && d < r2 && accept(__float_as_uint(d), j);
+        const uint64_t bm = __ballot(a);
+        const int slot = m0 + static_cast<int>(__popcll(bm & lanemask_lt()));
+        if (a && slot < K) L[slot] = j;
+        m0 += static_cast<int>(__popcll(bm));
+      });
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
       for (int m = lane; m < K; m += kWave) {
         const int v = L[m];
@@ -989,15 +1096,16 @@ __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t 
   }
 }
 
+template <int CAP>
 __global__ __launch_bounds__(kRgThreads) void rg_compact(RgWs w, const float* __restrict__ x,
                                                          int64_t N, const int64_t* __restrict__ batch,
                                                          int64_t B, int64_t ppc, float r2, int K,
                                                          int loop, const int64_t* __restrict__ row_ptr,
                                                          int64_t* __restrict__ row_out,
                                                          int64_t* __restrict__ col_out) {
-  __shared__ uint32_t s_key[kRgThreads / kWave][kRgSelCap];
-  __shared__ __align__(16) int32_t s_idx[kRgThreads / kWave][kRgSelCap];
-  __shared__ int32_t s_hist[kRgThreads / kWave][256];
+  __shared__ uint32_t s_key[kRgThreads / kWave][CAP];
+  __shared__ __align__(16) int32_t s_idx[kRgThreads / kWave][CAP];
+  __shared__ __align__(16) int32_t s_hist[kRgThreads / kWave][256];
   r2 = rg_r2(w, r2);
   const int64_t i = (xcd_block_runs(kRgXcdRun) * kRgThreads + threadIdx.x) / kRgGroup;
   const int sub = static_cast<int>(threadIdx.x) & (kRgGroup - 1);
@@ -1071,7 +1179,7 @@ __global__ __launch_bounds__(kRgThreads) void rg_compact(RgWs w, const float* __
     const float tx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pqx), leader));
     const float ty = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pqy), leader));
     const float tz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pqz), leader));
-    rg_wave_target(w, r2, K, loop != 0, ti, tc, to, tx, ty, tz, ra, rn, row_out, col_out,
+    rg_wave_target<CAP>(w, r2, K, loop != 0, ti, tc, to, tx, ty, tz, ra, rn, row_out, col_out,
                    s_key[threadIdx.x / kWave], s_idx[threadIdx.x / kWave], s_hist[threadIdx.x / kWave]);
   }
 }
@@ -1199,7 +1307,8 @@ static int radius_emit_impl(const float* x, int64_t N, const int64_t* batch, int
   const int K = static_cast<int>(max_num_neighbors);
   const int64_t blocks = ceil_div(N, kRgEmitThreads);
   if (w.list) {
-    hipLaunchKernelGGL(rg_compact, dim3(ceil_div(N * kRgGroup, kRgThreads)), dim3(kRgThreads), 0,
+    auto compact = K <= kRgSelSmallK ? rg_compact<kRgSelCap> : rg_compact<kRgSelCapMax>;
+    hipLaunchKernelGGL(compact, dim3(ceil_div(N * kRgGroup, kRgThreads)), dim3(kRgThreads), 0,
                        st, w, x, N, batch, B, points_per_cloud, r2, K, loop, row_ptr, row_out,
                        col_out);
     GEO_LAUNCH_CHECK("rg_compact");

@@ -1,0 +1,83 @@
+"""Radius graph where a target has more than K sources: the count stops early, the K-th source comes
+from one histogram bin (few members), from a bin split by its distance bits (many members at nearly or
+exactly the same distance), or from searches over the stencil (more in-radius sources than are staged).
+Edges equal the oracle's."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(x, r, K, **kw):
+    from gdl_amd.functional import radius_graph
+    dev = {k: (v.cuda() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
+    row, col = radius_graph(x.cuda(), r, max_num_neighbors=K, **dev)
+    host = {k: (v.numpy() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
+    want = oracle.radius_graph(x.numpy(), r, max_num_neighbors=K, **host)
+    np.testing.assert_array_equal(col.cpu().numpy(), want[1])
+    np.testing.assert_array_equal(row.cpu().numpy(), want[0])
+
+
+@pytest.mark.parametrize("K", [1, 7, 64, 256, 257])
+@pytest.mark.parametrize("r", [0.03, 0.08, 0.14, 0.2])  # about 1, 15, 80, 200 sources in radius
+def test_uniform_cloud(K, r):
+    g = torch.Generator().manual_seed(K)
+    _check(torch.rand(6007, 3, generator=g), r, K)
+
+
+@pytest.mark.parametrize("K", [3, 20, 32, 100])
+def test_surfaces_and_clumps(K):
+    g = torch.Generator().manual_seed(K)
+    flat = torch.rand(5003, 3, generator=g) * torch.tensor([1.0, 1.0, 0.01])
+    clump = 0.5 + 0.02 * torch.randn(900, 3, generator=g)  # stencil runs of several hundred points
+    _check(torch.cat([flat, clump]), 0.09, K, loop=bool(K % 2))
+
+
+@pytest.mark.parametrize("K", [2, 6, 18, 26, 30, 80])
+def test_lattice_ties_at_the_cap(K):
+    """Shells of equal distance: the K-th source lies inside a tie, taken by index."""
+    n = torch.arange(18.0)
+    x = torch.cartesian_prod(n, n, n)[torch.randperm(18 ** 3, generator=torch.Generator().manual_seed(K))]
+    _check(x.contiguous(), 2.5, K)
+
+
+@pytest.mark.parametrize("K", [1, 5, 40])
+def test_repeated_points(K):
+    """Every point 60 times: more than K sources at distance 0."""
+    g = torch.Generator().manual_seed(K)
+    x = torch.rand(100, 3, generator=g).repeat(60, 1)
+    _check(x[torch.randperm(6000, generator=g)].contiguous(), 0.2, K, loop=bool(K % 2))
+
+
+def test_mask_and_unsorted_batch():
+    g = torch.Generator().manual_seed(3)
+    x = torch.rand(9001, 3, generator=g)
+    batch = torch.randint(0, 2, (9001,), generator=g)
+    mask = torch.rand(9001, generator=g) > 0.2
+    _check(x, 0.15, 32, batch=batch, mask=mask, num_batch_elements=2)
+
+
+@pytest.mark.parametrize("K", [1, 3, 60, 66, 300])
+@pytest.mark.parametrize("rel", [0.0, 1e-6, 1e-4, 1e-2])
+@pytest.mark.parametrize("m", [200, 600, 1500])
+def test_shell_in_one_bin(K, rel, m):
+    """m sources within a relative distance `rel` of the same sphere around 40 close targets."""
+    g = torch.Generator().manual_seed(K)
+    shell = torch.nn.functional.normalize(torch.randn(m, 3, generator=g), dim=1)
+    shell = shell * 0.1 * (1 + rel * torch.rand(m, 1, generator=g))
+    x = torch.cat([shell, 1e-7 * torch.randn(40, 3, generator=g), torch.rand(4500, 3, generator=g) + 1])
+    _check(x[torch.randperm(x.shape[0], generator=g)].contiguous(), 0.15, K)
+
+
+@pytest.mark.parametrize("n", [512, 513, 1024, 1025, 1026, 3000])
+@pytest.mark.parametrize("K,loop", [(1, False), (64, True), (256, True), (257, True), (500, False), (1023, True), (1024, False), (1024, True), (1030, True)])
+def test_around_the_staged_number(n, K, loop):
+    """n points all within the radius of each other: 512 or (large K) 1024 of them are staged at most."""
+    g = torch.Generator().manual_seed(n)
+    x = torch.rand(n, 3, generator=g)
+    for r in (2.0, 1e19, 1e20):
+        _check(x, r, K, loop=loop)
