@@ -1210,7 +1210,8 @@ extern "C" int geo_fps_total(const float* pos, int64_t N_total, const int64_t* p
   GEO_REQUIRE(pos && ptr && out_ptr && out_idx, "fps: null pointer");
   hipStream_t st = as_stream(stream);
   const int64_t need = static_cast<int64_t>(geo_fps_workspace_bytes(B, N_total, max_cloud));
-  if (need > 0 && (workspace == nullptr || workspace_bytes < static_cast<size_t>(need)))
+  const bool room = workspace != nullptr && workspace_bytes >= static_cast<size_t>(need);
+  if (need > 0 && !room && max_cloud > kFpsRegisterPoints)
     return set_error(GEO_ERR_WORKSPACE, "fps: workspace %zu bytes, need %lld", workspace_bytes,
                      (long long)need);
   if (max_cloud <= kFpsLdsPoints) {
@@ -1225,7 +1226,9 @@ extern "C" int geo_fps_total(const float* pos, int64_t N_total, const int64_t* p
   // large kernel's sort and first rounds cost about 90 us more, its later rounds a tenth as much
   // per sample (12,000 points: 64 samples 197 against 225 us, 375 samples 1069 against 399 us,
   // 6000 samples 16.9 against 2.2 ms); they cross at 73 to 87 samples between 8,200 and 16,384.
-  if (max_cloud <= kFpsRegisterPoints && (total <= kFpsRegisterSamples * B || !fps_use_large(B, max_cloud))) {
+  // Callers that bring no workspace for such clouds get it as well.
+  if (max_cloud <= kFpsRegisterPoints &&
+      (total <= kFpsRegisterSamples * B || !room || !fps_use_large(B, max_cloud))) {
     hipLaunchKernelGGL((fps_register_kernel<kFpsRegisterPoints / kFpsThreads>), dim3(B),
                        dim3(kFpsThreads), 0, st, pos, ptr, out_ptr, out_idx);
     GEO_LAUNCH_CHECK("fps_register_kernel");

@@ -50,3 +50,16 @@ def test_fps_rounds_of_large_clouds(kind, sizes, samples):
     k = np.array([min(n, samples if kind != "same" else 40) for n in sizes])
     got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
+
+
+@pytest.mark.parametrize("n", [8193, 16384])
+def test_clouds_of_the_register_kernel_need_no_workspace(n):
+    from gdl_amd import _native as nat
+    pos = _points("cube", n, n).cuda()
+    k = 120  # above the few-samples rule
+    ptr, out_ptr = torch.tensor([0, n]).cuda(), torch.tensor([0, k]).cuda()
+    out = torch.empty(k, dtype=torch.int64, device="cuda")
+    nat.check(nat.lib().geo_fps(nat.ptr(pos), n, nat.ptr(ptr), nat.ptr(out_ptr), 1, n, nat.ptr(out),
+                                None, 0, nat.stream_of(pos.device)), "geo_fps")
+    want = oracle.fps(pos.cpu().numpy(), np.array([0, n]), np.array([k]))
+    np.testing.assert_array_equal(out.cpu().numpy(), want)

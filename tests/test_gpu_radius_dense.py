@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _check(x, r, K, **kw):
-    from gdl_amd.functional import radius_graph
+    from gdl_amd.functional.radius_graph import radius_graph
     dev = {k: (v.cuda() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
     row, col = radius_graph(x.cuda(), r, max_num_neighbors=K, **dev)
     host = {k: (v.numpy() if isinstance(v, torch.Tensor) else v) for k, v in kw.items()}
