@@ -391,7 +391,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
   //    (bits, index, lane, position) and the rest bound of slot s as scalars.
   float blx[TESTS], bly[TESTS], blz[TESTS], bhx[TESTS], bhy[TESTS], bhz[TESTS];
   uint32_t bmax[TESTS];
-  uint32_t bm[PTS], bi[PTS], al[PTS], rs[PTS];  // al: lane holding the max, kWave = unknown
+  uint32_t bm[PTS], bi[PTS], al[PTS], rs[PTS];
   float sx[PTS], sy[PTS], sz[PTS];
 #pragma unroll
   for (int h = 0; h < TESTS; ++h) {
@@ -409,14 +409,15 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const uint32_t h1 = wave_max_u32(valid ? float_order_key(py[s]) : 0u);
     const uint32_t h2 = wave_max_u32(valid ? float_order_key(pz[s]) : 0u);
     const bool any = (s * WAVES + w) * kWave < n;
-    // until the first update (all buckets take part in it): lane 0's point, nothing known
+    // every distance is +inf, so the record is the lowest index; it stands until that point falls,
+    // which it never does where squared distances overflow (no update then touches the bucket)
     bm[s] = any ? 0x7f800000u : 0u;
-    bi[s] = __builtin_amdgcn_readfirstlane(oi[s]);
-    al[s] = kWave;
+    bi[s] = wave_min_u32(oi[s]);
+    al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(oi[s] == bi[s]) | (1ull << 63)));
     rs[s] = 0x7f800000u;
-    sx[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(px[s])));
-    sy[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(py[s])));
-    sz[s] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(pz[s])));
+    sx[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
+    sy[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
+    sz[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
     if (lane / 16 == s % 4 && any) {
       blx[s / 4] = float_from_order_key(l0); bly[s / 4] = float_from_order_key(l1);
       blz[s / 4] = float_from_order_key(l2); bhx[s / 4] = float_from_order_key(h0);
@@ -495,8 +496,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
         md[s] = mb;
         // Values only fall: while the point holding the bucket's max keeps its value, the record
         // (max, lowest index attaining it) stands, and its rest bound still holds.
-        if (al[s] < static_cast<uint32_t>(kWave) && !((__ballot(mb < old) >> al[s]) & 1ull))
-          continue;
+        if (!((__ballot(mb < old) >> al[s]) & 1ull)) continue;
         const uint32_t mx = wave_max_u32(mb);
         const uint64_t hit = __ballot(mb == mx);
         if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
@@ -705,9 +705,10 @@ __global__ void fps_large_keys_kernel(const float* __restrict__ pos, const int64
   keys[i] = (static_cast<uint32_t>(lo) << (3 * mbits)) | code;
 }
 
-// Bucket j of cloud b (64 sorted points, one wave): positions and original index bits in sorted
-// order, min distances +inf, and the bucket's box at boxes[a][fps_large_box0 + j] (lo x, y, z,
-// hi x, y, z by a).
+// Bucket j of cloud b (64 sorted points, one wave): positions and original index bits, min distances
+// +inf, and the bucket's box at boxes[a][fps_large_box0 + j] (lo x, y, z, hi x, y, z by a).  The
+// points lie in sorted order, except that the one with the lowest index changes places with the
+// first: it is the bucket's record while all distances are +inf.
 __device__ __forceinline__ int64_t fps_large_box0(int64_t start, int b) { return (start >> 6) + b; }
 
 __global__ __launch_bounds__(256) void fps_large_gather_kernel(
@@ -723,8 +724,9 @@ __global__ __launch_bounds__(256) void fps_large_gather_kernel(
   const uint32_t i = order[at];
   const float x = pos[3 * static_cast<int64_t>(i)], y = pos[3 * static_cast<int64_t>(i) + 1],
               z = pos[3 * static_cast<int64_t>(i) + 2];
+  const int low = __builtin_ctzll(__ballot(i == wave_min_u32(i)) | (1ull << 63));
   if (l < n) {
-    q[at] = make_float4(x, y, z, __uint_as_float(i));
+    q[lane == low ? at - lane : (lane == 0 ? at + low : at)] = make_float4(x, y, z, __uint_as_float(i));
     md[at] = 0x7f800000u;
   }
   const uint32_t kx = float_order_key(x), ky = float_order_key(y), kz = float_order_key(z);
@@ -809,9 +811,9 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
     const float h2 = float_from_order_key(wave_max_u32(float_order_key(bhz[r])));
     if (row == r && kWave * (w + W * r) < nb) {
       slx = l0; sly = l1; slz = l2; shx = h0; shy = h1; shz = h2;
-      smax = 0x7f800000u;  // +inf: every bucket takes part in the first update
+      smax = 0x7f800000u;
     }
-    if (in) {  // until then: the bucket's first point, nothing known
+    if (in) {  // all distances +inf: the bucket's lowest index (its first point), nothing known
       const float4 p = Q[bk * kWave];
       rec[bk] = make_float4(p.x, p.y, p.z, __builtin_inff());
       rkey[bk] = fps_key(0x7f800000u, __float_as_uint(p.w) - ustart);
@@ -948,7 +950,7 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
         // Values only fall: while the point holding the bucket's max keeps its value, the record
         // (max, lowest index attaining it) stands, and its rest bound still holds.
         const uint32_t nidx = ~(__float_as_uint(pt.w) - ustart);
-        if (done != 1 && (__ballot(mb < old) & __ballot(nidx == holder)) == 0ull) continue;
+        if ((__ballot(mb < old) & __ballot(nidx == holder)) == 0ull) continue;
         const uint32_t mx = wave_max_u32(mb);
         const uint64_t hit = __ballot(mb == mx && q < n);
         int sl;

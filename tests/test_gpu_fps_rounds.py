@@ -52,6 +52,32 @@ def test_fps_rounds_of_large_clouds(kind, sizes, samples):
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
 
 
+@pytest.mark.parametrize("kind", ["far groups", "all far", "inf", "nan"])
+@pytest.mark.parametrize("sizes, samples", [
+    ([64, 130, 700], 50), ([4096, 300], 200), ([8192], 300),
+    ([9000], 60), ([9000], 300),  # register kernel, large kernel
+    ([20000, 500], 300), ([70000], 200),
+])
+def test_distances_that_overflow_or_are_not_finite(kind, sizes, samples):
+    """A bucket that no centroid can reach with a finite distance keeps all its points at +inf: the
+    lowest of their indices is the next sample, wherever the bucket's order puts it."""
+    from gdl_amd.csrc import fps_cuda
+    n = sum(sizes)
+    g = torch.Generator().manual_seed(n)
+    pos = torch.rand(n, 3, generator=g)
+    if kind == "far groups":  # squares overflow between the groups, not inside them
+        pos = 1e18 * pos + 1e20 * torch.randint(0, 3, (n, 1), generator=g).float()
+    elif kind == "all far":
+        pos = 1e30 * pos
+    else:
+        at = torch.rand(n, generator=g) < 0.02
+        pos[at, 1] = float(kind) * (torch.randint(0, 2, (int(at.sum()),), generator=g) * 2 - 1)
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    k = np.array([min(m - 1, samples) for m in sizes])
+    got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
+    np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
+
+
 @pytest.mark.parametrize("n", [8193, 16384])
 def test_clouds_of_the_register_kernel_need_no_workspace(n):
     from gdl_amd import _native as nat
