@@ -172,17 +172,30 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
 // (LDS counting sort), so the 64 points a wave holds in one register slot -- a bucket -- lie
 // close together.  Each bucket has its bounding box and a record of its farthest point: max min
 // distance, lowest index attaining it, position, and the rest bound: the most that any other point
-// of the bucket has left once that point is a centroid, max over p of min(md(p), d(p, farthest)).
+// of the bucket has left once that point is a centroid, max over p of min(md(p), d(p, farthest)),
+// with the lowest index attaining that.
 //
-// The loop takes several centroids per round.  Order all records by (distance, lower index), and
-// let i be ahead of j.  Record j is the greedy choice right after the records ahead of it if
+// The loop takes several centroids per round.  Order all records, and the rest bounds with them, by
+// (distance, lower index), and let i be ahead of j.  Record j is the greedy choice right after the
+// records ahead of it if
 //   d(point i, point j) >= md(point j) for every i ahead (none of them lowers its point), and
-//   rest bound of i < md(point j) for every i ahead (no other point of their buckets reaches it):
-// every other point lies below its own bucket's record and values only fall, so nothing can come
+//   rest bound of i comes after record j for every i ahead (no other point of their buckets, at the
+//   value it can still have, comes first):
+// every other point comes after its own bucket's record and values only fall, so nothing can come
 // between.  The round takes the records from the front up to the first that fails (the first one
 // never does).  Rounds therefore give exactly the one-at-a-time sequence; on 16 surface clouds of
 // 4096 points a round takes 7.6 centroids (at most 16), 135 rounds for 1024 samples, 1.6 us each,
-// where one centroid took 0.46 us: 470 -> 238 us.  A round costs two LDS barriers:
+// where one centroid took 0.46 us: 470 -> 239 us.
+// Equal distances (points on a lattice or in voxels): the rest bound's index is what keeps rounds
+// long there.  With its distance alone, another point of a bucket at the record's distance ended
+// the round, and rounds of one or two centroids cost more than one centroid at a time did.  16^3
+// lattice to 1024 samples, one at a time -> distance alone -> now: in order 524 -> 820 -> 459 us,
+// shuffled 525 -> 853 -> 268 us.  The index is looked for only where several points hold a
+// bucket's max (elsewhere 0, before all others, which ends a round at an equal distance in another
+// bucket: 3% more rounds on lattices).  It costs other clouds 1.6% (4096 points) to 4% (1024).
+// Where the first record's distance is 0 every point lies on a sample, and the lowest index is the
+// choice for all that is left: no further rounds (one point 4096 times: 855 -> 28 us a call).
+// A round costs two LDS barriers:
 //   check   every wave tests the listed records pairwise, lane = 16 * (j mod 4) + i
 //   update  the wave's buckets against the round's centroids (bound test below), records of the
 //           buckets whose farthest point fell; the wave with the most of them sets the pace
@@ -327,6 +340,9 @@ __device__ void fps_hilbert_order(const float* __restrict__ P, int n, int* hist,
 __device__ __forceinline__ double fps_key(uint32_t bits, uint32_t idx) {
   return __hiloint2double(static_cast<int>(bits), static_cast<int>(~idx));
 }
+__device__ __forceinline__ uint32_t fps_key_index(double key) {
+  return ~static_cast<uint32_t>(__double2loint(key));
+}
 
 template <int PTS, int THREADS>
 __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
@@ -340,9 +356,9 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
   // Launched before the host has seen the prepare kernel's summary: do nothing unless ptr was
   // valid and every cloud fits this variant (the host then launches the right one).
   if (guard != nullptr && (guard[2] != 0 || guard[1] > PTS * THREADS)) return;
-  __shared__ double rkey[NB];         // key of each bucket's farthest point, see fps_key
-  __shared__ float4 list[kFpsRound];  // the first records: position and (bits) rest bound
-  __shared__ uint2 lkey[kFpsRound];   // their min distance (bits) and index
+  __shared__ double rkey[NB < kWave ? kWave : NB];  // key of each bucket's farthest point, see fps_key
+  __shared__ float4 list[kFpsRound];   // the first records: position, (bits) min distance
+  __shared__ double2 lkey[kFpsRound];  // their keys and rest bounds
   __shared__ int hist[kCells];
   __shared__ uint32_t red[6][WAVES];
   extern __shared__ int2 scratch[];  // sort scratch, 12 B per point
@@ -392,6 +408,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
   float blx[TESTS], bly[TESTS], blz[TESTS], bhx[TESTS], bhy[TESTS], bhz[TESTS];
   uint32_t bmax[TESTS];
   uint32_t bm[PTS], bi[PTS], al[PTS], rs[PTS];
+  uint32_t ri[PTS];  // lowest index at the rest bound, 0 = not known
   float sx[PTS], sy[PTS], sz[PTS];
 #pragma unroll
   for (int h = 0; h < TESTS; ++h) {
@@ -415,6 +432,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     bi[s] = wave_min_u32(oi[s]);
     al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(oi[s] == bi[s]) | (1ull << 63)));
     rs[s] = 0x7f800000u;
+    ri[s] = 0u;
     sx[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
     sy[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
     sz[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
@@ -426,20 +444,22 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     }
     if (lane == 0) rkey[s * WAVES + w] = fps_key(bm[s], bi[s]);
   }
+  if (NB < kWave && t >= NB && t < kWave) rkey[t] = 0.0;  // no key is below 0
   if (t == 0) {
-    list[0] = make_float4(P[0], P[1], P[2], 0.f);
-    lkey[0] = make_uint2(0u, 0u);
+    list[0] = make_float4(P[0], P[1], P[2], __builtin_inff());
+    lkey[0] = make_double2(fps_key(0u, 0u), 0.0);
   }
   lds_barrier();
 
   // records that exist: no more can be taken in one round
   const int cap = min(kFpsRound, (n + kWave - 1) / kWave);
   const int li = lane & (kFpsRound - 1);
-  int done = 0;
+  int done = 0, kend = k;
   for (;;) {
     // which of the listed records are the next centroids: record j is one if no record i ahead of
-    // it can lower its point, and no other point of a bucket ahead can reach it
+    // it can lower its point, and no other point of a bucket ahead can come before it
     const float4 c = list[li];
+    const double rb = lkey[li].y;
     int A = 1;
     if (done != 0) {
       A = kFpsRound;
@@ -447,22 +467,22 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
       for (int g = 0; g < kFpsRound; g += 8) {  // four records per step, lane = 16 * record + i
         const int j0 = g + lane / 16, j1 = j0 + 4;
         const float4 p0 = list[j0], p1 = list[j1];
-        const uint32_t k0 = lkey[j0].x, k1 = lkey[j1].x;
         const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
         const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
-        const uint32_t rb = __float_as_uint(c.w);
-        const uint64_t b0 = (__ballot(d0 < k0) | __ballot(rb >= k0)) & __ballot(li < j0);
-        const uint64_t b1 = (__ballot(d1 < k1) | __ballot(rb >= k1)) & __ballot(li < j1);
+        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & __ballot(li < j0);
+        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & __ballot(li < j1);
         if (b0 | b1) {
           A = g + (b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16;
           break;
         }
       }
-      A = min(min(A, cap), k - done);
+      A = min(min(A, cap), kend - done);
+      // every point lies on a sample (through kend: another exit from the loop costs 2%)
+      if (A == 1 && __builtin_amdgcn_readfirstlane(__float_as_int(c.w)) == 0) kend = A = 0;
     }
-    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + lkey[li].y;
+    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + fps_key_index(lkey[li].x);
     done += A;
-    if (done >= k) break;
+    if (done >= kend) break;
 
     // update: the wave's buckets against the round's centroids
 #pragma unroll
@@ -475,7 +495,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
         gz = fmaxf(fmaxf(blz[h] - c.z, c.z - bhz[h]), 0.f);
       }
       const float lb = sqdist(gx, gy, gz, 0.f, 0.f, 0.f);
-      const uint64_t act = __ballot(li < A && __float_as_uint(lb) < bmax[h]);
+      const uint64_t act = __ballot(__float_as_uint(lb) < bmax[h]) & __ballot(li < A);
       if (!act) continue;
 #pragma unroll
       for (int s = 4 * h; s < PTS && s < 4 * h + 4; ++s) {
@@ -499,12 +519,19 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
         if (!((__ballot(mb < old) >> al[s]) & 1ull)) continue;
         const uint32_t mx = wave_max_u32(mb);
         const uint64_t hit = __ballot(mb == mx);
+        ri[s] = 0u;
         if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
           al[s] = static_cast<uint32_t>(__builtin_ctzll(hit));
           bi[s] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(oi[s]), al[s]));
         } else {
           bi[s] = wave_min_u32(mb == mx ? oi[s] : 0xffffffffu);
           al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(mb == mx && oi[s] == bi[s]) | (1ull << 63)));
+          // the others at the maximum that stay there
+          const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
+          const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
+          const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
+          const bool stay = mb == mx && __float_as_uint(sqdist(px[s], py[s], pz[s], x, y, z)) >= mx;
+          if (__ballot(stay)) ri[s] = wave_min_u32(stay ? oi[s] : 0xffffffffu);
         }
         bm[s] = mx;
         if (lane / 16 == s % 4) bmax[h] = mx;
@@ -524,9 +551,7 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     double kk[SETS];
 #pragma unroll
     for (int e = 0; e < SETS; ++e) {
-      const int i = e * kWave + lane;
-      kk[e] = rkey[i < NB ? i : 0];
-      if (NB < kWave && i >= NB) kk[e] = 0.0;  // no key is below 0
+      kk[e] = rkey[e * kWave + lane];
     }
 #pragma unroll
     for (int s = 0; s < PTS; ++s) {
@@ -535,12 +560,13 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
 #pragma unroll
       for (int e = 0; e < SETS; ++e) rank += __builtin_popcountll(__ballot(kk[e] > kj));
       if (rank < kFpsRound && (s * WAVES + w) * kWave < n && lane == 0) {
-        list[rank] = make_float4(sx[s], sy[s], sz[s], __uint_as_float(rs[s]));
-        lkey[rank] = make_uint2(bm[s], bi[s]);
+        list[rank] = make_float4(sx[s], sy[s], sz[s], __uint_as_float(bm[s]));
+        lkey[rank] = make_double2(kj, fps_key(rs[s], ri[s]));
       }
     }
     lds_barrier();
   }
+  for (int i = done + t; i < k; i += THREADS) out_idx[o0 + i] = start;  // distances all 0
 }
 
 template <int PTS, int THREADS>
@@ -626,8 +652,10 @@ __global__ __launch_bounds__(kFpsStreamThreads) void fps_stream_kernel(
 //           farthest point fell are re-reduced and their groups marked
 //   groups  buckets g, g + 128, ... form group g, so neighbouring buckets lie in different groups;
 //           best and second record of the marked groups, one 16-lane row each
-//   rank    no record other than a group's best exceeds the largest second record t0, so the bests
-//           above t0, in order, are the next records of the whole cloud: the list
+//   rank    no record other than a group's best comes before the first second record t0, so the bests
+//           before t0, in order, are the next records of the whole cloud: the list
+// A 32^3 lattice to 4096 samples, one at a time -> rounds by distance alone -> now: in order 5.55 ->
+// 7.79 -> 3.15 ms, shuffled 5.51 -> 7.76 -> 1.91 ms.
 // A 131,072-point lidar frame to 16,384 samples: 1,634 rounds of 10.0 centroids and 5.5 us,
 // 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,200 cycles issues 455
 // vector instructions per wave (59% of what the CU's four SIMDs can issue in that time), 290 of
@@ -742,7 +770,7 @@ __global__ __launch_bounds__(256) void fps_large_gather_kernel(
 // Bytes of dynamic LDS for clouds of up to nb buckets.
 constexpr int kFpsLargeGroups = 128;
 __host__ __device__ inline size_t fps_large_lds(int nb) {
-  return static_cast<size_t>(nb) * (sizeof(float4) + sizeof(double) + sizeof(uint32_t) + sizeof(uint16_t)) +
+  return static_cast<size_t>(nb) * (sizeof(float4) + sizeof(double) + 2 * sizeof(uint32_t) + sizeof(uint16_t)) +
          kFpsLargeGroups * sizeof(uint16_t) + 16;
 }
 
@@ -757,12 +785,14 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
   extern __shared__ float4 large_lds[];
   float4* rec = large_lds;                                       // farthest point, (bits) rest bound
   double* rkey = reinterpret_cast<double*>(rec + nb_max);        // its key, see fps_key
-  uint32_t* queue = reinterpret_cast<uint32_t*>(rkey + nb_max);  // bucket << 16 | centroids
+  uint32_t* rlow = reinterpret_cast<uint32_t*>(rkey + nb_max);   // lowest index at the rest bound, 0 = not known
+  uint32_t* queue = rlow + nb_max;                               // bucket << 16 | centroids
   uint16_t* dirty = reinterpret_cast<uint16_t*>(queue + nb_max); // groups whose records changed
   __shared__ double gkey[G];         // best record of each group (buckets g, g + G, ...)
-  __shared__ uint32_t gbkt[G], gsec[G];  // its bucket; distance bits of the group's second record
-  __shared__ float4 list[kFpsRound];
-  __shared__ uint2 lkey[kFpsRound];
+  __shared__ uint32_t gbkt[G];       // its bucket
+  __shared__ uint32_t gsec[G], glow[G];  // the group's second record: distance bits, complement of the index
+  __shared__ float4 list[kFpsRound];   // as in the bucketed kernel
+  __shared__ double2 lkey[kFpsRound];
   __shared__ int n_queue, n_dirty;
 
   const int b = blockIdx.x;
@@ -816,44 +846,45 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
     if (in) {  // all distances +inf: the bucket's lowest index (its first point), nothing known
       const float4 p = Q[bk * kWave];
       rec[bk] = make_float4(p.x, p.y, p.z, __builtin_inff());
+      rlow[bk] = 0u;
       rkey[bk] = fps_key(0x7f800000u, __float_as_uint(p.w) - ustart);
     }
   }
   if (t < G) dirty[t] = static_cast<uint16_t>(t);  // every group is formed in the first round
   if (t == 0) {
-    list[0] = make_float4(pos[3 * start], pos[3 * start + 1], pos[3 * start + 2], 0.f);
-    lkey[0] = make_uint2(0u, 0u);
+    list[0] = make_float4(pos[3 * start], pos[3 * start + 1], pos[3 * start + 2], __builtin_inff());
+    lkey[0] = make_double2(fps_key(0u, 0u), 0.0);
     n_queue = 0;
     n_dirty = G;
   }
   __syncthreads();
 
-  int done = 0, cap = 1;
+  int done = 0, cap = 1, kend = k;
   for (;;) {
     // check: as in the bucketed kernel, over the listed records
     const float4 c = list[li];
+    const double rb = lkey[li].y;
     int A = cap;
     if (cap > 1) {
 #pragma unroll
       for (int g = 0; g < kFpsRound; g += 8) {  // four records per step, lane = 16 * record + i
         const int j0 = g + row, j1 = j0 + 4;
         const float4 p0 = list[j0], p1 = list[j1];
-        const uint32_t k0 = lkey[j0].x, k1 = lkey[j1].x;
         const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
         const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
-        const uint32_t rb = __float_as_uint(c.w);
-        const uint64_t b0 = (__ballot(d0 < k0) | __ballot(rb >= k0)) & __ballot(li < j0);
-        const uint64_t b1 = (__ballot(d1 < k1) | __ballot(rb >= k1)) & __ballot(li < j1);
+        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & __ballot(li < j0);
+        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & __ballot(li < j1);
         if (b0 | b1) {
           A = min(A, g + static_cast<int>(b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16);
           break;
         }
       }
     }
-    A = min(A, k - done);
-    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + lkey[li].y;
+    A = min(A, kend - done);
+    if (A == 1 && __builtin_amdgcn_readfirstlane(__float_as_int(c.w)) == 0) kend = A = 0;
+    if (w == 0 && lane < A) out_idx[o0 + done + lane] = start + fps_key_index(lkey[li].x);
     done += A;
-    if (done >= k) break;
+    if (done >= kend) break;
 
     // test: slots against centroids, lane = 16 * slot + centroid, then the buckets of the slots that
     // a centroid may reach
@@ -954,13 +985,19 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
         const uint32_t mx = wave_max_u32(mb);
         const uint64_t hit = __ballot(mb == mx && q < n);
         int sl;
-        uint32_t ni;
+        uint32_t ni, nlow = 0u;
         if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
           sl = __builtin_ctzll(hit | (1ull << 63));
           ni = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(nidx), sl));
         } else {
           ni = wave_max_u32(mb == mx && q < n ? nidx : 0u);
           sl = __builtin_ctzll(__ballot(mb == mx && q < n && nidx == ni) | (1ull << 63));
+          // the others at the maximum that stay there
+          const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.x), sl));
+          const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.y), sl));
+          const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.z), sl));
+          const bool stay = mb == mx && q < n && __float_as_uint(sqdist(pt.x, pt.y, pt.z, x, y, z)) >= mx;
+          if (__ballot(stay)) nlow = ~wave_max_u32(stay ? nidx : 0u);
         }
         const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.x), sl));
         const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pt.y), sl));
@@ -969,6 +1006,7 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
             wave_max_u32(min(mb, __float_as_uint(sqdist(pt.x, pt.y, pt.z, x, y, z))));
         if (lane == 0) {
           rec[bk] = make_float4(x, y, z, __uint_as_float(rest));
+          rlow[bk] = nlow;
           rkey[bk] = fps_key(mx, ~ni);
           dirty[atomicAdd(&n_dirty, 1)] = static_cast<uint16_t>(bk % G);
         }
@@ -999,11 +1037,15 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
         const uint32_t lo = hi == top ? static_cast<uint32_t>(__double2loint(best)) : 0u;
         const uint32_t low = row_max_u32(lo);
         const bool winner = hi == top && lo == low;  // one lane, or lanes without a record
-        const uint32_t sec = row_max_u32(winner ? static_cast<uint32_t>(__double2hiint(other)) : hi);
+        const double left = winner ? other : best;
+        const uint32_t lhi = static_cast<uint32_t>(__double2hiint(left));
+        const uint32_t sec = row_max_u32(lhi);
+        const uint32_t slo = row_max_u32(lhi == sec ? static_cast<uint32_t>(__double2loint(left)) : 0u);
         if (winner) {
           gkey[g] = best;
           gbkt[g] = bk;
           gsec[g] = sec;
+          glow[g] = slo;
         }
       }
     }
@@ -1017,14 +1059,12 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
       if (t == 0) n_dirty = 0;
       uint64_t ca = __ballot(static_cast<uint32_t>(__double2hiint(ka)) > t0);
       uint64_t cb = __ballot(static_cast<uint32_t>(__double2hiint(kb)) > t0);
-      if (!(ca | cb)) {  // ties across groups: the very best record alone
-        const double m = fmax(ka, kb);
-        const uint32_t hi = wave_max_u32(static_cast<uint32_t>(__double2hiint(m)));
-        const uint32_t lo = wave_max_u32(
-            static_cast<uint32_t>(__double2hiint(m)) == hi ? static_cast<uint32_t>(__double2loint(m)) : 0u);
-        const double top = __hiloint2double(static_cast<int>(hi), static_cast<int>(lo));
-        ca = __ballot(ka == top);
-        cb = __ballot(kb == top);
+      if (!(ca | cb)) {  // equal distances across groups: by the indices too
+        const uint32_t lo = wave_max_u32(max(gsec[lane] == t0 ? glow[lane] : 0u,
+                                             gsec[kWave + lane] == t0 ? glow[kWave + lane] : 0u));
+        const double t1 = __hiloint2double(static_cast<int>(t0), static_cast<int>(lo));
+        ca = __ballot(ka > t1);
+        cb = __ballot(kb > t1);
       }
       const int na = __builtin_popcountll(ca), nc = na + __builtin_popcountll(cb);
       const uint64_t lt = lanemask_lt();
@@ -1036,14 +1076,17 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
         const double dj = __longlong_as_double(static_cast<long long>(kj));
         const int rank = __builtin_popcountll(__ballot(ka > dj)) + __builtin_popcountll(__ballot(kb > dj));
         if (rank < kFpsRound && lane == 0) {
-          list[rank] = rec[gbkt[l + (at < na ? 0 : kWave)]];
-          lkey[rank] = make_uint2(static_cast<uint32_t>(kj >> 32), ~static_cast<uint32_t>(kj));
+          const uint32_t bk = gbkt[l + (at < na ? 0 : kWave)];
+          const float4 r = rec[bk];
+          list[rank] = make_float4(r.x, r.y, r.z, __uint_as_float(static_cast<uint32_t>(kj >> 32)));
+          lkey[rank] = make_double2(dj, fps_key(__float_as_uint(r.w), rlow[bk]));
         }
       }
       cap = min(max(nc, 1), kFpsRound);
     }
     lds_barrier();
   }
+  for (int i = done + t; i < k; i += kFpsLargeThreads) out_idx[o0 + i] = start;  // distances all 0
 }
 
 struct FpsLargeWs {

@@ -19,12 +19,17 @@ def _points(kind: str, n: int, seed: int) -> torch.Tensor:
         return c[torch.randint(0, 7, (n,), generator=g)] + 0.01 * torch.randn(n, 3, generator=g)
     if kind == "lattice":  # equal distances and repeated points everywhere
         return torch.randint(0, 7, (n, 3), generator=g).float()
+    if kind == "grid":  # equal distances in index order, no repeated points
+        m = round(n ** (1 / 3)) + 1
+        return torch.cartesian_prod(*[torch.arange(float(m))] * 3)[:n].contiguous()
+    if kind == "voxel":  # a surface on a grid: ties, and more samples than distinct points
+        return (torch.nn.functional.normalize(torch.randn(n, 3, generator=g), dim=1) * 16).floor()
     if kind == "line":  # boxes without volume, equal gaps
         return torch.stack([torch.randperm(n, generator=g).float(), torch.zeros(n), torch.ones(n)], 1)
     return torch.full((n, 3), 0.25)  # one point n times: every distance 0
 
 
-@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "line", "same"])
+@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "grid", "voxel", "line", "same"])
 @pytest.mark.parametrize("sizes", [[2, 63, 64, 65], [1023, 1024, 1025], [2048, 2049], [4096, 1, 130], [8192]])
 def test_fps_rounds_follow_the_greedy_order(kind, sizes):
     from gdl_amd.csrc import fps_cuda
@@ -35,7 +40,7 @@ def test_fps_rounds_follow_the_greedy_order(kind, sizes):
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
 
 
-@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "line", "same"])
+@pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "grid", "voxel", "line", "same"])
 @pytest.mark.parametrize("sizes, samples", [
     ([8193, 3], 90),            # smallest cloud of the large kernel, above the few-samples rule
     ([16384, 40], 60),          # few samples per cloud: register kernel
@@ -47,7 +52,7 @@ def test_fps_rounds_of_large_clouds(kind, sizes, samples):
     from gdl_amd.csrc import fps_cuda
     pos = _points(kind, sum(sizes), len(sizes))
     ptr = np.concatenate([[0], np.cumsum(sizes)])
-    k = np.array([min(n, samples if kind != "same" else 40) for n in sizes])
+    k = np.array([min(n, samples) for n in sizes])
     got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
 
