@@ -9,7 +9,8 @@
 //     cloud, points ordered along a Hilbert cell grid so that each register slot of a wave holds
 //     a compact bucket of 64 points; a bucket is only updated when a new centroid can lower
 //     one of its distances (an exact test, see below), and several centroids are taken from the
-//     cached per-bucket maxima per round, where they provably follow each other.
+//     cached per-bucket maxima per round, where they provably follow each other.  A cloud of up
+//     to 384 points is sampled by one wave of that workgroup.
 //   register (8193 to 16384 points, few samples): thread t owns local points t, t+256, ... with x,
 //     y, z and the running min distance in VGPRs; every point is updated every iteration.
 //   large (8193 to 196,608 points): the bucket scheme with points sorted along the Hilbert curve
@@ -344,6 +345,55 @@ __device__ __forceinline__ uint32_t fps_key_index(double key) {
   return ~static_cast<uint32_t>(__double2loint(key));
 }
 
+// Clouds of up to kFpsWavePoints points: one wave, point s * 64 + lane in slot s of the lane, one
+// centroid per step and no barrier.  They have too few buckets for rounds (up to 64 points are one,
+// which gives one centroid per round).  What bounds a step is its chain of instructions, which grows
+// with the slots; a round's is its two barriers.  Batches of 64 clouds, kernel times one at a time
+// with a barrier -> rounds -> one wave: 64 points to 32 samples 18.2 -> 29.1 -> 6.2 us, 128 to 64 29.3
+// -> 37.4 -> 12.5, 256 to 128 51.0 -> 47.6 -> 32.7, 384 to 192 74 -> 66 -> 60, to 380 139 -> 116 -> 118.
+// With eight slots 512 points to 256 take 96 us against 75 of the rounds, 1024 with sixteen 165 / 77.
+constexpr int kFpsWavePoints = 384;
+template <int S>
+__device__ __forceinline__ void fps_one_wave(const float* __restrict__ P, int n, int k, int64_t start,
+                                             int64_t* __restrict__ out) {
+  const int lane = lane_id();
+  float px[S], py[S], pz[S];
+  uint32_t md[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int i = s * kWave + lane, at = i < n ? i : 0;
+    px[s] = P[3 * at]; py[s] = P[3 * at + 1]; pz[s] = P[3 * at + 2];
+    md[s] = i < n ? 0x7f800000u : 0u;  // padding never comes before point 0
+  }
+  int l = 0, idx = 0;
+  float cx = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(px[0])));
+  float cy = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(py[0])));
+  float cz = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(pz[0])));
+  for (int it = 0;; ++it) {
+    if (lane == 0) out[it] = start + idx;
+    if (it + 1 >= k) break;
+    uint32_t m = 0u;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      md[s] = min(md[s], __float_as_uint(sqdist(px[s], py[s], pz[s], cx, cy, cz)));
+      m = max(m, md[s]);
+    }
+    m = wave_max_u32(m);
+    // the first slot that holds the maximum, its first lane: the lowest index
+#pragma unroll
+    for (int s = S - 1; s >= 0; --s) {
+      const uint64_t hit = __ballot(md[s] == m);
+      if (hit) {  // wave-uniform
+        l = __builtin_ctzll(hit);
+        idx = s * kWave + l;
+        cx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), l));
+        cy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), l));
+        cz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), l));
+      }
+    }
+  }
+}
+
 template <int PTS, int THREADS>
 __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const float* __restrict__ pos, const int64_t* __restrict__ ptr,
@@ -377,6 +427,14 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     return;
   }
   const float* P = pos + start * 3;
+  if (n <= kFpsWavePoints) {
+    if (w != 0) return;
+    if (n <= kWave) fps_one_wave<1>(P, n, k, start, out_idx + o0);
+    else if (n <= 2 * kWave) fps_one_wave<2>(P, n, k, start, out_idx + o0);
+    else if (n <= 4 * kWave) fps_one_wave<4>(P, n, k, start, out_idx + o0);
+    else fps_one_wave<6>(P, n, k, start, out_idx + o0);
+    return;
+  }
 
   // 1-2. the cloud ordered along the Hilbert curve of its cell grid
   int2* code_rank = scratch;

@@ -30,7 +30,7 @@ def _points(kind: str, n: int, seed: int) -> torch.Tensor:
 
 
 @pytest.mark.parametrize("kind", ["cube", "clumps", "lattice", "grid", "voxel", "line", "same"])
-@pytest.mark.parametrize("sizes", [[2, 63, 64, 65], [1023, 1024, 1025], [2048, 2049], [4096, 1, 130], [8192]])
+@pytest.mark.parametrize("sizes", [[2, 63, 64, 65], [128, 129, 255, 256, 257, 383, 384, 385], [1023, 1024, 1025], [2048, 2049], [4096, 1, 130], [8192]])
 def test_fps_rounds_follow_the_greedy_order(kind, sizes):
     from gdl_amd.csrc import fps_cuda
     pos = _points(kind, sum(sizes), sum(sizes))
