@@ -35,6 +35,9 @@ _SIGNATURES = {
     "geo_fps_guarded": (c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "geo_fps_workspace_bytes": (c_size, [c_i64, c_i64, c_i64]),
     "geo_fps": (c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_size, c_vp]),
+    "geo_fps_prepare_most": (c_int, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp]),
+    "geo_fps_most": (c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_size,
+                             c_vp]),
     "geo_fps_total": (c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_size,
                               c_vp]),
     "geo_knn_workspace_bytes": (c_size, [c_i64, c_i64, c_i64, c_i64]),

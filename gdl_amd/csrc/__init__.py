@@ -777,7 +777,7 @@ def fps_cuda(pos: Tensor, ptr: Tensor, k_per_batch: Tensor) -> Tensor:
         raise ValueError("fps: ptr must have at least one entry")
     if kk.numel() != B:
         raise ValueError(f"fps: k_per_batch has {kk.numel()} entries for {B} clouds")
-    return _fps_run(pos, p, B, lambda L, out_ptr, info, s: L.geo_fps_prepare(
+    return _fps_run(pos, p, B, lambda L, out_ptr, info, s: L.geo_fps_prepare_most(
         _nat.ptr(p), _nat.ptr(kk), B, pos.shape[0], _nat.ptr(out_ptr), _nat.ptr(info), s))
 
 
@@ -828,22 +828,22 @@ def fps_uniform_hip(pos: Tensor, ptr: Tensor, num_samples: int) -> Tensor:
             return out
         ws_bytes = L.geo_fps_workspace_bytes(B, N, max_n)
         ws = _nat.workspace(ws_bytes, dev)
-        _nat.check(L.geo_fps_total(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, total,
-                                   _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
+        _nat.check(L.geo_fps_most(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, min(k, max_n),
+                                  _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
     return out
 
 
 def _fps_run(pos: Tensor, p: Tensor, B: int, prepare) -> Tensor:
-    """prepare (offsets, total, largest cloud, validity) -> one host sync -> geo_fps_total."""
+    """prepare (offsets, total, largest cloud, validity) -> one host sync -> geo_fps_most."""
     dev = pos.device
     N = pos.shape[0]
     L = _nat.lib()
     with _nat.on_device(dev):
         s = _nat.stream_of(dev)
         out_ptr = torch.empty(B + 1, dtype=torch.int64, device=dev)
-        info = torch.empty(3, dtype=torch.int64, device=dev)
-        _nat.check(prepare(L, out_ptr, info, s), "geo_fps_prepare")
-        total, max_n, bad = info.tolist()
+        info = torch.empty(4, dtype=torch.int64, device=dev)
+        _nat.check(prepare(L, out_ptr, info, s), "geo_fps_prepare_most")
+        total, max_n, bad, most = info.tolist()
         if bad:
             raise ValueError(f"fps: ptr is not a non-decreasing offset array within [0, {N}] "
                              f"(first bad entry: ptr[{bad - 1}])")
@@ -852,8 +852,8 @@ def _fps_run(pos: Tensor, p: Tensor, B: int, prepare) -> Tensor:
             return out
         ws_bytes = L.geo_fps_workspace_bytes(B, N, max_n)
         ws = _nat.workspace(ws_bytes, dev)
-        _nat.check(L.geo_fps_total(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, total,
-                                   _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
+        _nat.check(L.geo_fps_most(_nat.ptr(pos), N, _nat.ptr(p), _nat.ptr(out_ptr), B, max_n, most,
+                                  _nat.ptr(out), _nat.ptr(ws), ws_bytes, s), "geo_fps")
     return out
 
 

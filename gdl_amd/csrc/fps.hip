@@ -30,7 +30,7 @@ constexpr int kFpsThreads = 256;
 constexpr int kFpsWaves = kFpsThreads / kWave;
 constexpr int kFpsLdsPoints = 8192;         // largest cloud of the bucketed kernel
 constexpr int kFpsRegisterPoints = 16384;   // largest cloud of the register kernel
-constexpr int kFpsRegisterSamples = 80;     // most samples per cloud it is chosen for
+constexpr int kFpsRegisterSamples = 80;     // most samples of a cloud it is chosen for
 constexpr int kFpsBucketThreads = 1024;
 constexpr int kFpsRound = 16;  // most centroids that one round of the bucketed kernel takes
 constexpr int kFpsStreamThreads = 1024;
@@ -45,12 +45,12 @@ struct alignas(8) FpsSlot {
 __global__ __launch_bounds__(kScanThreads) void fps_prepare_kernel(
     const int64_t* __restrict__ ptr, const int64_t* __restrict__ kpb, int64_t k_all, int64_t B,
     int64_t N_total, int64_t* __restrict__ out_ptr, int64_t* __restrict__ info,
-    int64_t* __restrict__ info_host) {
+    int64_t* __restrict__ info_host, int64_t* __restrict__ most) {
   __shared__ int64_t lds[kScanThreads / kWave];
-  __shared__ unsigned long long s_max, s_bad;
+  __shared__ unsigned long long s_max, s_bad, s_most;
   constexpr unsigned long long kNone = ~0ull;
   if (threadIdx.x == 0) {
-    s_max = 0;
+    s_max = s_most = 0;
     s_bad = (ptr[0] >= 0 && ptr[0] <= N_total) ? kNone : 1ull;  // 1-based entry index
   }
   __syncthreads();
@@ -66,6 +66,7 @@ __global__ __launch_bounds__(kScanThreads) void fps_prepare_kernel(
       k = kpb ? kpb[b] : k_all;  // one k for every cloud when no per-cloud array is given
       k = k < 0 ? 0 : (k > nn ? nn : k);
       atomicMax(&s_max, static_cast<unsigned long long>(nn));
+      if (most) atomicMax(&s_most, static_cast<unsigned long long>(k));
     }
     int64_t total;
     const int64_t off = block_exclusive_scan<int64_t>(k, lds, total);
@@ -79,6 +80,7 @@ __global__ __launch_bounds__(kScanThreads) void fps_prepare_kernel(
     info[0] = carry;
     info[1] = static_cast<int64_t>(s_max);
     info[2] = bad;
+    if (most) *most = static_cast<int64_t>(s_most);
     if (info_host) {  // mapped pinned host copy, read by the host once this kernel has finished
       info_host[0] = carry;
       info_host[1] = static_cast<int64_t>(s_max);
@@ -1231,15 +1233,25 @@ int launch_large(const float* pos, int64_t N, const int64_t* ptr, const int64_t*
 
 using namespace geo;
 
-extern "C" int geo_fps_prepare(const int64_t* ptr, const int64_t* k_per_batch, int64_t B,
-                               int64_t N_total, int64_t* out_ptr, int64_t* info, void* stream) {
+static int fps_prepare(const int64_t* ptr, const int64_t* k_per_batch, int64_t B, int64_t N_total,
+                       int64_t* out_ptr, int64_t* info, int64_t* most, void* stream) {
   GEO_REQUIRE(B >= 0 && N_total >= 0, "fps_prepare: negative size");
   GEO_REQUIRE(ptr && out_ptr && info && (B == 0 || k_per_batch), "fps_prepare: null pointer");
   hipLaunchKernelGGL(fps_prepare_kernel, dim3(1), dim3(kScanThreads), 0, as_stream(stream), ptr,
                      k_per_batch, int64_t{0}, B, N_total, out_ptr, info,
-                     static_cast<int64_t*>(nullptr));
+                     static_cast<int64_t*>(nullptr), most);
   GEO_LAUNCH_CHECK("fps_prepare_kernel");
   return GEO_OK;
+}
+
+extern "C" int geo_fps_prepare(const int64_t* ptr, const int64_t* k_per_batch, int64_t B,
+                               int64_t N_total, int64_t* out_ptr, int64_t* info, void* stream) {
+  return fps_prepare(ptr, k_per_batch, B, N_total, out_ptr, info, nullptr, stream);
+}
+
+extern "C" int geo_fps_prepare_most(const int64_t* ptr, const int64_t* k_per_batch, int64_t B,
+                                    int64_t N_total, int64_t* out_ptr, int64_t* info, void* stream) {
+  return fps_prepare(ptr, k_per_batch, B, N_total, out_ptr, info, info ? info + 3 : nullptr, stream);
 }
 
 extern "C" int geo_fps_prepare_uniform(const int64_t* ptr, int64_t k, int64_t B, int64_t N_total,
@@ -1253,7 +1265,8 @@ extern "C" int geo_fps_prepare_uniform(const int64_t* ptr, int64_t k, int64_t B,
     GEO_REQUIRE(host_dev != nullptr, "fps_prepare: info_host is not mapped pinned memory");
   }
   hipLaunchKernelGGL(fps_prepare_kernel, dim3(1), dim3(kScanThreads), 0, as_stream(stream), ptr,
-                     static_cast<const int64_t*>(nullptr), k, B, N_total, out_ptr, info, host_dev);
+                     static_cast<const int64_t*>(nullptr), k, B, N_total, out_ptr, info, host_dev,
+                     static_cast<int64_t*>(nullptr));
   GEO_LAUNCH_CHECK("fps_prepare_kernel");
   return GEO_OK;
 }
@@ -1297,14 +1310,22 @@ extern "C" size_t geo_fps_workspace_bytes(int64_t B, int64_t N_total, int64_t ma
 extern "C" int geo_fps(const float* pos, int64_t N_total, const int64_t* ptr,
                        const int64_t* out_ptr, int64_t B, int64_t max_cloud, int64_t* out_idx,
                        void* workspace, size_t workspace_bytes, void* stream) {
-  return geo_fps_total(pos, N_total, ptr, out_ptr, B, max_cloud, N_total, out_idx, workspace,
-                       workspace_bytes, stream);
+  return geo_fps_most(pos, N_total, ptr, out_ptr, B, max_cloud, max_cloud, out_idx, workspace,
+                      workspace_bytes, stream);
 }
 
 extern "C" int geo_fps_total(const float* pos, int64_t N_total, const int64_t* ptr,
                              const int64_t* out_ptr, int64_t B, int64_t max_cloud, int64_t total,
                              int64_t* out_idx, void* workspace, size_t workspace_bytes,
                              void* stream) {
+  return geo_fps_most(pos, N_total, ptr, out_ptr, B, max_cloud, B > 0 ? ceil_div(total, B) : 0, out_idx,
+                      workspace, workspace_bytes, stream);
+}
+
+extern "C" int geo_fps_most(const float* pos, int64_t N_total, const int64_t* ptr,
+                            const int64_t* out_ptr, int64_t B, int64_t max_cloud, int64_t most,
+                            int64_t* out_idx, void* workspace, size_t workspace_bytes,
+                            void* stream) {
   GEO_REQUIRE(B >= 0 && N_total >= 0 && max_cloud >= 0, "fps: negative size");
   GEO_REQUIRE(max_cloud <= N_total, "fps: max_cloud %lld > N_total %lld", (long long)max_cloud,
               (long long)N_total);
@@ -1325,13 +1346,14 @@ extern "C" int geo_fps_total(const float* pos, int64_t N_total, const int64_t* p
     if (p2 <= 4) return launch_bucket<4, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
     return launch_bucket<8, kFpsBucketThreads>(pos, ptr, out_ptr, B, max_cloud, out_idx, st);
   }
-  // Up to 16,384 points and few samples per cloud: the register kernel, which has no set-up.  The
+  // Up to 16,384 points and few samples in every cloud (the register kernel's steps take as long
+  // for a small cloud, and the one with the most samples ends last): no set-up.  The
   // large kernel's sort and first rounds cost about 90 us more, its later rounds a tenth as much
   // per sample (12,000 points: 64 samples 197 against 225 us, 375 samples 1069 against 399 us,
   // 6000 samples 16.9 against 2.2 ms); they cross at 73 to 87 samples between 8,200 and 16,384.
   // Callers that bring no workspace for such clouds get it as well.
   if (max_cloud <= kFpsRegisterPoints &&
-      (total <= kFpsRegisterSamples * B || !room || !fps_use_large(B, max_cloud))) {
+      (most <= kFpsRegisterSamples || !room || !fps_use_large(B, max_cloud))) {
     hipLaunchKernelGGL((fps_register_kernel<kFpsRegisterPoints / kFpsThreads>), dim3(B),
                        dim3(kFpsThreads), 0, st, pos, ptr, out_ptr, out_idx);
     GEO_LAUNCH_CHECK("fps_register_kernel");

@@ -95,8 +95,16 @@ size_t geo_fps_workspace_bytes(int64_t B, int64_t N_total, int64_t max_cloud);
 int geo_fps(const float* pos, int64_t N_total, const int64_t* ptr, const int64_t* out_ptr,
             int64_t B, int64_t max_cloud, int64_t* out_idx, void* workspace,
             size_t workspace_bytes, void* stream);
-/* geo_fps told the batch's number of samples (info[0]): clouds of 8193 to 16,384 points with few
- * samples each then take a kernel without set-up.  geo_fps alone assumes many. */
+/* geo_fps_prepare with info of 4 entries: info[3] = the most samples of any cloud. */
+int geo_fps_prepare_most(const int64_t* ptr, const int64_t* k_per_batch, int64_t B, int64_t N_total,
+                         int64_t* out_ptr, int64_t* info, void* stream);
+/* geo_fps told the most samples of any cloud: where these are few, clouds of 8193 to 16,384 points
+ * take a kernel without set-up.  geo_fps alone assumes many; without a workspace it takes that
+ * kernel for such clouds. */
+int geo_fps_most(const float* pos, int64_t N_total, const int64_t* ptr, const int64_t* out_ptr,
+                 int64_t B, int64_t max_cloud, int64_t most, int64_t* out_idx, void* workspace,
+                 size_t workspace_bytes, void* stream);
+/* The same, told only the batch's number of samples (info[0]): taken as spread evenly. */
 int geo_fps_total(const float* pos, int64_t N_total, const int64_t* ptr, const int64_t* out_ptr,
                   int64_t B, int64_t max_cloud, int64_t total, int64_t* out_idx, void* workspace,
                   size_t workspace_bytes, void* stream);

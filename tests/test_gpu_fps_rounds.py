@@ -94,3 +94,21 @@ def test_clouds_of_the_register_kernel_need_no_workspace(n):
                                 None, 0, nat.stream_of(pos.device)), "geo_fps")
     want = oracle.fps(pos.cpu().numpy(), np.array([0, n]), np.array([k]))
     np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("counts", [[100, 3, 3, 3], [16, 200, 200, 200], [80, 80, 7, 80], [81, 0, 0, 0]])
+def test_unequal_samples_of_clouds_that_the_register_kernel_holds(counts):
+    """The kernel is chosen by the cloud with the most samples, which ends last."""
+    from gdl_amd import _native as nat
+    from gdl_amd.csrc import fps_cuda
+    sizes = [8400, 300, 700, 250]
+    pos = _points("cube", sum(sizes), 5)
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    k = np.array(counts)
+    p, kk = torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()
+    out_ptr, info = torch.empty(5, dtype=torch.int64).cuda(), torch.empty(4, dtype=torch.int64).cuda()
+    nat.check(nat.lib().geo_fps_prepare_most(nat.ptr(p), nat.ptr(kk), 4, sum(sizes), nat.ptr(out_ptr), nat.ptr(info),
+                                             nat.stream_of(info.device)), "geo_fps_prepare_most")
+    assert info.tolist() == [int(np.minimum(k, sizes).sum()), 8400, 0, int(np.minimum(k, sizes).max())]
+    got = fps_cuda(pos.cuda(), p, kk).cpu().numpy()
+    np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
