@@ -33,6 +33,8 @@ constexpr int kFpsRegisterPoints = 16384;   // largest cloud of the register ker
 constexpr int kFpsRegisterSamples = 80;     // most samples of a cloud it is chosen for
 constexpr int kFpsBucketThreads = 1024;
 constexpr int kFpsRound = 16;  // most centroids that one round of the bucketed kernel takes
+constexpr int kFpsFew = 96;    // samples up to which it takes one centroid per step, see fps_is_few
+constexpr int kFpsLead = 48;   // first centroids taken so by its largest variant; below kFpsFew
 constexpr int kFpsStreamThreads = 1024;
 constexpr int kFpsStreamWaves = kFpsStreamThreads / kWave;
 
@@ -396,6 +398,72 @@ __device__ __forceinline__ void fps_one_wave(const float* __restrict__ P, int n,
   }
 }
 
+// The greedy choice over a workgroup from each wave's maximum m (bits) and lowest index j attaining
+// it.  best: three zeroed slots used in turn, `at` the next one.
+__device__ __forceinline__ int fps_best(unsigned long long* best, int& at, uint32_t m, uint32_t j) {
+  if (lane_id() == 0) atomicMax(&best[at], (static_cast<unsigned long long>(m) << 32) | static_cast<uint32_t>(~j));
+  lds_barrier();
+  const int idx = __builtin_amdgcn_readfirstlane(static_cast<int>(~static_cast<uint32_t>(best[at])));
+  // every wave has read the slot before this one, which is next used two barriers on
+  at = at == 2 ? 0 : at + 1;
+  if (threadIdx.x == 0) best[at == 2 ? 0 : at + 1] = 0;
+  return idx;
+}
+
+// Few samples of a cloud of more than kFpsWavePoints points: one centroid per step by the whole
+// workgroup, the points in registers as they come and in LDS (xyz, 12 B per point).  Ordering the
+// cloud does not pay for so few, and the first centroids lower nearly every point, so that rounds
+// take one or two of them.  What bounds a step is its vector instructions (eight points a lane: 0.79
+// us) and below that its barrier, the atomic and the chain behind it (one point: 0.34 us).
+// Call times with rounds -> now, 16 surface clouds: 4096 points to 16 samples 41 -> 25 us, to 64 67 ->
+// 45, to 128 88 -> 81, to 192 100 / 116; 8192 points to 32 82 -> 38, to 96 125 -> 89; 1024 points to 64
+// 42 -> 32, to 128 57 / 56, to 192 70 / 79.  One cloud, where rounds pay earliest: 2048 points to 96 52 ->
+// 50, to 128 60 / 64; 4096 to 128 84 -> 79.  Above 4096 points the rounds begin with such steps too
+// (kFpsLead) and pay from about 110 samples on (4200 points to 128 104 / 121).
+template <int PTS>
+__device__ __forceinline__ bool fps_is_few(int k, int n) {
+  if (n <= 512) return k <= 128;  // at most eight buckets: 256 clouds of 400 to 128 61 -> 54 us
+  return k <= (PTS == 8 ? kFpsFew : max(kFpsFew, 64 + n / 64));
+}
+template <int PTS, int THREADS>
+__device__ __forceinline__ void fps_few(const float* __restrict__ P, int n, int k, int64_t start,
+                                        int64_t* __restrict__ out, float* xyz,
+                                        unsigned long long* best) {
+  const int t = threadIdx.x, lane = lane_id();
+  float px[PTS], py[PTS], pz[PTS];
+  uint32_t md[PTS];
+  for (int i = t; i < 3 * n; i += THREADS) xyz[i] = P[i];
+  if (t < 3) best[t] = 0;
+  lds_barrier();
+#pragma unroll
+  for (int s = 0; s < PTS; ++s) {
+    const int i = s * THREADS + t, at = i < n ? i : 0;
+    px[s] = xyz[3 * at]; py[s] = xyz[3 * at + 1]; pz[s] = xyz[3 * at + 2];
+    md[s] = i < n ? 0x7f800000u : 0u;  // padding never comes before point 0
+  }
+  int idx = 0, at = 0;  // at: the slot of best in use
+  for (int it = 0;; ++it) {
+    if (t == 0) out[it] = start + idx;
+    if (it + 1 >= k) break;
+    const float cx = xyz[3 * idx], cy = xyz[3 * idx + 1], cz = xyz[3 * idx + 2];
+    uint32_t m = 0u;
+#pragma unroll
+    for (int s = 0; s < PTS; ++s) {
+      md[s] = min(md[s], __float_as_uint(sqdist(px[s], py[s], pz[s], cx, cy, cz)));
+      m = max(m, md[s]);
+    }
+    m = wave_max_u32(m);
+    // the wave's first slot that holds the maximum, its first lane: the lowest index
+    uint32_t j = 0;
+#pragma unroll
+    for (int s = PTS - 1; s >= 0; --s) {
+      const uint64_t hit = __ballot(md[s] == m);
+      if (hit) j = static_cast<uint32_t>(s * THREADS + (t - lane) + __builtin_ctzll(hit));
+    }
+    idx = fps_best(best, at, m, j);
+  }
+}
+
 template <int PTS, int THREADS>
 __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const float* __restrict__ pos, const int64_t* __restrict__ ptr,
@@ -438,6 +506,12 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     return;
   }
 
+  if (fps_is_few<PTS>(k, n)) {
+    fps_few<PTS, THREADS>(P, n, k, start, out_idx + o0, reinterpret_cast<float*>(scratch),
+                          reinterpret_cast<unsigned long long*>(rkey));
+    return;
+  }
+
   // 1-2. the cloud ordered along the Hilbert curve of its cell grid
   int2* code_rank = scratch;
   int* order = reinterpret_cast<int*>(scratch + n);
@@ -463,6 +537,44 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     md[s] = in ? 0x7f800000u : 0u;  // padding: never changes, never wins
   }
 
+  // The first centroids lower nearly every point, and a round of one or two of them that forms all
+  // records again (eight a wave) takes longer than a step that only lowers and compares: without
+  // them 16 clouds of 8192 points to 192 samples took 180 us (143 with), to 512 269 (237), 6000
+  // points to 192 161 (140); a cloud of 8192 to 4096 972 (937).
+  constexpr int lead = PTS == 8 ? kFpsLead : 0;
+  if constexpr (lead > 0) {
+    float* xyz = reinterpret_cast<float*>(scratch);
+    unsigned long long* best = reinterpret_cast<unsigned long long*>(rkey);
+    lds_barrier();  // the order is read
+#pragma unroll
+    for (int s = 0; s < PTS; ++s) {
+      if (oi[s] == 0xffffffffu) continue;
+      xyz[3 * oi[s]] = px[s];
+      xyz[3 * oi[s] + 1] = py[s];
+      xyz[3 * oi[s] + 2] = pz[s];
+    }
+    if (t < 3) best[t] = 0;
+    lds_barrier();
+    int idx = 0, at = 0;
+    for (int it = 0;; ++it) {
+      if (t == 0) out_idx[o0 + it] = start + idx;
+      const float cx = xyz[3 * idx], cy = xyz[3 * idx + 1], cz = xyz[3 * idx + 2];
+      uint32_t m = 0u;
+#pragma unroll
+      for (int s = 0; s < PTS; ++s) {
+        md[s] = min(md[s], __float_as_uint(sqdist(px[s], py[s], pz[s], cx, cy, cz)));
+        m = max(m, md[s]);
+      }
+      if (it + 1 == lead) break;
+      m = wave_max_u32(m);
+      uint32_t j = 0xffffffffu;
+#pragma unroll
+      for (int s = 0; s < PTS; ++s) j = min(j, md[s] == m ? oi[s] : 0xffffffffu);
+      idx = fps_best(best, at, m, wave_min_u32(j));
+    }
+    lds_barrier();  // rkey holds the records from here on
+  }
+
   // 4. bucket records: box and max (bits) of slot 4 h + lane / 16 in the lane; the farthest point
   //    (bits, index, lane, position) and the rest bound of slot s as scalars.
   float blx[TESTS], bly[TESTS], blz[TESTS], bhx[TESTS], bhy[TESTS], bhz[TESTS];
@@ -470,6 +582,35 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
   uint32_t bm[PTS], bi[PTS], al[PTS], rs[PTS];
   uint32_t ri[PTS];  // lowest index at the rest bound, 0 = not known
   float sx[PTS], sy[PTS], sz[PTS];
+  // the record and rest bound of slot s, whose points have the min distances mb (bits)
+  auto record = [&](int s, uint32_t mb) {
+    const uint32_t mx = wave_max_u32(mb);
+    const uint64_t hit = __ballot(mb == mx);
+    ri[s] = 0u;
+    if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
+      al[s] = static_cast<uint32_t>(__builtin_ctzll(hit));
+      bi[s] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(oi[s]), al[s]));
+    } else {
+      bi[s] = wave_min_u32(mb == mx ? oi[s] : 0xffffffffu);
+      al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(mb == mx && oi[s] == bi[s]) | (1ull << 63)));
+      // the others at the maximum that stay there
+      const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
+      const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
+      const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
+      const bool stay = mb == mx && __float_as_uint(sqdist(px[s], py[s], pz[s], x, y, z)) >= mx;
+      if (__ballot(stay)) ri[s] = wave_min_u32(stay ? oi[s] : 0xffffffffu);
+    }
+    bm[s] = mx;
+    if (lane / 16 == s % 4) bmax[s / 4] = mx;
+    if (lane == 0) rkey[s * WAVES + w] = fps_key(mx, bi[s]);
+    sx[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
+    sy[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
+    sz[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
+    // what the bucket's other points can reach once that point is a centroid (its own lane
+    // gives 0)
+    rs[s] = wave_max_u32(
+        min(mb, __float_as_uint(sqdist(px[s], py[s], pz[s], sx[s], sy[s], sz[s]))));
+  };
 #pragma unroll
   for (int h = 0; h < TESTS; ++h) {
     blx[h] = bly[h] = blz[h] = __builtin_inff();
@@ -486,7 +627,16 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     const uint32_t h1 = wave_max_u32(valid ? float_order_key(py[s]) : 0u);
     const uint32_t h2 = wave_max_u32(valid ? float_order_key(pz[s]) : 0u);
     const bool any = (s * WAVES + w) * kWave < n;
-    // every distance is +inf, so the record is the lowest index; it stands until that point falls,
+    if constexpr (lead > 0) {
+      if (lane / 16 == s % 4 && any) {
+        blx[s / 4] = float_from_order_key(l0); bly[s / 4] = float_from_order_key(l1);
+        blz[s / 4] = float_from_order_key(l2); bhx[s / 4] = float_from_order_key(h0);
+        bhy[s / 4] = float_from_order_key(h1); bhz[s / 4] = float_from_order_key(h2);
+      }
+      record(s, md[s]);
+      continue;
+    }
+    // no centroid yet: every distance is +inf, so the record is the lowest index; it stands until that point falls,
     // which it never does where squared distances overflow (no update then touches the bucket)
     bm[s] = any ? 0x7f800000u : 0u;
     bi[s] = wave_min_u32(oi[s]);
@@ -509,12 +659,35 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
     list[0] = make_float4(P[0], P[1], P[2], __builtin_inff());
     lkey[0] = make_double2(fps_key(0u, 0u), 0.0);
   }
+  // rank: every wave places its own records among all of them and lists the first kFpsRound
+  auto rank_records = [&]() {
+    double kk[SETS];
+#pragma unroll
+    for (int e = 0; e < SETS; ++e) {
+      kk[e] = rkey[e * kWave + lane];
+    }
+#pragma unroll
+    for (int s = 0; s < PTS; ++s) {
+      const double kj = fps_key(bm[s], bi[s]);
+      int rank = 0;
+#pragma unroll
+      for (int e = 0; e < SETS; ++e) rank += __builtin_popcountll(__ballot(kk[e] > kj));
+      if (rank < kFpsRound && (s * WAVES + w) * kWave < n && lane == 0) {
+        list[rank] = make_float4(sx[s], sy[s], sz[s], __uint_as_float(bm[s]));
+        lkey[rank] = make_double2(kj, fps_key(rs[s], ri[s]));
+      }
+    }
+  };
   lds_barrier();
+  if constexpr (lead > 0) {
+    rank_records();
+    lds_barrier();
+  }
 
   // records that exist: no more can be taken in one round
   const int cap = min(kFpsRound, (n + kWave - 1) / kWave);
   const int li = lane & (kFpsRound - 1);
-  int done = 0, kend = k;
+  int done = lead, kend = k;
   for (;;) {
     // which of the listed records are the next centroids: record j is one if no record i ahead of
     // it can lower its point, and no other point of a bucket ahead can come before it
@@ -577,53 +750,12 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
         // Values only fall: while the point holding the bucket's max keeps its value, the record
         // (max, lowest index attaining it) stands, and its rest bound still holds.
         if (!((__ballot(mb < old) >> al[s]) & 1ull)) continue;
-        const uint32_t mx = wave_max_u32(mb);
-        const uint64_t hit = __ballot(mb == mx);
-        ri[s] = 0u;
-        if ((hit & (hit - 1)) == 0) {  // one lane holds the maximum (distance ties are rare)
-          al[s] = static_cast<uint32_t>(__builtin_ctzll(hit));
-          bi[s] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(oi[s]), al[s]));
-        } else {
-          bi[s] = wave_min_u32(mb == mx ? oi[s] : 0xffffffffu);
-          al[s] = static_cast<uint32_t>(__builtin_ctzll(__ballot(mb == mx && oi[s] == bi[s]) | (1ull << 63)));
-          // the others at the maximum that stay there
-          const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
-          const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
-          const float z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
-          const bool stay = mb == mx && __float_as_uint(sqdist(px[s], py[s], pz[s], x, y, z)) >= mx;
-          if (__ballot(stay)) ri[s] = wave_min_u32(stay ? oi[s] : 0xffffffffu);
-        }
-        bm[s] = mx;
-        if (lane / 16 == s % 4) bmax[h] = mx;
-        if (lane == 0) rkey[s * WAVES + w] = fps_key(mx, bi[s]);
-        sx[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(px[s]), al[s]));
-        sy[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(py[s]), al[s]));
-        sz[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pz[s]), al[s]));
-        // what the bucket's other points can reach once that point is a centroid (its own lane
-        // gives 0)
-        rs[s] = wave_max_u32(
-            min(mb, __float_as_uint(sqdist(px[s], py[s], pz[s], sx[s], sy[s], sz[s]))));
+        record(s, mb);
       }
     }
     lds_barrier();  // waves share only LDS in this loop
 
-    // rank: every wave places its own records among all of them and lists the first kFpsRound
-    double kk[SETS];
-#pragma unroll
-    for (int e = 0; e < SETS; ++e) {
-      kk[e] = rkey[e * kWave + lane];
-    }
-#pragma unroll
-    for (int s = 0; s < PTS; ++s) {
-      const double kj = fps_key(bm[s], bi[s]);
-      int rank = 0;
-#pragma unroll
-      for (int e = 0; e < SETS; ++e) rank += __builtin_popcountll(__ballot(kk[e] > kj));
-      if (rank < kFpsRound && (s * WAVES + w) * kWave < n && lane == 0) {
-        list[rank] = make_float4(sx[s], sy[s], sz[s], __uint_as_float(bm[s]));
-        lkey[rank] = make_double2(kj, fps_key(rs[s], ri[s]));
-      }
-    }
+    rank_records();
     lds_barrier();
   }
   for (int i = done + t; i < k; i += THREADS) out_idx[o0 + i] = start;  // distances all 0

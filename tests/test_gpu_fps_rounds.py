@@ -112,3 +112,17 @@ def test_unequal_samples_of_clouds_that_the_register_kernel_holds(counts):
     assert info.tolist() == [int(np.minimum(k, sizes).sum()), 8400, 0, int(np.minimum(k, sizes).max())]
     got = fps_cuda(pos.cuda(), p, kk).cpu().numpy()
     np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
+
+
+@pytest.mark.parametrize("kind", ["cube", "lattice", "same"])
+@pytest.mark.parametrize("sizes,counts", [
+    ([385, 1024, 700], [1, 2, 96]), ([1025, 2048], [96, 97]), ([2049, 4096, 4095], [97, 128, 128]),
+    ([4097, 8192, 8191, 500], [96, 97, 140, 3]), ([8192, 6000, 2000], [300, 2, 400]),
+])
+def test_few_samples(kind, sizes, counts):
+    from gdl_amd.csrc import fps_cuda
+    pos = _points(kind, sum(sizes), sum(counts))
+    ptr = np.concatenate([[0], np.cumsum(sizes)])
+    k = np.array(counts)
+    got = fps_cuda(pos.cuda(), torch.from_numpy(ptr).cuda(), torch.from_numpy(k).cuda()).cpu().numpy()
+    np.testing.assert_array_equal(got, oracle.fps(pos.numpy(), ptr, k))
