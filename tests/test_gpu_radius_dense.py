@@ -81,3 +81,15 @@ def test_around_the_staged_number(n, K, loop):
     x = torch.rand(n, 3, generator=g)
     for r in (2.0, 1e19, 1e20):
         _check(x, r, K, loop=loop)
+
+
+@pytest.mark.parametrize("m", [513, 1025, 3000])
+@pytest.mark.parametrize("K,loop", [(1, False), (32, True), (255, True), (256, False), (600, True), (1024, True), (1030, False)])
+def test_many_copies(m, K, loop):
+    """More sources at one distance than are staged (a padded cloud): the K-th by parts of the index
+    range, for the copies themselves, for targets beside them and where others lie just before them."""
+    g = torch.Generator().manual_seed(m + K)
+    near = 1e-4 * torch.randn(40, 3, generator=g)
+    x = torch.cat([torch.zeros(m, 3), near, torch.tensor([[0.05, 0.0, 0.0]]).repeat(m // 3, 1), torch.rand(300, 3, generator=g)])
+    x = x[torch.randperm(x.shape[0], generator=g)].contiguous() if K % 2 else x
+    _check(x, 0.1, K, loop=loop)
