@@ -18,6 +18,7 @@ CONFIGS = [
     (36, 3, 0, 20, 3, 0), (64, 17, 5, 8, 0, 3), (60, 32, 0, 16, 16, 0),
     (68, 16, 0, 16, 16, 0), (128, 32, 0, 32, 8, 0), (100, 7, 3, 6, 0, 2), (128, 20, 16, 0, 0, 4),
     (0, 9, 4, 3, 2, 2), (8, 0, 16, 3, 0, 5),
+    (7, 20, 0, 5, 4, 0), (15, 32, 3, 4, 4, 2), (32, 20, 8, 16, 16, 4), (16, 17, 0, 4, 3, 2),
     (132, 4, 0, 4, 4, 0), (16, 33, 0, 4, 4, 0), (16, 4, 17, 4, 4, 2),  # one channel too many
 ]
 
