@@ -459,17 +459,18 @@ def _se3_backward(ctx, g_s, g_v, g_t, _gXs, _gXv, _gXt):
 _se3_fwd_op.register_autograd(_se3_backward, setup_context=_se3_setup)
 
 
-def _plain_eager(x: Tensor) -> bool:
-    """True for a plain tensor outside tracing: the eager path may call the implementations
-    directly.  Fake or other subclassed tensors, and torch.compile, take the custom ops."""
-    return type(x) is torch.Tensor and not torch.compiler.is_compiling()
+def _direct(*grads: Optional[Tensor]) -> bool:
+    """Whether a backward may call its implementation directly.  Gradients that are recorded
+    themselves (create_graph) go through the op, whose backward is an error: the kernels' outputs
+    alone would look like constants."""
+    return not torch.is_grad_enabled() and all(g is None or _nat.plain_eager(g) for g in grads)
 
 
 class _SE3ConvEager(torch.autograd.Function):
     """Eager mode: the custom ops' forward and backward implementations called directly.  The
     custom-op layers (schema defaults, dispatch, the registered autograd) cost more host time per
-    call than a C2 layer's kernels take; under torch.compile the custom ops are used, so the
-    compiled graph still traces through them."""
+    call than a C2 layer's kernels take; where anything but plain eager execution is under way
+    (plain_eager) the custom ops are used, which all of it can see."""
 
     @staticmethod
     def forward(ctx, *args):
@@ -479,7 +480,9 @@ class _SE3ConvEager(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_s, g_v, g_t, _gXs, _gXv, _gXt):
-        return _se3_grads(ctx, g_s, g_v, g_t, _se3_bwd_impl)
+        return _se3_grads(ctx, g_s, g_v, g_t, _se3_bwd_impl if _direct(g_s, g_v, g_t)
+                          else torch.ops.geoembodied.se3_conv_bwd)
+
 
 _DEFAULT_CG: Dict[torch.device, Tensor] = {}
 
@@ -556,7 +559,7 @@ def se3_message_aggregate(
     Wl = [_nat.f32c(w) if w is not None else None for w in Wl]
     direction = _nat.f32c(graph.direction)
     args = (s, v, t, row, col, perm, ns, ne, direction, Y, R, avg, m, b, cg, dims, *Wl)
-    if _plain_eager(s):
+    if _nat.plain_eager(s):
         s_out, v_out, t_out, _, _, _ = _SE3ConvEager.apply(*args)
     else:
         s_out, v_out, t_out, _, _, _ = torch.ops.geoembodied.se3_conv_fwd(*args)
@@ -656,7 +659,8 @@ class _RadialEager(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dR):
-        return _radial_grads(ctx, dR, _radial_bwd_impl)
+        return _radial_grads(ctx, dR, _radial_bwd_impl if _direct(dR)
+                             else torch.ops.geoembodied.radial_mlp_bwd)
 
 
 def radial_mlp(dist: Tensor, freqs: Tensor, cutoff: float, W1: Tensor, b1: Tensor, W2: Tensor,
@@ -667,7 +671,7 @@ def radial_mlp(dist: Tensor, freqs: Tensor, cutoff: float, W1: Tensor, b1: Tenso
     _require_gpu("radial_mlp", dist)
     c = [_nat.f32c(x) for x in (dist, freqs, W1, b1, W2, b2)]
     args = (c[0], c[1], float(cutoff), c[2], c[3], c[4], c[5])
-    if _plain_eager(c[0]):
+    if _nat.plain_eager(c[0]):
         return _RadialEager.apply(*args)
     return torch.ops.geoembodied.radial_mlp(*args)
 
