@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kFpsThreads) void fps_register_kernel(
 // lattice to 1024 samples, one at a time -> distance alone -> now: in order 524 -> 820 -> 459 us,
 // shuffled 525 -> 853 -> 268 us.  The index is looked for only where several points hold a
 // bucket's max (elsewhere 0, before all others, which ends a round at an equal distance in another
-// bucket: 3% more rounds on lattices).  It costs other clouds 1.6% (4096 points) to 4% (1024).
+// bucket: 3% more rounds on lattices).  It costs clouds of 1000 to 2000 points 1 to 3%.
 // Where the first record's distance is 0 every point lies on a sample, and the lowest index is the
 // choice for all that is left: no further rounds (one point 4096 times: 855 -> 28 us a call).
 // A round costs two LDS barriers:
@@ -347,6 +347,16 @@ __device__ __forceinline__ double fps_key(uint32_t bits, uint32_t idx) {
 }
 __device__ __forceinline__ uint32_t fps_key_index(double key) {
   return ~static_cast<uint32_t>(__double2loint(key));
+}
+
+// The lanes of a round's check that hold a pair (i, j): i = lane % 16 ahead of j = `j` + lane / 16.
+// As constants: formed by a compare in every round they cost a few of the 1000 to 1600 ns it takes
+// (16 clouds of 4096 points to 1024 samples 237.6 -> 234.3 us, one of 2048 to 512 145.4 -> 143.2; a
+// branch around the compare of keys, taken where distances are equal, 152).
+constexpr uint64_t fps_ahead(int j) {
+  uint64_t m = 0;
+  for (int r = 0; r < 4; ++r) m |= static_cast<uint64_t>((1u << (j + r)) - 1u) << (16 * r);
+  return m;
 }
 
 // Clouds of up to kFpsWavePoints points: one wave, point s * 64 + lane in slot s of the lane, one
@@ -702,8 +712,8 @@ __global__ __launch_bounds__(THREADS) void fps_bucket_kernel(
         const float4 p0 = list[j0], p1 = list[j1];
         const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
         const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
-        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & __ballot(li < j0);
-        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & __ballot(li < j1);
+        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & fps_ahead(g);
+        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & fps_ahead(g + 4);
         if (b0 | b1) {
           A = g + (b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16;
           break;
@@ -849,12 +859,12 @@ __global__ __launch_bounds__(kFpsStreamThreads) void fps_stream_kernel(
 // A 32^3 lattice to 4096 samples, one at a time -> rounds by distance alone -> now: in order 5.55 ->
 // 7.79 -> 3.15 ms, shuffled 5.51 -> 7.76 -> 1.91 ms.
 // A 131,072-point lidar frame to 16,384 samples: 1,634 rounds of 10.0 centroids and 5.5 us,
-// 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,200 cycles issues 455
-// vector instructions per wave (59% of what the CU's four SIMDs can issue in that time), 290 of
-// them in update.  Tried without gain: the queue's buckets handed to whichever wave is free (9.3 ms),
-// tests per 16 buckets with a centroid list per row (9.3), one bucket prefetched ahead (9.6), four
-// or eight loaded together (9.2, 9.6), min distances stored only where they fell (9.5: the
-// conditional store makes every later load wait for it).
+// 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,300 cycles issues 469
+// vector instructions per wave, 57% of what the CU's four SIMDs can issue in that time.  Tried
+// without gain: the queue's buckets handed to whichever wave is free (9.3 ms), tests per 16 buckets
+// with a centroid list per row (9.3), one bucket prefetched ahead (9.6), four or eight loaded
+// together (9.2, 9.6), min distances stored only where they fell (9.5: the conditional store makes
+// every later load wait for it).
 constexpr int kFpsLargeThreads = 1024;
 constexpr int kFpsLargeWaves = kFpsLargeThreads / kWave;
 constexpr int kFpsLargeSlots = 3;
@@ -1064,8 +1074,8 @@ __global__ __launch_bounds__(kFpsLargeThreads) void fps_large_kernel(
         const float4 p0 = list[j0], p1 = list[j1];
         const uint32_t d0 = __float_as_uint(sqdist(c.x, c.y, c.z, p0.x, p0.y, p0.z));
         const uint32_t d1 = __float_as_uint(sqdist(c.x, c.y, c.z, p1.x, p1.y, p1.z));
-        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & __ballot(li < j0);
-        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & __ballot(li < j1);
+        const uint64_t b0 = (__ballot(d0 < __float_as_uint(p0.w)) | __ballot(rb > lkey[j0].x)) & fps_ahead(g);
+        const uint64_t b1 = (__ballot(d1 < __float_as_uint(p1.w)) | __ballot(rb > lkey[j1].x)) & fps_ahead(g + 4);
         if (b0 | b1) {
           A = min(A, g + static_cast<int>(b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) / 16);
           break;
