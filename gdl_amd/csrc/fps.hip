@@ -859,8 +859,8 @@ __global__ __launch_bounds__(kFpsStreamThreads) void fps_stream_kernel(
 // A 32^3 lattice to 4096 samples, one at a time -> rounds by distance alone -> now: in order 5.55 ->
 // 7.79 -> 3.15 ms, shuffled 5.51 -> 7.76 -> 1.91 ms.
 // A 131,072-point lidar frame to 16,384 samples: 1,634 rounds of 10.0 centroids and 5.5 us,
-// 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,300 cycles issues 469
-// vector instructions per wave, 57% of what the CU's four SIMDs can issue in that time.  Tried
+// 22.4 -> 9.1 ms (one centroid per iteration took 1.36 us).  A round of 13,300 cycles issues 461
+// vector instructions per wave, 55% of what the CU's four SIMDs can issue in that time.  Tried
 // without gain: the queue's buckets handed to whichever wave is free (9.3 ms), tests per 16 buckets
 // with a centroid list per row (9.3), one bucket prefetched ahead (9.6), four or eight loaded
 // together (9.2, 9.6), min distances stored only where they fell (9.5: the conditional store makes

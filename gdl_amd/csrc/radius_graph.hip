@@ -768,10 +768,15 @@ __global__ __launch_bounds__(kRgThreads) void rg_count(RgWs w, const int64_t* __
 // wave, one at a time (rg_wave_target).
 constexpr int kRgSlots = 8;
 // Candidates of one target whose distance bits a wave keeps in LDS for the selection.
-// The waves wait for LDS and L2 more than they compute, so how many fit a CU counts, against the
-// targets with more candidates, which read the stencil twice: a lidar frame of 131,072 points at
-// radius 0.5 and K = 64 takes 278 us in all with 512 (20 KB per workgroup), 293 with 768, 315 with
-// 1024, 303 with 384 and 326 with 256.  Large K keep 1024, so that they are still staged.
+// The waves wait for LDS and L2 more than they compute, so how many fit a CU counts (512: 20 KB per
+// workgroup), against the targets with more candidates, which read the stencil twice.  Whole calls
+// with 256 / 384 / 512 / 768 / 1024, us: a lidar frame of 131,072 points at radius 0.5 and K = 64
+// 342 / 334 / 318 / 296 / 320, radius 0.3 and K = 16 262 / 253 / 253 / 259 / 278, radius 0.8 599 / 592 /
+// 580 / 597 / 629; 65,536 points with about 160 in radius 187 / 187 / 187 / 191 / 198, 330 329 / 243 / 234
+// / 241 / 253, 400 528 / 477 / 342 / 357 / 367.  Where most targets have more than 512, more would be
+// better (about 700 on a surface 547 / 550 / 549 / 413 / 391, in a cube 823 / 827 / 811 / 635 / 539), but
+// such a K leaves out nine of ten neighbours, and the common densities pay 2 to 10% for it.  Large K
+// keep 1024, so that they are still staged.
 constexpr int kRgSelCap = 512;
 constexpr int kRgSelCapMax = 1024;
 constexpr int kRgSelSmallK = 256;  // up to this K the smaller number
@@ -819,9 +824,9 @@ __device__ __forceinline__ void wave_scan_runs(const RgWs& w, const int (&ra)[9]
 // What bounds it is the staging pass (about 1200 stencil sources per dense target of a lidar frame)
 // and the chain of LDS steps behind it.  The selection used to be a radix select of four passes over
 // the staged keys, and targets with more than 1024 in-radius sources a binary search of about 32
-// passes over the stencil: that frame 374 -> 278 us in all, radius 0.8 and K = 16 1717 -> 524 us; a
-// sphere of 65,536 points at about 160 sources and K = 64 249 -> 186 us, a cube of 20,000 at about
-// 2000 15.4 -> 0.85 ms.
+// passes over the stencil: whole calls on a lidar frame of 131,072 points at radius 0.5 and K = 64 425
+// -> 317 us, at radius 0.8 and K = 16 7.1 -> 0.58 ms; a sphere of 65,536 points at about 160 sources
+// and K = 64 248 -> 187 us, a cube of 32,768 at about 1500 11.8 -> 0.82 ms.
 // The target's row offset o, and for c > K its position and stencil runs, come from the caller.
 template <int CAP>
 __device__ void rg_wave_target(const RgWs& w, float r2, int K, bool lp, int64_t i, int c, int64_t o,

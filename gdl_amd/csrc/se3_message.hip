@@ -820,7 +820,9 @@ __global__ __launch_bounds__(kSeThreads) void se3_fwd_fused(SeEdges g, SeFeat f,
 // (four scalar channels per lane before), 15 + 7 107 -> 39, 64 + 32 142 -> 87, 128 + 32 97 -> 50,
 // 32 + 16 + 8 156 -> 53, 64 + 16 + 8 199 -> 85; 64 + 16 62 -> 60 (no second zeroing of absent edges).
 // Without type-2 channels four source rows are in flight per lane, with them two (32 + 16 + 8:
-// four 63 us, the wave's registers then leave room for fewer waves; one 53 us).
+// four 63 us, the wave's registers then leave room for fewer waves; one 53 us).  64 + 32 also have
+// two: 32 clouds of 4096 points 235 us a call against 246 with four (339 by the walk), but graphs of
+// a few very long rows, where one wave's chain of loads decides, 1083 against 940 (943).
 constexpr int kRowNodes = kFuTile / kSeWaves;  // nodes per wave = 16-lane rows
 constexpr int kRowStage = 16;                  // edges staged per row per round
 constexpr uint32_t kPastRows = 0x80000000u;    // a byte offset past every array (each < 2 GiB)
